@@ -13,8 +13,9 @@
 //
 //   1. stage the tile's record bytes (16-byte loads) and its constant medians
 //      in LDS;
-//   2. decode every block in parallel, 4 values per lane, a block being an
-//      aligned group of bs/4 lanes (the mirror of the compressor's layout);
+//   2. decode every block in parallel, LV consecutive values per lane, a block
+//      being an aligned group of bs/LV lanes (the mirror of the compressor's
+//      layout);
 //   3. check the index against the records: a scan of the decoded record
 //      sizes must reproduce every start, and the tile's records must end
 //      exactly at the next tile's first record; a stream or index that fails
@@ -23,9 +24,11 @@
 // The decode of one record mirrors szxd_float.cc:34-244 / szxd_double.cc:25-449:
 // value i takes its top min(lead_i, rb) bytes from value i-1 and the rest of
 // its rb bytes from the stream.  The "from value i-1" chain is resolved in
-// parallel: each lane folds its 4 values into a last-writer record of the
+// parallel: each lane folds its values into a last-writer record of the
 // (at most 3) copyable byte positions, and an exclusive segmented scan with
 // the last-writer-wins operator gives every lane the bytes it inherits.
+#include <type_traits>
+
 #include "szx_common.hpp"
 #include "szx_batch.hpp"
 #include "szx_index.hpp"
@@ -105,53 +108,6 @@ __global__ void k_check_header(const uint8_t *s, uint64_t len, uint64_t n, int b
     }
 }
 
-// Whole-vector fp32 output stores are non-temporal: the decoded array is
-// written once and not read back by this kernel, so it streams past the
-// caches (k_decode_tiles 0.178 -> 0.136 ms at 512^3 fp32).
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-template <typename T> struct Store4;
-template <> struct Store4<float> {
-    __device__ static void store_full(float *o, uint64_t e0, const float v[4])
-    {
-        f32x4_t w = {v[0], v[1], v[2], v[3]};
-        __builtin_nontemporal_store(w, reinterpret_cast<f32x4_t *>(o + e0));
-    }
-    __device__ static void store(float *o, uint64_t e0, uint64_t n, const float v[4])
-    {
-        if (e0 + 4 <= n) {
-            *reinterpret_cast<float4 *>(o + e0) = make_float4(v[0], v[1], v[2], v[3]);
-        } else {
-            for (int k = 0; k < 4; k++)
-                if (e0 + k < n) o[e0 + k] = v[k];
-        }
-    }
-};
-template <> struct Store4<double> {
-    // plain stores (the fp64 tile decoder writes whole tiles through LDS
-    // instead; non-temporal stores here ran at 1.3-1.4 TB/s against 2.2-2.5)
-    __device__ static void store_full(double *o, uint64_t e0, const double v[4])
-    {
-        *reinterpret_cast<double2 *>(o + e0) = make_double2(v[0], v[1]);
-        *reinterpret_cast<double2 *>(o + e0 + 2) = make_double2(v[2], v[3]);
-    }
-    __device__ static void store(double *o, uint64_t e0, uint64_t n, const double v[4])
-    {
-        if (e0 + 4 <= n) {
-            *reinterpret_cast<double2 *>(o + e0) = make_double2(v[0], v[1]);
-            *reinterpret_cast<double2 *>(o + e0 + 2) = make_double2(v[2], v[3]);
-        } else {
-            for (int k = 0; k < 4; k++)
-                if (e0 + k < n) o[e0 + k] = v[k];
-        }
-    }
-};
-
-__device__ inline float be_f32(const uint8_t *p)
-{
-    return bits_f32(((uint32_t)p[0] << 24) | ((uint32_t)p[1] << 16) | ((uint32_t)p[2] << 8) |
-                    (uint32_t)p[3]);
-}
-
 // Exclusive prefix sum over the 64 lanes of a wave.
 __device__ inline uint32_t wave_excl_scan(uint32_t v, int lane)
 {
@@ -178,8 +134,9 @@ __device__ inline void stage_bytes(uint8_t *dst, const uint8_t *src, uint32_t nb
         if (g >= lo && g + 16 <= hi)
             *reinterpret_cast<uint4 *>(dst + 16 * c) = *reinterpret_cast<const uint4 *>(g);
     }
-    // the first and last chunks may be partial: one byte per thread
-    if (tid < 32 && nchunk) {
+    // a first or last chunk that leaves the buffer: one byte per thread
+    const uintptr_t last = a + 16 * (uintptr_t)nchunk;
+    if ((a < (uintptr_t)lo || last > (uintptr_t)hi) && tid < 32 && nchunk) {
         const uint32_t c = tid < 16 ? 0 : nchunk - 1;
         const uint32_t k = tid & 15;
         const uint8_t *g = reinterpret_cast<const uint8_t *>(a + 16 * (uintptr_t)c) + k;
@@ -189,9 +146,10 @@ __device__ inline void stage_bytes(uint8_t *dst, const uint8_t *src, uint32_t nb
 
 // Everything the slab decoder reads from the tile's LDS staging.
 struct TileLds {
-    const uint8_t *st;          // staged record bytes (16-byte aligned base)
-    uint32_t rdel;              // offset of the tile's first record byte in st
-    const uint8_t *meds;        // the tile's constant medians (big-endian)
+    const uint32_t *stw;        // staged record bytes
+    uint32_t rdel;              // offset of the tile's first record byte in them
+    const uint32_t *medw;       // staged constant medians (big-endian)
+    uint32_t mdel;              // offset of the tile's first median in them
     uint32_t nct, tb;           // constant blocks, record bytes of the tile
     const uint16_t *start;      // per block: record start / constant rank
     uint16_t *size;             // per block: decoded record size
@@ -202,125 +160,150 @@ struct TileLds {
 
 // Decode the LV values of one lane: lane lseg of the BS/LV lanes holding
 // block lb, first value e0.  FULL: the whole block lies inside the array.
-// KEEP: leave the values in vout for the caller to store (FULL only).
-template <typename T, int BS, int LV, bool FULL, bool KEEP = false>
+//
+// The kernel is bound by its VALU work as much as by memory, so the lead
+// codes are handled four values to a word: z[j] holds the codes of the lane's
+// values j, 4 + j, 8 + j, 12 + j, one per byte (two operations from the lane's
+// lead-code bytes), and byte sums of such words give every value's first mid
+// byte.  A value then costs one add for its position, two LDS words and a
+// byte funnel, and one bit-field insert (512^3 fp32, bs 128, whole call on cold
+// buffers: 0.159 -> 0.148 ms; 8192^2 fp64, bs 64: 0.149 -> 0.137 ms).
+template <typename T, int BS, int LV, bool FULL>
 __device__ inline void decode_lane(const TileLds &L, uint64_t e0, uint64_t n, int lb, int lane, int lseg,
-                                   T *out, int exact, T *vout = nullptr)
+                                   int exact, T (&v)[LV])
 {
     using U = typename Word<T>::U;
     constexpr int W = Word<T>::W;
     constexpr int SEG = BS / LV;
     constexpr int NLB = LV / 4;          // lead-code bytes per lane
-    static_assert(!KEEP || FULL, "kept values are whole blocks");
-    T v[LV];
+    static_assert(NLB <= 4 && LV * W < 256, "a lane's lead codes fit a word, its mid bytes a byte");
     if (!L.state[lb]) {
         const uint32_t rank = L.start[lb];
         float med = 0.0f;
         if (rank < L.nct) {
-            const uint8_t *p = L.meds + 4 * rank;
-            const uint32_t be = ((uint32_t)p[0] << 24) | ((uint32_t)p[1] << 16) | ((uint32_t)p[2] << 8) |
-                                (uint32_t)p[3];
-            med = bits_f32(L.medle ? bswap32(be) : be);
+            const uint32_t le = lds_window4(L.medw, L.mdel + 4 * rank);
+            med = bits_f32(L.medle ? le : bswap32(le));
         } else if (lseg == 0) {
             *L.err = 1;
         }
 #pragma unroll
         for (int k = 0; k < LV; k++) v[k] = (T)med;
-    } else {
-        const uint64_t bstart = e0 - (uint64_t)LV * lseg;
-        const int nel = FULL ? BS : (n - bstart >= (uint64_t)BS ? BS : (int)(n - bstart));
-        const int nlead = (nel + 3) >> 2;
-        const uint32_t start = L.start[lb];
-        const bool head_ok = start + 5u + (uint32_t)nlead <= L.tb;   // fixed part staged
-        const uint8_t *rec = L.st + L.rdel + (head_ok ? start : 0u);
-        const int rl = head_ok ? rec[0] : 1;
-        const bool rl_ok = head_ok && rl >= 1 && rl <= 8 * W;
-        const int rb = rl_ok ? (rl + 7) >> 3 : 1;
-        const int shift = (8 - (rl & 7)) & 7;
-        const int lo = W - rb;
-        const float med = bits_f32(((uint32_t)rec[1] << 24) | ((uint32_t)rec[2] << 16) |
-                                   ((uint32_t)rec[3] << 8) | (uint32_t)rec[4]);
-        uint32_t code[NLB];
+        return;
+    }
+    const uint64_t bstart = e0 - (uint64_t)LV * lseg;
+    const int nel = FULL ? BS : (n - bstart >= (uint64_t)BS ? BS : (int)(n - bstart));
+    const int nlead = (nel + 3) >> 2;
+    const uint32_t start = L.start[lb];
+    const bool head_ok = start + 5u + (uint32_t)nlead <= L.tb;   // fixed part staged
+    const uint32_t rec = L.rdel + (head_ok ? start : 0u);
+    const uint64_t hw = lds_window8(L.stw, rec);                 // reqLength, big-endian median
+    const int rl = head_ok ? (int)((uint32_t)hw & 0xFFu) : 1;
+    const bool rl_ok = head_ok && rl >= 1 && rl <= 8 * W;
+    const int rb = rl_ok ? (rl + 7) >> 3 : 1;
+    const int shift = (8 - (rl & 7)) & 7;
+    const float med = bits_f32(bswap32((uint32_t)(hw >> 8)));
+    // the lane's lead codes, capped at rb: a record of fewer than 3 bytes per
+    // value has no code above rb (3 -> 2, then 2 -> 1, two bits at a time)
+    const bool lead_ok = rl_ok && (FULL || lseg * NLB < nlead);
+    uint32_t code = lead_ok ? lds_window4(L.stw, rec + 5u + (uint32_t)(lseg * NLB)) : 0u;
+    if constexpr (NLB < 4) code &= (1u << (8 * NLB)) - 1u;
+    if constexpr (!FULL) {   // lead bytes and values past the array's end: no bytes
+        const int have = nlead - lseg * NLB;
+        code = have <= 0 ? 0u : have < NLB ? code & ((1u << (8 * have)) - 1u) : code;
+    }
+    code -= code & (code >> 1) & (rb <= 2 ? 0x55555555u : 0u);
+    code -= (code >> 1) & (rb <= 1 ? 0x55555555u : 0u);
+    // lead bytes z, 8 z, mid bytes m = rb - z and first-mid-byte offsets pk
+    // of value 4 b + j in byte b of word j
+    uint32_t z8[4], pk[4], m[4];
+    const uint32_t rbx = (uint32_t)rb * 0x01010101u;
 #pragma unroll
-        for (int b = 0; b < NLB; b++)
-            code[b] = (rl_ok && (lseg * NLB + b) < nlead) ? rec[5 + lseg * NLB + b] : 0u;
-        // lead bytes lk = min(code, rb) and mid bytes m = rb - lk per value
-        // (past the array end: no bytes)
-        uint32_t lk[LV], mk[LV], tot = 0;
+    for (int j = 0; j < 4; j++) {
+        const uint32_t z = (code >> (6 - 2 * j)) & 0x03030303u;
+        z8[j] = z << 3;
+        m[j] = rbx - z;
+        if constexpr (!FULL) {
+            uint32_t keep = 0;
+#pragma unroll
+            for (int b = 0; b < NLB; b++)
+                if (e0 + 4 * b + j < n) keep |= 0xFFu << (8 * b);
+            m[j] &= keep;
+        }
+    }
+    uint32_t bt = (m[0] + m[1]) + (m[2] + m[3]);   // per lead byte: mid bytes of its values
+    if constexpr (NLB >= 2) bt += bt << 8;
+    if constexpr (NLB >= 3) bt += bt << 16;
+    const uint32_t tot = (bt >> (8 * (NLB - 1))) & 0xFFu;
+    pk[0] = NLB >= 2 ? bt << 8 : 0u;
+#pragma unroll
+    for (int j = 1; j < 4; j++) pk[j] = pk[j - 1] + m[j - 1];
+
+    const uint32_t inc = seg_scan_incl<SEG>(tot, lane);
+    const uint32_t rsize = 5u + (uint32_t)nlead + seg_last<SEG>(inc);
+    const bool ok = rl_ok && start + rsize <= L.tb;
+    if (lseg == 0) {
+        if (ok) L.size[lb] = (uint16_t)rsize;
+        else *L.err = 1;
+    }
+    // A value's m bytes (from stage byte p on; a bad record reads from byte 0
+    // on and is flagged above) land on word bytes [W - rb, W - z): the
+    // gathered word shifted up by W - rb bytes supplies bytes [0, W - z)
+    // (zeros below), the value before it the top z <= 3 bytes -- one bit-field
+    // insert in the word's top 32 bits.  Bits the final shift drops are never
+    // masked.  This pass runs with a zero carry-in: hi[k] is the top of value
+    // k's word if nothing came from the previous lane; inh[k] marks the bytes
+    // it still inherits from before the lane.  At most 8 W bytes past the
+    // record's end are read, inside the stage.
+    const uint32_t p0 = ok ? rec + 5u + (uint32_t)nlead + (inc - tot) : 0u;
+    const int lo8 = 8 * (W - rb);
+    const uint8_t *stb = reinterpret_cast<const uint8_t *>(L.stw);
+    uint32_t hi[LV], inh[LV];
+    uint32_t lw[W == 8 ? LV : 1];
+    uint32_t tp = 0, ih = ~0u;
+    auto values = [&](auto byte7) {
 #pragma unroll
         for (int k = 0; k < LV; k++) {
-            const uint32_t ld = (code[k >> 2] >> (6 - 2 * (k & 3))) & 3u;
-            lk[k] = ld < (uint32_t)rb ? ld : (uint32_t)rb;
-            mk[k] = (FULL || e0 + k < n) ? (uint32_t)rb - lk[k] : 0u;
-            tot += mk[k];
-        }
-        const uint32_t inc = seg_scan_incl<SEG>(tot, lane);
-        const uint32_t rsize = 5u + (uint32_t)nlead + seg_last<SEG>(inc);
-        const bool ok = rl_ok && start + rsize <= L.tb;
-        if (lseg == 0) {
-            if (ok) L.size[lb] = (uint16_t)rsize;
-            else *L.err = 1;
-        }
-        // Value k's m bytes start at stage byte p (p runs through the lane's
-        // bytes; a bad record reads from byte 0 on and is flagged above).  They
-        // land on word bytes [W - rb, W - lk): the gathered word shifted up by
-        // lo = W - rb bytes supplies bytes [0, W - lk) (zeros below lo), value
-        // k-1 the top lk bytes -- one bit-field insert.  Bits the final shift
-        // drops are never masked.  Pass 1 runs with a zero carry-in: t0[k] is
-        // value k's word if nothing came from the previous lane; inh[k] marks
-        // the top bytes value k still inherits from before the lane.
-        // (two or three aligned LDS words and a byte funnel per value:
-        // unaligned LDS reads are slow)
-        const uint32_t *stw = reinterpret_cast<const uint32_t *>(L.st);
-        uint32_t p = ok ? (uint32_t)(rec - L.st) + 5u + (uint32_t)nlead + (inc - tot) : 0u;
-        const int lo8 = 8 * lo;
-        U t0[LV], inh[LV];
-        U tp = 0, ih = ~(U)0;
-#pragma unroll
-        for (int k = 0; k < LV; k++) {
-            const uint32_t *w = stw + (p >> 2);
-            const uint32_t sh = p & 3u;
-            U xk;
+            const int j = k & 3, b = 8 * (k >> 2);
+            const uint32_t p = p0 + ((pk[j] >> b) & 0xFFu);
+            const uint32_t z = (z8[j] >> b) & 0xFFu;
+            const uint32_t *w = reinterpret_cast<const uint32_t *>(stb + (p & ~3u));
+            uint32_t xh;
             if constexpr (W == 4) {
-                xk = __builtin_amdgcn_alignbyte(w[1], w[0], sh);
+                xh = __builtin_amdgcn_alignbyte(w[1], w[0], p) << lo8;
             } else {
                 const uint32_t d0 = w[0], d1 = w[1], d2 = w[2];
-                xk = (U)__builtin_amdgcn_alignbyte(d1, d0, sh) | ((U)__builtin_amdgcn_alignbyte(d2, d1, sh) << 32);
+                const uint32_t x0 = __builtin_amdgcn_alignbyte(d1, d0, p);
+                const U xs = ((U)x0 | ((U)__builtin_amdgcn_alignbyte(d2, d1, p) << 32)) << lo8;
+                xh = (uint32_t)(xs >> 32);
+                lw[k] = (uint32_t)xs;
+                if constexpr (decltype(byte7)::value) {   // szxd_double.cc:244 reads q[3]
+                    if (rb == 5 && z == 0 && ((m[j] >> b) & 0xFFu)) xh = (xh & 0xFFFFFFu) | (x0 & 0xFF000000u);
+                }
             }
-            U xs = xk << lo8;
-            if constexpr (W == 8) {
-                if (!exact && rb == 5 && lk[k] == 0 && mk[k])   // szxd_double.cc:244 reads q[3]
-                    xs = (xs & ~((U)0xFF << 56)) | (((xk >> 24) & 0xFF) << 56);
-            }
-            const U take = ~(U)0 >> (lk[k] << 3);   // bytes below W - lk
-            tp = (xs & take) | (tp & ~take);
+            const uint32_t take = ~0u >> z;   // bytes below W - z
+            tp = (xh & take) | (tp & ~take);
             ih &= ~take;
-            t0[k] = tp;
+            hi[k] = tp;
             inh[k] = ih;
-            p += mk[k];   // at most 8 W bytes past the start, inside the stage
         }
-        // the lane's copyable bytes W-3..W-1: the ones it wrote (no longer
-        // inherited) and their values; a last-writer scan over the segment
-        // then gives every lane what it inherits from the lanes before it
-        const uint32_t wm = ~(uint32_t)(ih >> (8 * (W - 3))) & 0xFFFFFFu;
-        uint32_t cd = (uint32_t)(tp >> (8 * (W - 3))) & wm, cm = wm;
-        seg_scan_last_writer<SEG>(cd, cm, lane);
-        const uint32_t cin = seg_prev<SEG>(cd, lane);
-        const U cw = (U)cin << (8 * (W - 3));
-        const T mT = (T)med;
+    };
+    if (W == 8 && !exact && __builtin_amdgcn_ballot_w64(rb == 5) != 0)
+        values(std::true_type{});
+    else
+        values(std::false_type{});
+    // the lane's top bytes and which of them it wrote; a last-writer scan over
+    // the segment gives every lane what it inherits from the lanes before it.
+    // The segment's first lane counts as having written all of them (a block
+    // starts from a zero word), so nothing crosses segments.
+    uint32_t cd = tp, cm = lseg == 0 ? ~0u : ~ih;
+    seg_scan_last_writer_head<SEG>(cd, cm);
+    const uint32_t cin = seg_prev<SEG>(cd, lane);
+    const T mT = (T)med;
 #pragma unroll
-        for (int k = 0; k < LV; k++) v[k] = from_bits<T>((t0[k] | (cw & inh[k])) << shift) + mT;
-    }
-    if (KEEP) {
-#pragma unroll
-        for (int k = 0; k < LV; k++) vout[k] = v[k];
-    } else if (FULL) {
-#pragma unroll
-        for (int k = 0; k < LV; k += 4) Store4<T>::store_full(out, e0 + k, v + k);
-    } else {
-#pragma unroll
-        for (int k = 0; k < LV; k++)
-            if (e0 + k < n) out[e0 + k] = v[k];
+    for (int k = 0; k < LV; k++) {
+        const uint32_t h = hi[k] | (cin & inh[k]);
+        if constexpr (W == 4) v[k] = from_bits<T>(h << shift) + mT;
+        else v[k] = from_bits<T>((((U)h << 32) | lw[k]) << shift) + mT;
     }
 }
 
@@ -352,6 +335,16 @@ struct TileSrc {
     uint32_t field, tile;       // batched decode: the field and its tile
     uint32_t medle, pad;
 };
+
+// Values per lane of the tile decoder: a lane's fixed work (record header,
+// block scans, last-writer scan) is shared by as many values as its lead codes
+// fit one word -- 16 for fp32 (an index tile of 4096 values is one slab of 256
+// lanes; 512^3, bs 128: 0.148 ms with 8, 0.144 with 16) -- while the 2048
+// values of an fp64 tile give every lane 8.
+constexpr int decode_lv(int w, int bs)
+{
+    return w == 4 && bs >= 16 ? 16 : bs >= 8 ? 8 : 4;
+}
 
 template <typename T, int BS, int LV> struct DecodeShape {
     static constexpr int W = Word<T>::W;
@@ -473,58 +466,61 @@ __device__ inline void decode_tile_core(const DecodeParams &p, uint64_t tile, co
     }
     __syncthreads();
 
-    const TileLds L{st, rdel, s_med + mdel, nct, tb, s_start, s_size, s_state, &s_err, (int)ts.medle};
+    const TileLds L{reinterpret_cast<const uint32_t *>(st), rdel, reinterpret_cast<const uint32_t *>(s_med), mdel,
+                    nct, tb, s_start, s_size, s_state, &s_err, (int)ts.medle};
     const bool full = (tile + 1) * (uint64_t)TILE <= n;
-    if (full && sizeof(T) == 8) {
-        // fp64: a lane's values are 8 LV consecutive bytes, and its own four
-        // 16-byte stores per 8 values leave every line partly written per
-        // instruction.  The tile's values go through the stage instead (free
-        // once every lane has decoded) and out in whole 16-byte chunks
-        // across the wave, non-temporal (8192^2 fp64: 0.214 -> 0.118 ms;
-        // fp32, whose lanes write 32 bytes each, gains nothing from it).
+    if (full) {
+        // A lane's values are up to 64 consecutive bytes, and its own 16-byte
+        // stores would leave every line partly written per instruction.  The
+        // tile's values go through the stage instead (free once every lane
+        // has decoded) and out in whole 16-byte chunks across the wave,
+        // non-temporal (8192^2 fp64: 0.214 -> 0.118 ms on warm buffers; fp32
+        // 512^3 on cold ones, its stream and output read and written for the
+        // first time: 0.177 -> 0.159 ms).  The chunks of a row of eight are
+        // permuted (slot) so that lanes 64 bytes apart use different banks.
         T vv[SLABS][LV];
 #pragma unroll
         for (int u = 0; u < SLABS; u++) {
             const uint64_t e0 = tile * TILE + (uint64_t)u * SLAB + (uint64_t)LV * tid;
-            decode_lane<T, BS, LV, true, true>(L, e0, n, u * BPS + tid / SEG, lane, lseg, out, exact, vv[u]);
+            decode_lane<T, BS, LV, true>(L, e0, n, u * BPS + tid / SEG, lane, lseg, exact, vv[u]);
         }
         __syncthreads();
         static_assert(TILE * (int)sizeof(T) <= STAGE, "the tile's values fit the stage");
         typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
-        T *so = reinterpret_cast<T *>(st);
+        constexpr int VC = 16 / (int)sizeof(T);   // values per chunk
+        u32x4_t *sv = reinterpret_cast<u32x4_t *>(st);
+        const auto slot = [](int c) { return c ^ ((c >> 3) & 3); };
 #pragma unroll
         for (int u = 0; u < SLABS; u++)
 #pragma unroll
-            for (int k = 0; k < LV; k += 16 / (int)sizeof(T)) {
+            for (int k = 0; k < LV; k += VC) {
                 u32x4_t w;
                 __builtin_memcpy(&w, &vv[u][k], 16);
-                *reinterpret_cast<u32x4_t *>(so + u * SLAB + LV * tid + k) = w;
+                sv[slot((u * SLAB + LV * tid + k) / VC)] = w;
             }
         __syncthreads();
-        const u32x4_t *sv = reinterpret_cast<const u32x4_t *>(so);
         u32x4_t *ov = reinterpret_cast<u32x4_t *>(out + tile * TILE);
-        constexpr int CHUNKS = TILE * (int)sizeof(T) / 16;
+        constexpr int CHUNKS = TILE / VC;
 #pragma unroll
-        for (int c = tid; c < CHUNKS; c += 256) __builtin_nontemporal_store(sv[c], ov + c);
+        for (int c = tid; c < CHUNKS; c += 256) __builtin_nontemporal_store(sv[slot(c)], ov + c);
     } else {
 #pragma unroll
         for (int u = 0; u < SLABS; u++) {
             const uint64_t e0 = tile * TILE + (uint64_t)u * SLAB + (uint64_t)LV * tid;
-            const int lb = u * BPS + tid / SEG;
-            if (full) {
-                decode_lane<T, BS, LV, true>(L, e0, n, lb, lane, lseg, out, exact);
-            } else {
-                if (e0 - (uint64_t)LV * lseg >= n) continue;   // the whole block is past the end
-                decode_lane<T, BS, LV, false>(L, e0, n, lb, lane, lseg, out, exact);
-            }
+            if (e0 - (uint64_t)LV * lseg >= n) continue;   // the whole block is past the end
+            T vp[LV];
+            decode_lane<T, BS, LV, false>(L, e0, n, u * BPS + tid / SEG, lane, lseg, exact, vp);
+#pragma unroll
+            for (int k = 0; k < LV; k++)
+                if (e0 + k < n) out[e0 + k] = vp[k];
         }
+        __syncthreads();
     }
-    __syncthreads();
 
     // the index must be what the records say: starts are the exclusive scan
     // of the record sizes, constant ranks count the constant blocks, and the
     // tile's records and medians end where the next tile's begin
-    if (tid < 64) {
+    if (tid < 64) {   // every lane's records are decoded: a barrier lies behind
         uint32_t bytes = 0, consts = 0;
 #pragma unroll
         for (int k = 0; k < PER_LANE; k++) {
@@ -550,10 +546,8 @@ __device__ inline void decode_tile_core(const DecodeParams &p, uint64_t tile, co
             }
         }
         if (lane == 63) bad |= eb != tb || ec != nct;
-        if (__ballot(bad) && lane == 0) s_err = 1;
+        if ((__ballot(bad) || s_err) && lane == 0) atomicMin(status, -21);
     }
-    __syncthreads();
-    if (s_err && tid == 0) atomicMin(status, -21);
 }
 
 template <typename T, int BS, int LV>
@@ -585,12 +579,12 @@ __global__ void k_decode_header_batch(const BatchDecodeField *f, int nf, int bs)
 // Every tile's bytes (tile_src), one thread per tile, so that a decode
 // workgroup starts staging its records after one load (the field's result
 // words, header and index entries are resolved here, off its path).
-template <int BS, int LV>
+template <int BS, int LVF, int LVD>
 __global__ __launch_bounds__(256) void k_decode_setup_batch(const BatchDecodeField *f, const uint64_t *tbase,
                                                             const uint32_t *tmap, TileSrc *recs, uint64_t total)
 {
-    using S32 = DecodeShape<float, BS, LV>;
-    using S64 = DecodeShape<double, BS, LV>;
+    using S32 = DecodeShape<float, BS, LVF>;
+    using S64 = DecodeShape<double, BS, LVD>;
     const uint64_t g = blockIdx.x * 256ull + threadIdx.x;
     if (g >= total) return;
     const uint32_t fi = tmap[g];   // the field holding tile g
@@ -604,30 +598,30 @@ __global__ __launch_bounds__(256) void k_decode_setup_batch(const BatchDecodeFie
     recs[g] = r;
 }
 
-template <int BS, int LV>
+template <int BS, int LVF, int LVD>
 __global__ __launch_bounds__(256) void k_decode_batch(const BatchDecodeField *f, const TileSrc *recs, int exact)
 {
     __shared__ union Lds {
-        DecodeLds<float, BS, LV> f;
-        DecodeLds<double, BS, LV> d;
+        DecodeLds<float, BS, LVF> f;
+        DecodeLds<double, BS, LVD> d;
     } lds;
     const TileSrc r = recs[blockIdx.x];
     const BatchDecodeField &d = f[r.field];
     // the core reads only the values count, status, output and mode of p
     const DecodeParams p{nullptr, 0, d.n, nullptr, nullptr, nullptr, d.status, d.dst, exact};
-    if (d.w == 4) decode_tile_core<float, BS, LV>(p, r.tile, r, lds.f);
-    else decode_tile_core<double, BS, LV>(p, r.tile, r, lds.d);
+    if (d.w == 4) decode_tile_core<float, BS, LVF>(p, r.tile, r, lds.f);
+    else decode_tile_core<double, BS, LVD>(p, r.tile, r, lds.d);
 }
 
 template <int BS>
 static void launch_decode_batch(const BatchDecodeField *f, const uint64_t *tbase, const uint32_t *tmap,
                                 TileSrc *recs, uint64_t total, int exact, hipStream_t st)
 {
-    constexpr int LV = BS >= 8 ? 8 : 4;
+    constexpr int LVF = decode_lv(4, BS), LVD = decode_lv(8, BS);
     if (!total) return;
-    hipLaunchKernelGGL((k_decode_setup_batch<BS, LV>), dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, f,
+    hipLaunchKernelGGL((k_decode_setup_batch<BS, LVF, LVD>), dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, f,
                        tbase, tmap, recs, total);
-    hipLaunchKernelGGL((k_decode_batch<BS, LV>), dim3((unsigned)total), dim3(256), 0, st, f, recs, exact);
+    hipLaunchKernelGGL((k_decode_batch<BS, LVF, LVD>), dim3((unsigned)total), dim3(256), 0, st, f, recs, exact);
 }
 
 uint64_t batch_decode_records_bytes(uint64_t total) { return total * sizeof(TileSrc); }
@@ -669,9 +663,7 @@ static void launch_decode(const uint8_t *s, uint64_t len, uint64_t n, const Deco
                           const uint64_t *index, int32_t *status, void *out, int exact,
                           uint64_t ntiles, hipStream_t st)
 {
-    // 8 values per lane where a block spans at least 8 values (fp64 tiles of
-    // 2048 values take one slab of 256 x 8), else 4
-    constexpr int LV = BS >= 8 ? 8 : 4;
+    constexpr int LV = decode_lv((int)sizeof(T), BS);
     const DecodeParams p{s, len, n, h, index,
                          reinterpret_cast<const uint16_t *>(index + 2 * (ntiles + 1)), status, out,
                          exact};

@@ -165,6 +165,28 @@ __device__ inline void seg_scan_last_writer(uint32_t &d, uint32_t &m, int lane)
 #undef SZX_LW_STEP
 }
 
+// The same scan where the first lane of every segment has marked all bytes as
+// written: then nothing crosses a segment's start, and no lane predicate is
+// needed for segments shorter than a row either.
+template <int SEG>
+__device__ inline void seg_scan_last_writer_head(uint32_t &d, uint32_t &m)
+{
+#define SZX_LW_STEP(CTRL, RM)                                           \
+    {                                                                   \
+        const uint32_t od = dpp32<CTRL, RM>(0u, d);                     \
+        const uint32_t om = dpp32<CTRL, RM>(0u, m);                     \
+        d = (d & m) | (od & ~m);                                        \
+        m |= om;                                                        \
+    }
+    if constexpr (SEG >= 2) SZX_LW_STEP(DPP_ROW_SHR(1), 0xF)
+    if constexpr (SEG >= 4) SZX_LW_STEP(DPP_ROW_SHR(2), 0xF)
+    if constexpr (SEG >= 8) SZX_LW_STEP(DPP_ROW_SHR(4), 0xF)
+    if constexpr (SEG >= 16) SZX_LW_STEP(DPP_ROW_SHR(8), 0xF)
+    if constexpr (SEG >= 32) SZX_LW_STEP(DPP_ROW_BCAST15, 0xA)
+    if constexpr (SEG >= 64) SZX_LW_STEP(DPP_ROW_BCAST31, 0xC)
+#undef SZX_LW_STEP
+}
+
 // Value held by lane-1 (0 in the first lane of each segment).
 template <int SEG, typename V>
 __device__ inline V seg_prev(V v, int lane)

@@ -423,3 +423,36 @@ def test_copy_kernel(device):
         Z.copy_dev(torch.zeros(6, dtype=torch.int8, device=device), torch.zeros(6, dtype=torch.int8, device=device))
     with pytest.raises(Z.SZxError):
         Z.copy_dev(torch.zeros(16, device=device), torch.zeros(8, device=device))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("bs", POW2)
+def test_decode_tile_edges(bs, dtype, device):
+    """Whole, partial and one-value tiles; records of one to all bytes per
+    value; streams that start and end at any byte of their buffer."""
+    import torch
+    r = np.random.default_rng(bs)
+    tile = 4096 if dtype == np.float32 else 2048
+    t = np.arange(3 * tile + 3)
+    base = np.where(t // 700 % 3 == 0, 0.5, np.sin(t * 0.013) + r.standard_normal(t.size) * 1e-3).astype(dtype)
+    for n in (1, tile - 1, tile, tile + bs // 2 + 1, 3 * tile + 3):
+        for eb in (0.4, 1e-2, 1e-4, 1e-12):
+            x = base[:n]
+            say("tile edge", dtype.__name__, bs, n, eb)
+            comp = Z.DeviceCompressor(n, dtype, bs)
+            comp(torch.from_numpy(x).to(device), Z.ABS, eb)
+            view, _, size, _ = comp.stream_view()
+            s = view.cpu().numpy().tobytes()
+            assert s == O.compress(x, float(np.float32(eb)), bs)
+            for at in (0, 5):
+                buf = torch.empty(at + size, dtype=torch.uint8, device=device)
+                buf[at:] = view
+                for index in (comp.index, None):
+                    dec = Z.DeviceDecompressor(n, dtype, bs, size)
+                    dec.out.fill_(-7.0)
+                    dec(buf[at:], size, Z.DECODE_REFERENCE, index=index)
+                    assert dec.check() == 0
+                    assert bits_equal(dec.out.cpu().numpy(), O.decompress(s, n, dtype, ref_quirk=True))
+                    dec(buf[at:], size, Z.DECODE_EXACT, index=index)
+                    assert dec.check() == 0
+                    assert bits_equal(dec.out.cpu().numpy(), O.decompress(s, n, dtype, ref_quirk=False))
