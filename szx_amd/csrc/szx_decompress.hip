@@ -123,26 +123,55 @@ __device__ inline uint32_t wave_excl_scan(uint32_t v, int lane)
 // Copy bytes [src, src + nbytes) of global memory into LDS at dst + (src & 15)
 // (dst 16-byte aligned): 16-byte loads for the aligned chunks that lie wholly
 // inside [lo, hi) -- the caller's buffer -- and single bytes for the rest.
-__device__ inline void stage_bytes(uint8_t *dst, const uint8_t *src, uint32_t nbytes,
-                                   const uint8_t *lo, const uint8_t *hi, int tid)
-{
-    const uintptr_t a = (uintptr_t)src & ~(uintptr_t)15;
-    const uint32_t head = (uint32_t)((uintptr_t)src - a);
-    const uint32_t nchunk = (head + nbytes + 15) / 16;
-    for (uint32_t c = tid; c < nchunk; c += 256) {
-        const uint8_t *g = reinterpret_cast<const uint8_t *>(a + 16 * (uintptr_t)c);
-        if (g >= lo && g + 16 <= hi)
-            *reinterpret_cast<uint4 *>(dst + 16 * c) = *reinterpret_cast<const uint4 *>(g);
+// In two halves, so that a tile's loads are all in flight before the first of
+// them is waited for: load() issues a lane's first N chunks, store() puts them
+// in LDS and copies what is left.  (A tile's life was a chain of four or five
+// memory round trips -- header, index, chunk after chunk of records, medians,
+// bitmap and block entries -- and is now two; whole calls on cold buffers,
+// 512^3 fp32 bs 128: 0.144 -> 0.117 ms, 6.0 TB/s; 8192^2 fp64 bs 64: 0.137 ->
+// 0.113 ms.  The copy kernel takes 0.108 ms for these bytes.)
+template <int N> struct StageCopy {
+    typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
+    using G16 = const __attribute__((address_space(1))) u32x4_t *;   // global, not flat, loads
+    u32x4_t v[N];
+    uint64_t a;                  // address of chunk 0
+    uint32_t c0, c1, nchunk;     // chunks [c0, c1) lie inside the buffer
+    const uint8_t *lo, *hi;
+    __device__ u32x4_t chunk(uint32_t c) const { return *(G16)(a + 16ull * c); }
+    __device__ bool whole(uint32_t c) const { return c >= c0 && c < c1; }
+    __device__ void load(const uint8_t *src, uint32_t nbytes, const uint8_t *lo_, const uint8_t *hi_, int tid)
+    {
+        a = (uint64_t)src & ~15ull;
+        nchunk = nbytes ? ((uint32_t)((uint64_t)src - a) + nbytes + 15) / 16 : 0u;
+        lo = lo_;
+        hi = hi_;
+        // only the first and the last chunk can stick out (src .. src + nbytes is inside)
+        c0 = a < (uint64_t)lo ? 1u : 0u;
+        c1 = nchunk && a + 16ull * nchunk > (uint64_t)hi ? nchunk - 1 : nchunk;
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            const uint32_t c = (uint32_t)tid + 256u * i;
+            if (whole(c)) v[i] = chunk(c);
+        }
     }
-    // a first or last chunk that leaves the buffer: one byte per thread
-    const uintptr_t last = a + 16 * (uintptr_t)nchunk;
-    if ((a < (uintptr_t)lo || last > (uintptr_t)hi) && tid < 32 && nchunk) {
-        const uint32_t c = tid < 16 ? 0 : nchunk - 1;
-        const uint32_t k = tid & 15;
-        const uint8_t *g = reinterpret_cast<const uint8_t *>(a + 16 * (uintptr_t)c) + k;
-        if (g >= lo && g < hi) dst[16 * c + k] = *g;
+    __device__ void store(uint8_t *dst, int tid)
+    {
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            const uint32_t c = (uint32_t)tid + 256u * i;
+            if (whole(c)) *reinterpret_cast<u32x4_t *>(dst + 16 * c) = v[i];
+        }
+        for (uint32_t c = (uint32_t)tid + 256u * N; c < c1; c += 256)
+            *reinterpret_cast<u32x4_t *>(dst + 16 * c) = chunk(c);
+        // a first or last chunk that leaves the buffer: one byte per thread
+        if ((c0 != 0 || c1 != nchunk) && nchunk && tid < 32) {
+            const uint32_t c = tid < 16 ? 0 : nchunk - 1;
+            const uint32_t k = tid & 15;
+            const uint8_t *g = reinterpret_cast<const uint8_t *>(a + 16ull * c) + k;
+            if (g >= lo && g < hi) dst[16 * c + k] = *g;
+        }
     }
-}
+};
 
 // Everything the slab decoder reads from the tile's LDS staging.
 struct TileLds {
@@ -370,35 +399,29 @@ template <int NBLK, int STAGE>
 __device__ inline TileSrc tile_src(const DecodeParams &p, uint64_t tile)
 {
     TileSrc t{};
-    const DecodeHeader *h = p.h;
-    // gate on the header check, which an earlier kernel wrote
-    if (h->rc != 0) {
-        t.flags = 1;
-        return t;
-    }
-    const uint64_t *index = p.index;
-    const uint64_t nb = h->nb, q0 = h->q0, nconst = h->nconst;
+    // The header and the index entries in one round trip: no branch between
+    // their loads (the index is readable whatever the header check says, and
+    // what is computed from a bad one is not used).
+    const DecodeHeader h = *p.h;
+    const uint64_t *index = p.index + 2 * tile;
+    const uint64_t rel = index[0], cbase = index[1], rend = index[2], cend = index[3];
     const uint64_t gb0 = tile * NBLK;
-    const uint64_t off = q0 + index[2 * tile];
-    const uint64_t end = q0 + index[2 * tile + 2];
-    const uint64_t cbase = index[2 * tile + 1];
-    const uint64_t cend = index[2 * tile + 3];
-    if (end < off || end > p.len || end - off > (uint64_t)STAGE || cend < cbase ||
-        cend - cbase > (uint64_t)NBLK || cend > nconst) {
-        t.flags = 2;
-        return t;
-    }
+    const uint64_t off = h.q0 + rel;
+    const uint64_t end = h.q0 + rend;
+    const bool bad = (end < off) | (end > p.len) | (end - off > (uint64_t)STAGE) | (cend < cbase) |
+                     (cend - cbase > (uint64_t)NBLK) | (cend > h.nconst);
     t.rsrc = p.s + off;
-    t.msrc = p.s + h->qmed + 4 * cbase;   // inside [0, q0) <= len
+    t.msrc = p.s + h.qmed + 4 * cbase;   // inside [0, q0) <= len
     t.lo = p.s;
     t.hi = p.s + p.len;
-    t.bmp = p.s + h->qbit + (gb0 >> 3);   // NBLK is a multiple of 8
+    t.bmp = p.s + h.qbit + (gb0 >> 3);   // NBLK is a multiple of 8
     t.bidx = p.bidx + gb0;
     t.tb = (uint32_t)(end - off);
     t.nct = (uint32_t)(cend - cbase);
-    t.nvb = gb0 >= nb ? 0u : (nb - gb0 < (uint64_t)NBLK ? (uint32_t)(nb - gb0) : (uint32_t)NBLK);
-    t.medle = (uint32_t)h->medle;
-    t.flags = 0;
+    t.nvb = gb0 >= h.nb ? 0u : (h.nb - gb0 < (uint64_t)NBLK ? (uint32_t)(h.nb - gb0) : (uint32_t)NBLK);
+    t.medle = (uint32_t)h.medle;
+    // gate on the header check, which an earlier kernel wrote
+    t.flags = h.rc != 0 ? 1u : bad ? 2u : 0u;
     return t;
 }
 
@@ -444,10 +467,9 @@ __device__ inline void decode_tile_core(const DecodeParams &p, uint64_t tile, co
     // kernels wrote, so every thread of the workgroup takes the same branch
     // (the status word itself may change while this kernel runs: other
     // tiles report into it).
-    if (ts.flags == 1) return;
     const int tid = threadIdx.x;
     if (ts.flags != 0) {
-        if (tid == 0) atomicMin(status, -20);
+        if (ts.flags != 1 && tid == 0) atomicMin(status, -20);
         return;
     }
     const int lane = tid & 63;
@@ -457,12 +479,30 @@ __device__ inline void decode_tile_core(const DecodeParams &p, uint64_t tile, co
     const uint8_t *msrc = ts.msrc;
     const uint32_t rdel = (uint32_t)((uintptr_t)rsrc & 15), mdel = (uint32_t)((uintptr_t)msrc & 15);
     if (tid == 0) s_err = 0;
-    stage_bytes(st, rsrc, tb, ts.lo, ts.hi, tid);
-    stage_bytes(s_med, msrc, 4 * nct, ts.lo, ts.hi, tid);
-    for (int lb = tid; lb < NBLK; lb += 256) {
-        s_state[lb] = (uint32_t)lb < nvb ? (ts.bmp[lb >> 3] >> (7 - (lb & 7))) & 1 : 0;
-        s_start[lb] = (uint32_t)lb < nvb ? ts.bidx[lb] : 0;
-        s_size[lb] = 0;
+    // two chunks per lane cover 8 KiB of records (2x compression and above)
+    StageCopy<2> recs;
+    StageCopy<1> meds;
+    static_assert(NBLK <= 4 * 256, "up to four blocks per lane");
+    constexpr int BPL = (NBLK + 255) / 256;
+    recs.load(rsrc, tb, ts.lo, ts.hi, tid);
+    meds.load(msrc, 4 * nct, ts.lo, ts.hi, tid);
+    uint32_t bit[BPL], ent[BPL];
+#pragma unroll
+    for (int i = 0; i < BPL; i++) {
+        const uint32_t lb = (uint32_t)tid + 256u * i;
+        bit[i] = lb < nvb ? ts.bmp[lb >> 3] : 0u;
+        ent[i] = lb < nvb ? ts.bidx[lb] : 0u;
+    }
+    recs.store(st, tid);
+    meds.store(s_med, tid);
+#pragma unroll
+    for (int i = 0; i < BPL; i++) {
+        const int lb = tid + 256 * i;
+        if (lb < NBLK) {
+            s_state[lb] = (uint8_t)((bit[i] >> (7 - (lb & 7))) & 1);
+            s_start[lb] = (uint16_t)ent[i];
+            s_size[lb] = 0;
+        }
     }
     __syncthreads();
 
