@@ -9,14 +9,15 @@
 // single-field compress at the same arguments.
 //
 // Launch sequence of a batched compress:
-//   k_zero_batch      clear look-back words, totals, error flags (flattened)
-//   k_batch_range     REL fields only: min/max of 2^20-value items
+//   k_batch_prepare   clear look-back words, totals, error flags (flattened);
+//                     REL fields: min/max per item
 //   k_batch_range_final   per REL field: the bound, rounded as the reference
 //   k_compress_batch  one workgroup per tile of the global tile list
 //   k_assemble_batch  header, bitmap, constant medians (flattened)
 // and of a batched decompress:
-//   k_decode_header_batch, k_decode_batch (one workgroup per index tile of
-//   every field, the streams located through the result words).
+//   k_decode_setup_batch (header checks and every tile's bytes, the streams
+//   located through the result words), k_decode_batch (one workgroup per index
+//   tile of every field).
 //
 // The tile shape of k_compress_batch (values per lane, index tiles per
 // workgroup tile) is chosen per batch by szx_amd_batch_tune, which times every
@@ -63,7 +64,7 @@ struct FieldSlot {
     CompressLayout L;
     uint64_t ws;      // single-field compress workspace (compress_layout)
     uint64_t index;   // record index
-    uint64_t hdr;     // decode header (256 bytes)
+    uint64_t hdr;     // decode header (256 bytes), per-field decodes
     uint64_t nidx;    // index tiles
     uint64_t ntiles[3];
     uint64_t range_items;
@@ -74,7 +75,7 @@ struct FieldSlot {
 
 struct Layout {
     uint64_t bf, df, bases, res, status, part, fields, dmap, drec, cmap[3], bytes;
-    uint64_t total[3] = {0, 0, 0}, nitems = 0, dtotal = 0, zitems = 0, aitems = 0;
+    uint64_t total[3] = {0, 0, 0}, nitems = 0, item = 0, dtotal = 0, zitems = 0, aitems = 0;
     std::vector<FieldSlot> slot;
 };
 
@@ -95,6 +96,10 @@ bool plan_layout(const szx_amd_field *f, int nf, int bs, Layout &Y)
     Y.bases = off;  off = al(off + NBASE * (nf + 1) * sizeof(uint64_t));
     Y.res = off;    off = al(off + 4 * (uint64_t)nf * sizeof(uint64_t));
     Y.status = off; off = al(off + (uint64_t)nf * sizeof(int32_t));
+    uint64_t rel_values = 0;
+    for (int i = 0; i < nf; i++)
+        if (f[i].errBoundMode == REL) rel_values += f[i].n;
+    Y.item = range_item_values(rel_values);
     for (int i = 0; i < nf; i++) {
         FieldSlot &s = Y.slot[i];
         s.w = width_of(f[i].dataType);
@@ -110,7 +115,7 @@ bool plan_layout(const szx_amd_field *f, int nf, int bs, Layout &Y)
         s.ntiles[0] = s.nidx;
         s.ntiles[1] = (n + INDEX_PER_TILE * tile_values(s.w) - 1) / (INDEX_PER_TILE * tile_values(s.w));
         s.ntiles[2] = (n + INDEX_PER_TILE_WIDE * tile_values(s.w) - 1) / (INDEX_PER_TILE_WIDE * tile_values(s.w));
-        s.range_items = f[i].errBoundMode == REL ? (n + RANGE_ITEM - 1) / RANGE_ITEM : 0;
+        s.range_items = f[i].errBoundMode == REL ? (n + Y.item - 1) / Y.item : 0;
         s.zero_items = ((s.L.ws_misc + 64 * sizeof(uint64_t)) / 8 + ZERO_ITEM - 1) / ZERO_ITEM;
         const uint64_t work = s.L.nbit > 4 * s.L.nb ? s.L.nbit : 4 * s.L.nb;
         uint64_t blocks = (work + 256 * ASSEMBLE_BYTES_PER_THREAD - 1) / (256 * ASSEMBLE_BYTES_PER_THREAD);
@@ -304,9 +309,8 @@ int enqueue_compress(szx_amd_batch *b, int mode, hipStream_t st)
         return hip_ok(hipGetLastError(), "launch") ? SZx_SCES : SZx_NSCS;
     }
     if (mode != SZX_AMD_BATCH_FUSED) { api_error("unknown batch mode %d", mode); return SZx_NSCS; }
-    batch_zero_launch(b->d_bf(), b->d_base(4), b->nf, Y.zitems, st);
-    if (Y.nitems) batch_range_launch(b->d_bf(), b->d_base(2), b->nf, Y.nitems,
-                                     reinterpret_cast<double *>(b->work + Y.part), st);
+    batch_prepare_launch(b->d_bf(), b->d_base(4), Y.zitems, b->d_base(2), b->nf, Y.nitems, Y.item,
+                         reinterpret_cast<double *>(b->work + Y.part), st);
     timing_mark_begin(KK_COMPRESS, st);
     const int rc = batch_compress_launch(b->bs, b->lv, b->ipt, b->d_bf(), b->d_base(tbase_slot(b->ipt)),
                                          b->d_cmap(tile_slot(b->ipt)), Y.total[tile_slot(b->ipt)], st);
@@ -428,7 +432,6 @@ szx_amd_batch *szx_amd_batch_create(const szx_amd_field *fields, int nfields, in
         D.index = p.index;
         D.dst = f.d_dec;
         D.status = b->d_status() + i;
-        D.h = reinterpret_cast<DecodeHeader *>(b->work + s.hdr);
         D.ntidx = s.nidx;
         D.w = s.w;
 
@@ -534,7 +537,7 @@ int szx_amd_batch_decompress(szx_amd_batch *b, int flags, int mode, void *hipStr
     }
     if (mode != SZX_AMD_BATCH_FUSED) { api_error("unknown batch mode %d", mode); return SZx_NSCS; }
     timing_mark_begin(KK_DECODE, st);
-    const int rc = batch_decode_launch(b->bs, b->d_df(), b->d_base(3), b->d_dmap(), b->work + b->Y.drec, b->nf,
+    const int rc = batch_decode_launch(b->bs, b->d_df(), b->d_base(3), b->d_dmap(), b->work + b->Y.drec,
                                        b->Y.dtotal, exact, st);
     timing_mark_end(KK_DECODE, st);
     if (rc) { api_error("unsupported blockSize"); return SZx_NSCS; }

@@ -61,8 +61,20 @@ struct AssembleParams {
 // partials the compressor folds itself.
 constexpr int RANGE_LB_PARTS = 256;
 
-// Values per REL range item of the batched range pass.
-constexpr uint64_t RANGE_ITEM = 1ull << 20;
+// Values per REL range item (one workgroup of 256 lanes) of the batched range
+// pass: a power of two, as large as leaves RANGE_ITEMS_WANTED workgroups over
+// the batch (eight per CU), between the bounds.  A fixed 2^20 left a 280 MB
+// batch of 30 fields with 90 workgroups and 0.235 ms for the pass (1.2 TB/s);
+// the large batches keep 2^20 (6.3 TB/s over 34.6 GB), below 2^14 a workgroup
+// would hold less than one sweep of its lanes' loads.
+constexpr uint64_t RANGE_ITEM_MIN = 1ull << 14, RANGE_ITEM_MAX = 1ull << 20;
+constexpr uint64_t RANGE_ITEMS_WANTED = 2048;
+inline uint64_t range_item_values(uint64_t values)
+{
+    uint64_t v = RANGE_ITEM_MAX;
+    while (v > RANGE_ITEM_MIN && values / v < RANGE_ITEMS_WANTED) v /= 2;
+    return v;
+}
 // Words per block of the batched clear; bytes per thread of the batched
 // header/bitmap/median assembly.
 constexpr uint64_t ZERO_ITEM = 1024;
@@ -85,18 +97,17 @@ struct BatchField {
 
 // Batched kernels (szx_compress.hip), all reading device copies of the
 // field table.  tbase: first global tile of each field (nf + 1 entries) for
-// the chosen tile shape; rbase: first range item of each field (nf + 1).
-void batch_range_launch(const BatchField *bf, const uint64_t *rbase, int nf, uint64_t nitems, double *part,
-                        hipStream_t st);
+// the chosen tile shape; rbase: first range item of each field (nf + 1); zbase
+// / abase: first block of each field in the flattened clear / assembly grids
+// (nf + 1 entries; the last is the grid size).
+// Clears every field's look-back state and, in the same launch, takes the
+// REL fields' ranges (nitems items of `item` values each).
+void batch_prepare_launch(const BatchField *bf, const uint64_t *zbase, uint64_t zitems, const uint64_t *rbase, int nf,
+                          uint64_t nitems, uint64_t item, double *part, hipStream_t st);
 // tmap: the field of every tile of the global tile list (total).
 int batch_compress_launch(int bs, int lv, int ipt, const BatchField *bf, const uint64_t *tbase,
                           const uint32_t *tmap, uint64_t total, hipStream_t st);
-// zbase / abase: first block of each field in the flattened clear / assembly
-// grids (nf + 1 entries; the last is the grid size).
-void batch_zero_launch(const BatchField *bf, const uint64_t *zbase, int nf, uint64_t nitems, hipStream_t st);
 void batch_assemble_launch(const BatchField *bf, const uint64_t *abase, int nf, uint64_t nitems, hipStream_t st);
-
-struct DecodeHeader;
 
 // One field of a batched decode (the stream sits at out + result[0]).
 struct BatchDecodeField {
@@ -106,17 +117,16 @@ struct BatchDecodeField {
     const uint64_t *index;   // record index written by the batched compress
     void *dst;
     int32_t *status;
-    DecodeHeader *h;         // workspace
     uint64_t ntidx;          // index tiles
     int w;
 };
 
-// Batched decode (szx_decompress.hip): header checks, every tile's bytes
-// (into recs, batch_decode_records_bytes(total) bytes), then every index tile
-// of every field.  tbase: first global index tile of each field (nf + 1);
+// Batched decode (szx_decompress.hip): header checks and every tile's bytes
+// (into recs, batch_decode_records_bytes(total) bytes) in one pass, then every
+// index tile of every field.  tbase: first global index tile of each field (nf + 1);
 // tmap: the field of every global index tile (total).
 uint64_t batch_decode_records_bytes(uint64_t total);
 int batch_decode_launch(int bs, const BatchDecodeField *f, const uint64_t *tbase, const uint32_t *tmap,
-                        void *recs, int nf, uint64_t total, int exact, hipStream_t st);
+                        void *recs, uint64_t total, int exact, hipStream_t st);
 
 }  // namespace szxamd

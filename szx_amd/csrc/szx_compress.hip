@@ -1010,11 +1010,11 @@ __device__ inline int field_of(const uint64_t *base, int nf, uint64_t item)
     return lo;
 }
 
-// REL range over the batch: items of RANGE_ITEM values, field by field.
+// REL range over the batch, item by item (range_item_values), field by field.
 template <typename T>
 __device__ inline void range_item(const T *x, uint64_t a, uint64_t b, double *slot)
 {
-    // a is a multiple of RANGE_ITEM and x 16-byte aligned, so every quad of
+    // a is a multiple of the item size and x 16-byte aligned, so every quad of
     // values starts on a 16-byte boundary; RU quads per thread are in flight
     constexpr int RU = 4;
     T mn = pos_inf<T>(), mx = -pos_inf<T>();
@@ -1061,30 +1061,55 @@ __device__ inline void range_item(const T *x, uint64_t a, uint64_t b, double *sl
     }
 }
 
-__global__ __launch_bounds__(256) void k_batch_range(const BatchField *bf, const uint64_t *rbase, int nf,
-                                                     double *part)
+// Clear block zi of the flattened look-back words, totals and error flags.
+__device__ inline void zero_item(const BatchField *bf, const uint64_t *zbase, int nf, uint64_t zi)
 {
-    const uint64_t item = blockIdx.x;
+    const int f = field_of(zbase, nf, zi);
+    const uint64_t a = (zi - zbase[f]) * ZERO_ITEM;
+    const uint64_t b = a + ZERO_ITEM < bf[f].zwords ? a + ZERO_ITEM : bf[f].zwords;
+    unsigned long long *z = bf[f].p.tiles;
+    for (uint64_t i = a + threadIdx.x; i < b; i += blockDim.x) z[i] = 0;
+}
+
+// What a batched compress needs before its tiles: the look-back state cleared
+// (the first zitems workgroups) and the REL items' ranges, in one launch.
+__global__ __launch_bounds__(256) void k_batch_prepare(const BatchField *bf, const uint64_t *zbase, uint64_t zitems,
+                                                       const uint64_t *rbase, int nf, uint64_t item_values,
+                                                       double *part)
+{
+    if (blockIdx.x < zitems) {
+        zero_item(bf, zbase, nf, blockIdx.x);
+        return;
+    }
+    const uint64_t item = blockIdx.x - zitems;
     const int fi = field_of(rbase, nf, item);
     const BatchField &f = bf[fi];
     const uint64_t k = item - rbase[fi];
-    const uint64_t a = k * RANGE_ITEM, b = a + RANGE_ITEM < f.p.n ? a + RANGE_ITEM : f.p.n;
+    const uint64_t a = k * item_values, b = a + item_values < f.p.n ? a + item_values : f.p.n;
     if (f.w == 4) range_item(static_cast<const float *>(f.p.x), a, b, part + 2 * item);
     else range_item(static_cast<const double *>(f.p.x), a, b, part + 2 * item);
 }
 
-// Fold a REL field's items into its bound (the reference's rounding).
-__global__ void k_batch_range_final(BatchField *bf, const uint64_t *rbase, int nf, const double *part)
+// Fold a REL field's items into its bound (the reference's rounding), one wave
+// per field.
+__global__ __launch_bounds__(64) void k_batch_range_final(const BatchField *bf, const uint64_t *rbase,
+                                                          const double *part)
 {
-    const int fi = blockIdx.x * blockDim.x + threadIdx.x;
-    if (fi >= nf) return;
+    const int fi = blockIdx.x, lane = threadIdx.x;
     const BatchField &f = bf[fi];
     if (!f.rel) return;
     double mn = __builtin_inf(), mx = -__builtin_inf();
-    for (uint64_t i = rbase[fi]; i < rbase[fi + 1]; i++) {
+    for (uint64_t i = rbase[fi] + lane; i < rbase[fi + 1]; i += 64) {
         mn = part[2 * i] < mn ? part[2 * i] : mn;
         mx = part[2 * i + 1] > mx ? part[2 * i + 1] : mx;
     }
+    for (int m = 1; m < 64; m <<= 1) {
+        double o = __shfl_xor(mn, m, 64);
+        mn = o < mn ? o : mn;
+        o = __shfl_xor(mx, m, 64);
+        mx = o > mx ? o : mx;
+    }
+    if (lane != 0) return;
     float *eb = const_cast<float *>(f.p.eb_dev);
     if (f.w == 4) {
         const float first = static_cast<const float *>(f.p.x)[0];
@@ -1119,17 +1144,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
     p.ntiles = bf[f].ntiles[IPT == 4 ? 2 : IPT - 1];
     if (bf[f].w == 4) compress_tile<float, BS, LVF, SF, IPT>(p, g - tbase[f], lds.f);
     else compress_tile<double, BS, LVD, SD, IPT>(p, g - tbase[f], lds.d);
-}
-
-// Clear every field's look-back words, totals and error flag (one block per
-// ZERO_ITEM words, flattened over the fields).
-__global__ __launch_bounds__(256) void k_zero_batch(const BatchField *bf, const uint64_t *zbase, int nf)
-{
-    const int f = field_of(zbase, nf, blockIdx.x);
-    const uint64_t a = (blockIdx.x - zbase[f]) * ZERO_ITEM;
-    const uint64_t b = a + ZERO_ITEM < bf[f].zwords ? a + ZERO_ITEM : bf[f].zwords;
-    unsigned long long *z = bf[f].p.tiles;
-    for (uint64_t i = a + threadIdx.x; i < b; i += blockDim.x) z[i] = 0;
 }
 
 // Header, bitmap and medians of every field; abase gives each field's
@@ -1379,12 +1393,13 @@ int compress_launch(const void *d_in, uint64_t n, int w, int rel_mode, float abs
 // batched launchers
 // ---------------------------------------------------------------------------
 
-void batch_range_launch(const BatchField *bf, const uint64_t *rbase, int nf, uint64_t nitems, double *part,
-                        hipStream_t st)
+void batch_prepare_launch(const BatchField *bf, const uint64_t *zbase, uint64_t zitems, const uint64_t *rbase, int nf,
+                          uint64_t nitems, uint64_t item, double *part, hipStream_t st)
 {
-    if (nitems) hipLaunchKernelGGL(k_batch_range, dim3((unsigned)nitems), dim3(256), 0, st, bf, rbase, nf, part);
-    hipLaunchKernelGGL(k_batch_range_final, dim3((nf + 255) / 256), dim3(256), 0, st,
-                       const_cast<BatchField *>(bf), rbase, nf, part);
+    if (zitems + nitems)
+        hipLaunchKernelGGL(k_batch_prepare, dim3((unsigned)(zitems + nitems)), dim3(256), 0, st, bf, zbase, zitems,
+                           rbase, nf, item, part);
+    if (nitems) hipLaunchKernelGGL(k_batch_range_final, dim3((unsigned)nf), dim3(64), 0, st, bf, rbase, part);
 }
 
 // Persistent grid: every workgroup resident at once (the round-robin walk
@@ -1443,11 +1458,6 @@ int batch_compress_launch(int bs, int lv, int ipt, const BatchField *bf, const u
     case 256: return batch_shape<256>(lv, ipt, bf, tbase, tmap, total, st);
     default: return -1;
     }
-}
-
-void batch_zero_launch(const BatchField *bf, const uint64_t *zbase, int nf, uint64_t nitems, hipStream_t st)
-{
-    if (nitems) hipLaunchKernelGGL(k_zero_batch, dim3((unsigned)nitems), dim3(256), 0, st, bf, zbase, nf);
 }
 
 void batch_assemble_launch(const BatchField *bf, const uint64_t *abase, int nf, uint64_t nitems, hipStream_t st)

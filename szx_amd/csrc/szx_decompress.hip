@@ -607,18 +607,12 @@ __global__ __launch_bounds__(256) void k_decode_tiles(DecodeParams p)
 // (or captured) together.
 // ---------------------------------------------------------------------------
 
-__global__ void k_decode_header_batch(const BatchDecodeField *f, int nf, int bs)
-{
-    const int fi = blockIdx.x * blockDim.x + threadIdx.x;
-    if (fi >= nf) return;
-    const BatchDecodeField &d = f[fi];
-    const uint8_t *s = d.out + d.result[0];
-    check_header(s, d.result[1], d.n, bs, d.h, d.status);
-}
-
 // Every tile's bytes (tile_src), one thread per tile, so that a decode
 // workgroup starts staging its records after one load (the field's result
-// words, header and index entries are resolved here, off its path).
+// words, header and index entries are resolved here, off its path).  Every
+// thread checks its field's header itself -- thirteen bytes that its whole
+// field shares in the caches, against a launch of their own -- and the thread
+// of the field's first tile sets the field's status before any tile decodes.
 template <int BS, int LVF, int LVD>
 __global__ __launch_bounds__(256) void k_decode_setup_batch(const BatchDecodeField *f, const uint64_t *tbase,
                                                             const uint32_t *tmap, TileSrc *recs, uint64_t total)
@@ -629,9 +623,14 @@ __global__ __launch_bounds__(256) void k_decode_setup_batch(const BatchDecodeFie
     if (g >= total) return;
     const uint32_t fi = tmap[g];   // the field holding tile g
     const BatchDecodeField &d = f[fi];
-    const DecodeParams p{d.out + d.result[0], d.result[1], d.n, d.h, d.index,
-                         reinterpret_cast<const uint16_t *>(d.index + 2 * (d.ntidx + 1)), d.status, d.dst, 0};
-    const uint64_t t = g - tbase[fi];
+    const uint8_t *s = d.out + d.result[0];
+    const uint64_t len = d.result[1], t = g - tbase[fi];
+    DecodeHeader h;
+    int32_t rc;
+    check_header(s, len, d.n, BS, &h, &rc);
+    if (t == 0) *d.status = rc;
+    const DecodeParams p{s, len, d.n, &h, d.index, reinterpret_cast<const uint16_t *>(d.index + 2 * (d.ntidx + 1)),
+                         d.status, d.dst, 0};
     TileSrc r = d.w == 4 ? tile_src<S32::NBLK, S32::STAGE>(p, t) : tile_src<S64::NBLK, S64::STAGE>(p, t);
     r.field = fi;
     r.tile = (uint32_t)t;
@@ -667,10 +666,9 @@ static void launch_decode_batch(const BatchDecodeField *f, const uint64_t *tbase
 uint64_t batch_decode_records_bytes(uint64_t total) { return total * sizeof(TileSrc); }
 
 int batch_decode_launch(int bs, const BatchDecodeField *f, const uint64_t *tbase, const uint32_t *tmap,
-                        void *recs, int nf, uint64_t total, int exact, hipStream_t st)
+                        void *recs, uint64_t total, int exact, hipStream_t st)
 {
     TileSrc *r = static_cast<TileSrc *>(recs);
-    hipLaunchKernelGGL(k_decode_header_batch, dim3((nf + 255) / 256), dim3(256), 0, st, f, nf, bs);
     switch (bs) {
     case 4: launch_decode_batch<4>(f, tbase, tmap, r, total, exact, st); break;
     case 8: launch_decode_batch<8>(f, tbase, tmap, r, total, exact, st); break;
