@@ -309,17 +309,24 @@ unsigned char *host_compress_nb(const void *data, size_t n, int w, int rel_mode,
     }
     HostCtx &c = g_ctx;
     if (!c.ready()) return nullptr;
-    if (!c.in.reserve(n * (size_t)w) || !c.out.reserve(nb_capacity(n, w)) || !c.ws.reserve(nb_workspace(n)) ||
+    if (!c.in.reserve(n * (size_t)w) || !c.out.reserve(nb_capacity(n, w)) || !c.ws.reserve(nb_workspace(n, w)) ||
         !c.res.reserve(64))
         return nullptr;
     if (!hip_ok(hipMemcpyAsync(c.in.p, data, n * (size_t)w, hipMemcpyHostToDevice, c.stream), "H2D"))
         return nullptr;
-    nb_compress_launch(c.in.p, n, w, rel_mode, abs_eb, rel, (uint8_t *)c.out.p, (uint8_t *)c.ws.p,
-                       (uint64_t *)c.res.p, c.stream);
     uint64_t res[4] = {0, 0, 0, 0};
-    if (!hip_ok(hipMemcpyAsync(res, c.res.p, sizeof res, hipMemcpyDeviceToHost, c.stream), "D2H") ||
-        !hip_ok(hipStreamSynchronize(c.stream), "compress"))
+    for (int attempt = 0; attempt < 2; attempt++) {
+        nb_compress_launch(c.in.p, n, w, rel_mode, abs_eb, rel, (uint8_t *)c.out.p, (uint8_t *)c.ws.p,
+                           (uint64_t *)c.res.p, c.stream);
+        if (!hip_ok(hipMemcpyAsync(res, c.res.p, sizeof res, hipMemcpyDeviceToHost, c.stream), "D2H") ||
+            !hip_ok(hipStreamSynchronize(c.stream), "compress"))
+            return nullptr;
+        if (!res[3]) break;
+    }
+    if (res[3]) {
+        set_err("compress: a look-back wait overran its bound twice (device busy?)");
         return nullptr;
+    }
     unsigned char *out = (unsigned char *)malloc(res[1] ? res[1] : 1);
     if (!out) {
         set_err("malloc failed");
@@ -341,7 +348,7 @@ void *host_decompress_nb(const unsigned char *bytes, size_t len, size_t n, int w
     }
     HostCtx &c = g_ctx;
     if (!c.ready()) return nullptr;
-    if (!c.in.reserve(len ? len : 1) || !c.out.reserve(n * (size_t)w) || !c.ws.reserve(nb_workspace(n)) ||
+    if (!c.in.reserve(len ? len : 1) || !c.out.reserve(n * (size_t)w) || !c.ws.reserve(nb_workspace(n, w)) ||
         !c.res.reserve(64))
         return nullptr;
     if (!hip_ok(hipMemcpyAsync(c.in.p, bytes, len, hipMemcpyHostToDevice, c.stream), "H2D"))
@@ -858,7 +865,7 @@ size_t szx_amd_nb_capacity(size_t n, int dataType)
 size_t szx_amd_nb_workspace(size_t n, int dataType)
 {
     const int w = width_of(dataType);
-    return w && n ? nb_workspace(n) : 0;
+    return w && n ? nb_workspace(n, w) : 0;
 }
 
 int szx_amd_compress_nb_dev(const void *d_in, size_t n, int dataType, int errBoundMode, float absErrBound,
@@ -870,7 +877,7 @@ int szx_amd_compress_nb_dev(const void *d_in, size_t n, int dataType, int errBou
     if (!w) { set_err("unsupported dataType %d", dataType); return SZx_TERR; }
     if (errBoundMode != ABS && errBoundMode != REL) { set_err("bad errBoundMode"); return SZx_BERR; }
     if (!d_in || !d_out || !d_work || !d_result || n == 0) { set_err("NULL argument or n == 0"); return SZx_NSCS; }
-    if (outCapacity < nb_capacity(n, w) || workBytes < nb_workspace(n)) {
+    if (outCapacity < nb_capacity(n, w) || workBytes < nb_workspace(n, w)) {
         set_err("output buffer or workspace too small");
         return SZx_NSCS;
     }
@@ -886,7 +893,7 @@ int szx_amd_decompress_nb_dev(const void *d_stream, size_t streamBytes, size_t n
     const int w = width_of(dataType);
     if (!w) { set_err("unsupported dataType %d", dataType); return SZx_TERR; }
     if (!d_stream || !d_out || !d_work || !d_status || n == 0) { set_err("NULL argument or n == 0"); return SZx_NSCS; }
-    if (workBytes < nb_workspace(n)) { set_err("workspace too small"); return SZx_NSCS; }
+    if (workBytes < nb_workspace(n, w)) { set_err("workspace too small"); return SZx_NSCS; }
     nb_decompress_launch((const uint8_t *)d_stream, streamBytes, n, w, d_out, (uint8_t *)d_work,
                          flags & SZX_AMD_DECODE_EXACT, d_status, (hipStream_t)hipStream);
     return hip_ok(hipGetLastError(), "launch") ? SZx_SCES : SZx_NSCS;
@@ -1335,7 +1342,7 @@ void *SZx_fast_decompress_pred(int dataType, float *preData, unsigned char *curB
     }
     HostCtx &c = g_ctx;
     if (!c.ready()) return nullptr;
-    if (!c.in.reserve(byteLength ? byteLength : 1) || !c.out.reserve(n * 4) || !c.ws.reserve(nb_workspace(n)) ||
+    if (!c.in.reserve(byteLength ? byteLength : 1) || !c.out.reserve(n * 4) || !c.ws.reserve(nb_workspace(n, 4)) ||
         !c.res.reserve(64) || !c.fx.reserve(n * 4))
         return nullptr;
     if (!hip_ok(hipMemcpyAsync(c.in.p, curBytes, byteLength, hipMemcpyHostToDevice, c.stream), "H2D") ||

@@ -93,6 +93,11 @@ void range_launch(const void *d_in, uint64_t n, int w, uint8_t *d_ws, void *d_mi
 void range_bound_launch(const void *d_in, uint64_t n, int w, float rel, uint8_t *d_ws, float *eb_out,
                         void *d_minmax, hipStream_t st);
 
+// The pass alone, left as RANGE_LB_PARTS {min, max} pairs of the array's type
+// in parts for the next kernel to fold (RangeFold); clears nzero words of zero.
+void range_partials_launch(const void *d_in, uint64_t n, int w, void *parts, unsigned long long *zero, uint64_t nzero,
+                           hipStream_t st);
+
 // Non-blocked codec (fastMode 1, szx_nonblocked.hip): one record over all
 // values against the global median.
 // Reader of the reference's CUDA codec (cuSZx) stream, fp32 (szx_cuszx.hip).
@@ -108,7 +113,7 @@ void cuszx_compress_launch(const float *d_in, uint64_t n, float eb, int bs, uint
                            uint64_t *d_result, hipStream_t st);
 
 uint64_t nb_capacity(uint64_t n, int w);
-uint64_t nb_workspace(uint64_t n);
+uint64_t nb_workspace(uint64_t n, int w);
 void nb_compress_launch(const void *d_in, uint64_t n, int w, int rel_mode, float abs_eb, float rel, uint8_t *d_out,
                         uint8_t *d_ws, uint64_t *d_result, hipStream_t st);
 void nb_decompress_launch(const uint8_t *d_stream, uint64_t len, uint64_t n, int w, void *d_out, uint8_t *d_ws,

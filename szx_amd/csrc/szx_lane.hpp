@@ -1,0 +1,184 @@
+// szx_lane.hpp -- what one lane does with its consecutive values, shared by
+// the blocked and the non-blocked codec: lead codes to mid-byte positions and
+// words (decoding), and runs of mid bytes into an LDS stage (encoding).
+#pragma once
+
+#include <type_traits>
+
+#include "szx_common.hpp"
+#include "szx_wave.hpp"
+
+namespace szxamd {
+
+// A lane's lead codes, four values to a word: bytes b of words j belong to
+// value 4 b + j, so two operations per word replace two per value, and byte
+// sums of the words give every value's first mid byte.
+template <int LV> struct LaneCodes {
+    static constexpr int NLB = LV / 4;   // lead-code bytes per lane
+    uint32_t z8[4];   // 8 x lead bytes
+    uint32_t m[4];    // mid bytes
+    uint32_t pk[4];   // mid bytes of the lane's earlier values
+    uint32_t tot;     // mid bytes of the lane
+
+    // code: the lane's lead-code bytes (first value in the top bits of byte
+    // 0), zero past them; rb: bytes per value; nv: the lane's values (LV
+    // unless the array ends inside the lane)
+    __device__ void set(uint32_t code, int rb, int nv)
+    {
+        static_assert(NLB >= 1 && NLB <= 4, "a lane's lead codes fit a word");
+        // codes above rb count as rb (only records of one or two bytes per
+        // value have any): 3 -> 2, then 2 -> 1, two bits at a time
+        code -= code & (code >> 1) & (rb <= 2 ? 0x55555555u : 0u);
+        code -= (code >> 1) & (rb <= 1 ? 0x55555555u : 0u);
+        const uint32_t rbx = (uint32_t)rb * 0x01010101u;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const uint32_t z = (code >> (6 - 2 * j)) & 0x03030303u;
+            z8[j] = z << 3;
+            m[j] = rbx - z;
+            if (nv < LV) {
+                uint32_t keep = 0;
+#pragma unroll
+                for (int b = 0; b < NLB; b++)
+                    if (4 * b + j < nv) keep |= 0xFFu << (8 * b);
+                m[j] &= keep;
+            }
+        }
+        uint32_t bt = (m[0] + m[1]) + (m[2] + m[3]);   // per lead byte: mid bytes of its values
+        if constexpr (NLB >= 2) bt += bt << 8;
+        if constexpr (NLB >= 3) bt += bt << 16;
+        tot = (bt >> (8 * (NLB - 1))) & 0xFFu;
+        pk[0] = NLB >= 2 ? bt << 8 : 0u;
+#pragma unroll
+        for (int j = 1; j < 4; j++) pk[j] = pk[j - 1] + m[j - 1];
+    }
+};
+
+// A lane's words from its mid bytes alone, in two passes around a scan.
+//
+// A value's m bytes (from stage byte p on) land on word bytes [W - rb, W - z):
+// the gathered word shifted up by W - rb bytes supplies bytes [0, W - z)
+// (zeros below), the value before it the top z <= 3 bytes -- one bit-field
+// insert in the word's top 32 bits.  Bits the final shift drops are never
+// masked.  gather() runs with a zero carry-in: hi[k] is the top of value k's
+// word if nothing came from the previous lane, inh[k] marks the bytes it still
+// inherits from before the lane.  top / wrote are what the lane passes on:
+// its last top bytes and which of them it wrote itself.
+template <typename T, int LV> struct LaneWords {
+    using U = typename Word<T>::U;
+    static constexpr int W = Word<T>::W;
+    static_assert(LV * W < 256, "a lane's mid bytes fit a byte");
+    uint32_t hi[LV], inh[LV];
+    uint32_t lw[W == 8 ? LV : 1];
+    uint32_t top, wrote;
+
+    // stb: 4-byte aligned stage; p0: the lane's first mid byte in it (up to 11
+    // bytes past the lane's last are read); byte7: fp64 with the reference
+    // decoder's byte-7 read for records of five bytes (szxd_double.cc:244)
+    template <bool BYTE7>
+    __device__ void gather_as(const uint8_t *stb, uint32_t p0, const LaneCodes<LV> &c, int rb)
+    {
+        const int lo8 = 8 * (W - rb);
+        uint32_t tp = 0, ih = ~0u;
+#pragma unroll
+        for (int k = 0; k < LV; k++) {
+            const int j = k & 3, b = 8 * (k >> 2);
+            const uint32_t p = p0 + ((c.pk[j] >> b) & 0xFFu);
+            const uint32_t z = (c.z8[j] >> b) & 0xFFu;
+            // two or three aligned words and a byte funnel (unaligned LDS
+            // reads are slow)
+            const uint32_t *w = reinterpret_cast<const uint32_t *>(stb + (p & ~3u));
+            uint32_t xh;
+            if constexpr (W == 4) {
+                xh = __builtin_amdgcn_alignbyte(w[1], w[0], p) << lo8;
+            } else {
+                const uint32_t d0 = w[0], d1 = w[1], d2 = w[2];
+                const uint32_t x0 = __builtin_amdgcn_alignbyte(d1, d0, p);
+                const U xs = ((U)x0 | ((U)__builtin_amdgcn_alignbyte(d2, d1, p) << 32)) << lo8;
+                xh = (uint32_t)(xs >> 32);
+                lw[k] = (uint32_t)xs;
+                if constexpr (BYTE7) {
+                    if (rb == 5 && z == 0 && ((c.m[j] >> b) & 0xFFu)) xh = (xh & 0xFFFFFFu) | (x0 & 0xFF000000u);
+                }
+            }
+            const uint32_t take = ~0u >> z;   // bytes below W - z
+            tp = (xh & take) | (tp & ~take);
+            ih &= ~take;
+            hi[k] = tp;
+            inh[k] = ih;
+        }
+        top = tp;
+        wrote = ~ih;
+    }
+    __device__ void gather(const uint8_t *stb, uint32_t p0, const LaneCodes<LV> &c, int rb, int exact)
+    {
+        if (W == 8 && !exact && __builtin_amdgcn_ballot_w64(rb == 5) != 0) gather_as<true>(stb, p0, c, rb);
+        else gather_as<false>(stb, p0, c, rb);
+    }
+    // cin: the top bytes the lane inherits
+    __device__ T value(int k, uint32_t cin, int shift, T med) const
+    {
+        const uint32_t h = hi[k] | (cin & inh[k]);
+        if constexpr (W == 4) return from_bits<T>(h << shift) + med;
+        else return from_bits<T>((((U)h << 32) | lw[k]) << shift) + med;
+    }
+};
+
+// OR a run of nbits <= 64 bits (a multiple of 8, zero above) into a zeroed LDS
+// stage of 8-byte words from bit o8 on: the one or two words it touches.  LDS
+// atomics are the expensive part, so lanes with nothing to add sit out
+// (measured on 512^3 fp32: two unconditional ORs per value ran 0.28 ms against
+// 0.22 ms for predicated ones).  OR is idempotent and every stage byte has one
+// writer, so words shared with neighbouring lanes need no care.
+__device__ inline void stage_run(uint64_t *sq, uint32_t o8, uint64_t run, uint32_t nbits)
+{
+    if (!nbits) return;
+    const uint32_t s = o8 & 63u;
+    uint64_t *pq = sq + (o8 >> 6);
+    __hip_atomic_fetch_or(pq, run << s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    // bits past the first word (only when s > 0): the run's top s
+    if (s + nbits > 64u)
+        __hip_atomic_fetch_or(pq + 1, run >> (64u - s), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// One wave copies nbytes of its LDS stage (from byte 0 of sw, 4-byte aligned)
+// to dst: 16-byte stores inside, bytes at the edges, whose other bytes belong
+// to the neighbours.  Non-temporal: the stream is not read again by the
+// launch, which leaves the caches to its input.
+__device__ inline void wave_copy_out(uint8_t *dst, const uint32_t *sw, uint32_t nbytes, int lane)
+{
+    typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
+    const uint8_t *sb = reinterpret_cast<const uint8_t *>(sw);
+    const uint32_t head = (uint32_t)((16 - ((uintptr_t)dst & 15)) & 15);
+    const uint32_t h = head < nbytes ? head : nbytes;
+    if (lane < (int)h) dst[lane] = sb[lane];
+    const uint32_t nchunk = (nbytes - h) >> 4;
+    const int r = h & 3;
+    for (uint32_t c = lane; c < nchunk; c += 64) {
+        const uint32_t o = h + 16 * c;
+        const uint32_t *w = sw + (o >> 2);
+        const uint32_t a0 = w[0], a1 = w[1], a2 = w[2], a3 = w[3], a4 = w[4];
+        const u32x4_t v = {__builtin_amdgcn_alignbyte(a1, a0, r), __builtin_amdgcn_alignbyte(a2, a1, r),
+                           __builtin_amdgcn_alignbyte(a3, a2, r), __builtin_amdgcn_alignbyte(a4, a3, r)};
+        __builtin_nontemporal_store(v, reinterpret_cast<u32x4_t *>(dst + o));
+    }
+    const uint32_t tail0 = h + 16 * nchunk;
+    if (lane < (int)(nbytes - tail0)) dst[tail0 + lane] = sb[tail0 + lane];
+}
+
+// Zero the first nbytes (rounded up to 16) of a wave's LDS stage.
+__device__ inline void wave_clear(uint32_t *sw, uint32_t nbytes, int lane)
+{
+    for (uint32_t i = lane; i < (nbytes + 15) / 16; i += 64) reinterpret_cast<uint4 *>(sw)[i] = make_uint4(0, 0, 0, 0);
+}
+
+// Orders a wave's own LDS accesses of different lanes (no other wave touches
+// the data).
+__device__ inline void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+}  // namespace szxamd

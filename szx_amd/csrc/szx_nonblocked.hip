@@ -9,120 +9,70 @@
 // median is formed); reqLength, the shift, the lead codes and the mid bytes
 // follow the blocked codec's rules with the whole array as one block.
 //
-// Every value's lead code depends only on its predecessor, so the stream is
-// built in tiles of 4096 values (16 consecutive values per lane):
-//   compress:   k_nb_setup (median, reqLength), k_nb_pass<T, false> (lead
-//               codes straight into the stream, mid-byte count per tile), a
-//               scan over the tiles, k_nb_pass<T, true> (mid bytes at their
-//               offsets), k_nb_finish (header, sizes)
-//   decompress: k_nb_header, k_nb_dcount (mid-byte count per tile from the
-//               lead codes), a scan, k_nb_carry (per tile: the last bytes it
-//               writes at the three positions a later value can inherit),
-//               k_nb_carry_scan (the bytes every tile inherits, last writer
-//               wins), k_nb_decode.  The decoder stages each tile's mid bytes
-//               (contiguous in the stream) in LDS with aligned word loads.
+// Every value's lead code depends only on its predecessor, and its place in
+// the stream on the mid bytes before it.
+//
+//   compress:   the range pass, then k_nb_encode in one pass over the input:
+//               a wave takes a run of consecutive values, writes their lead
+//               codes to their fixed place and collects their mid bytes in
+//               its own part of LDS; the workgroup's total goes through the
+//               compressor's decoupled look-back, and the waves copy their
+//               mid bytes out.  k_nb_finish writes the header and results.
+//   decompress: k_nb_count (header check; per tile, from the lead codes
+//               alone, its mid bytes and where the bytes lie that a later
+//               tile could inherit), k_nb_scan (every tile's mid-byte offset
+//               and the stream positions of the bytes it inherits, last
+//               writer wins), k_nb_decode.
 // A value inherits its first min(lead, rb) bytes from the previous value
-// (szxd_float.cc:78-199), possibly across many tiles; the carry scan resolves
-// that chain with the same last-writer operator the blocked decoders use.
+// (szxd_float.cc:78-199), possibly across many tiles; only three byte
+// positions can be inherited, so a tile passes on three stream positions.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include "szx_common.hpp"
 #include "szx_internal.hpp"
+#include "szx_lane.hpp"
+#include "szx_range.hpp"
+#include "szx_wave.hpp"
 
 namespace szxamd {
 
-constexpr int NB_PER = 16;                 // values per lane
-constexpr int NB_TILE = 256 * NB_PER;      // values per tile
 constexpr uint64_t NB_HDR = 17;            // header bytes before the lead codes
 
-// Codec parameters decided on the device (k_nb_setup / k_nb_header).
+// Values per lane, and per wave step of 64 lanes (4 KiB / 8 KiB of input):
+// 16 fp32 values have one word of lead codes.
+template <typename T> constexpr int NB_LV = sizeof(T) == 4 ? 16 : 8;
+// A wave's run in the encoder: NB_STEPS steps, 16 KiB of input; the workgroup
+// of four waves owns a look-back tile of 64 KiB.
+constexpr int NB_STEPS = 4;
+template <typename T> constexpr int NB_RUN = 64 * NB_LV<T> * NB_STEPS;
+template <typename T> constexpr int NB_TILE = 4 * NB_RUN<T>;
+// Mid bytes a wave collects in LDS before its place is known: above (under
+// 1.6x compression) it drops them and encodes its run again afterwards, step
+// by step.  Four workgroups fit a CU's LDS.
+constexpr uint32_t NB_CAP = 10240 - 128;
+constexpr int NB_STAGE_DW = 10240 / 4;
+// A decoder tile: one step of four waves.
+template <typename T> constexpr int NB_DTILE = 256 * NB_LV<T>;
+
+// Codec parameters decided on the device (k_nb_encode / k_nb_count).
 struct NbParams {
     int32_t len, rb, shift, ok;
     uint32_t hdr_bits;     // stored median (f32 bits)
     float eb;
-    double msub;           // median subtracted before the shift (fp32: the stored one)
     float med;             // decoder: the stored median
+    int32_t err;           // encoder: a look-back wait overran its bound
     uint64_t total;        // mid bytes
+    double msub;           // median subtracted before the shift (fp32: the stored one)
 };
-
-template <typename U> __device__ inline int nb_lead(U xr)
-{
-    constexpr int W = sizeof(U);
-    if ((xr >> (8 * (W - 3))) == 0) return 3;
-    if ((xr >> (8 * (W - 2))) == 0) return 2;
-    if ((xr >> (8 * (W - 1))) == 0) return 1;
-    return 0;
-}
-
-// Exclusive sum over the 256 lanes of a workgroup; *total receives the sum.
-__device__ inline uint32_t nb_block_excl(uint32_t v, uint32_t *total)
-{
-    __shared__ uint32_t s_w[4];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    uint32_t inc = v;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t o = __shfl_up(inc, d, 64);
-        if (lane >= d) inc += o;
-    }
-    if (lane == 63) s_w[wv] = inc;
-    __syncthreads();
-    uint32_t pre = 0, tot = 0;
-    for (int k = 0; k < 4; k++) {
-        if (k < wv) pre += s_w[k];
-        tot += s_w[k];
-    }
-    __syncthreads();
-    *total = tot;
-    return pre + inc - v;
-}
-
-// Last-writer record of the three inheritable byte positions W-1, W-2, W-3:
-// bytes 0..2 hold them, bits 24..26 say which were written; b's written bytes
-// win over a's.
-__device__ inline uint32_t nb_combine(uint32_t a, uint32_t b)
-{
-    const uint32_t f = b >> 24;
-    const uint32_t keep = ((f & 1u) ? 0xFFu : 0u) | ((f & 2u) ? 0xFF00u : 0u) | ((f & 4u) ? 0xFF0000u : 0u);
-    return ((b & keep) | (a & ~keep & 0xFFFFFFu)) | ((a | b) & 0x7000000u);
-}
-
-// Exclusive last-writer scan over the 256 lanes (lane 0 gets 0).
-__device__ inline uint32_t nb_block_excl_lw(uint32_t v, uint32_t *total)
-{
-    __shared__ uint32_t s_w[4];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    uint32_t inc = v;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t o = __shfl_up(inc, d, 64);
-        if (lane >= d) inc = nb_combine(o, inc);
-    }
-    uint32_t ex = __shfl_up(inc, 1, 64);
-    if (lane == 0) ex = 0;
-    if (lane == 63) s_w[wv] = inc;
-    __syncthreads();
-    uint32_t pre = 0, tot = 0;
-    for (int k = 0; k < 4; k++) {
-        if (k < wv) pre = nb_combine(pre, s_w[k]);
-        tot = nb_combine(tot, s_w[k]);
-    }
-    __syncthreads();
-    *total = tot;
-    return nb_combine(pre, ex);
-}
 
 // ---- compression ----
 
 // Median, radius and reqLength from the range (szx_float.cc:494-495,
 // szx_double.cc:1153-1154; computeReqLength_*, szx_float.cc:1708-1717).
-template <typename T>
-__global__ void k_nb_setup(const T *mm, const float *eb_dev, float eb_abs, NbParams *P)
+template <typename T> __device__ inline NbParams nb_params(T lo, T hi, float eb)
 {
-    if (threadIdx.x != 0) return;
-    const float eb = eb_dev ? *eb_dev : eb_abs;
-    const T lo = mm[0], hi = mm[1];
+    NbParams P{};
     float rad_f, med_f;
     if (sizeof(T) == 4) {
         const T rad = (hi - lo) / (T)2;
@@ -133,91 +83,239 @@ __global__ void k_nb_setup(const T *mm, const float *eb_dev, float eb_abs, NbPar
         med_f = (float)(lo + (T)rad_f);
     }
     int clamped;
-    const int len = req_length<T>(rad_expo(rad_f), req_expo(eb), clamped);
+    P.len = req_length<T>(rad_expo(rad_f), req_expo(eb), clamped);
     const float hdr = clamped ? 0.0f : med_f;
-    P->len = len;
-    P->rb = (len + 7) >> 3;
-    P->shift = (-len) & 7;
-    P->ok = 1;
-    P->hdr_bits = f32_bits(hdr);
-    P->eb = eb;
-    P->msub = sizeof(T) == 4 ? (double)hdr : (double)med_f;   // szx_float.cc:1516 / szx_double.cc:1597
+    P.rb = (P.len + 7) >> 3;
+    P.shift = (-P.len) & 7;
+    P.ok = 1;
+    P.hdr_bits = f32_bits(hdr);
+    P.eb = eb;
+    P.msub = sizeof(T) == 4 ? (double)hdr : (double)med_f;   // szx_float.cc:1516 / szx_double.cc:1597
+    return P;
 }
 
-template <typename T>
-__device__ inline typename Word<T>::U nb_word(T v, const NbParams &P)
+template <typename T> struct NbEncode {
+    const T *x;
+    uint64_t n;
+    const T *parts;        // the range pass's {min, max} pairs
+    int rel_mode;
+    float abs_eb, rel;
+    uint8_t *out;
+    NbParams *P;
+    unsigned long long *tiles;
+    ChunkState *chunks;
+    unsigned long long *cacc;
+    uint64_t ntiles;
+};
+
+// One step of a wave's run: the lane's NB_LV values at e0.  Returns the lane's
+// mid bytes and their bits as runs (fp32: two values a run) in run[] / bits[];
+// code = its lead-code bytes; last = its last value's word.
+template <typename T> struct NbStep {
+    using U = typename Word<T>::U;
+    static constexpr int LV = NB_LV<T>;
+    static constexpr int NR = 8;           // runs of at most 64 bits
+    uint64_t run[NR];
+    uint32_t bits[NR];
+    uint32_t tot, code;
+    U last;
+
+    __device__ void encode(const T (&v)[LV], int nv, U before, T msub, int rb, int shift, int lane)
+    {
+        constexpr int W = Word<T>::W;
+        U w[LV];
+#pragma unroll
+        for (int k = 0; k < LV; k++) w[k] = to_bits<T>(v[k] - msub) >> shift;
+        U prev = seg_prev<64>(w[LV - 1], lane);
+        if (lane == 0) prev = before;
+        last = w[LV - 1];
+        const uint32_t rb8 = 8u * (uint32_t)rb;
+        const int lo8 = 8 * W - (int)rb8;
+        uint32_t c8[2] = {0, 0}, t8 = 0;
+#pragma unroll
+        for (int k = 0; k < LV; k++) {
+            const U xr = w[k] ^ prev;
+            const uint32_t top = W == 4 ? (uint32_t)xr : (uint32_t)((uint64_t)xr >> 32);
+            const int lz = __builtin_clzg(top, 32);
+            uint32_t ld8 = (uint32_t)((lz < 24 ? lz : 24) & ~7);
+            uint32_t m8 = __builtin_elementwise_sub_sat(rb8, ld8);
+            if (k >= nv) {
+                ld8 = 0;
+                m8 = 0;
+            }
+            c8[k >> 3] |= ld8 << (8 * ((k & 7) >> 2) + 6 - 2 * (k & 3));
+            if constexpr (W == 4) {
+                // the value's m8 low bits from bit lo8 on
+                const uint32_t mid = m8 < 32 ? __builtin_amdgcn_ubfe((uint32_t)w[k], (uint32_t)lo8, m8) : (uint32_t)w[k];
+                if ((k & 1) == 0) {
+                    run[k / 2] = mid;
+                    bits[k / 2] = m8;
+                } else {
+                    run[k / 2] |= (uint64_t)mid << bits[k / 2];
+                    bits[k / 2] += m8;
+                }
+            } else {
+                const uint64_t mid = (uint64_t)w[k] >> lo8;
+                run[k] = m8 >= 64 ? mid : mid & ((1ull << m8) - 1ull);
+                bits[k] = m8;
+            }
+            t8 += m8;
+            prev = w[k];
+        }
+        tot = t8 >> 3;
+        code = (c8[0] >> 3) | ((c8[1] >> 3) << 16);
+    }
+    __device__ void stage(uint64_t *sq, uint32_t byte) const
+    {
+        uint32_t o8 = 8u * byte;
+#pragma unroll
+        for (int r = 0; r < NR; r++) {
+            stage_run(sq, o8, run[r], bits[r]);
+            o8 += bits[r];
+        }
+    }
+};
+
+// The wave's last lane's word.
+__device__ inline uint32_t last_lane(uint32_t v) { return (uint32_t)__builtin_amdgcn_readlane((int)v, 63); }
+__device__ inline uint64_t last_lane(uint64_t v)
 {
-    return to_bits<T>(v - (T)P.msub) >> P.shift;
+    return (uint64_t)last_lane((uint32_t)v) | ((uint64_t)last_lane((uint32_t)(v >> 32)) << 32);
 }
 
-// Lead codes of the lane's 16 values and their mid-byte counts.  WRITE =
-// false stores the lead-code bytes (4 per lane, at their fixed place) and the
-// tile's mid-byte count; WRITE = true stores the mid bytes at their offsets.
-template <typename T, bool WRITE>
-__global__ __launch_bounds__(256) void k_nb_pass(const T *x, uint64_t n, const NbParams *Pp, uint8_t *out,
-                                                 uint32_t *tsum, const uint64_t *toff)
+// The lane's values at e0 (zeros past the end).  x needs no more than its
+// type's alignment.
+template <typename T, int LV>
+__device__ inline void nb_load(const T *x, uint64_t e0, uint64_t n, T (&v)[LV])
+{
+    typedef unsigned int u32x4_t __attribute__((ext_vector_type(4), aligned(4)));
+    constexpr int VC = 16 / (int)sizeof(T);
+    if (e0 + LV <= n) {
+#pragma unroll
+        for (int k = 0; k < LV; k += VC) {
+            const u32x4_t q = *reinterpret_cast<const u32x4_t *>(x + e0 + k);
+            __builtin_memcpy(&v[k], &q, 16);
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < LV; k++) v[k] = e0 + k < n ? x[e0 + k] : (T)0;
+    }
+}
+
+// One look-back tile per workgroup, a run of NB_RUN consecutive values per
+// wave.  Every lane issues its next values' loads before it encodes the present
+// ones, and nothing is shared between waves until their totals are known; LDS
+// (four workgroups per CU) and vector work per value bound it.  256^3 fp32, REL
+// 1e-3: a sizes pass of 43 us, a scan of 6 and a bytes pass of 90 with a byte
+// store per mid byte -> 32 us (0.6 of the copy kernel's rate on such a size).
+template <typename T>
+__global__ __launch_bounds__(256) void k_nb_encode(NbEncode<T> p)
 {
     using U = typename Word<T>::U;
-    constexpr int W = Word<T>::W;
-    const NbParams P = *Pp;
-    const uint64_t e0 = blockIdx.x * (uint64_t)NB_TILE + threadIdx.x * (uint64_t)NB_PER;
-    U s[NB_PER];
-    int ld[NB_PER];
-    uint32_t cnt = 0;
-    U prev = e0 > 0 && e0 <= n ? nb_word<T>(x[e0 - 1], P) : (U)0;
-#pragma unroll
-    for (int k = 0; k < NB_PER; k++) {
-        const bool valid = e0 + k < n;
-        s[k] = valid ? nb_word<T>(x[e0 + k], P) : (U)0;
-        ld[k] = valid ? nb_lead<U>(s[k] ^ prev) : 0;
-        if (valid && ld[k] < P.rb) cnt += P.rb - ld[k];
-        prev = s[k];
-    }
-    uint32_t total;
-    const uint32_t ex = nb_block_excl(cnt, &total);
-    if (!WRITE) {
-        // lead codes, MSB-first four to a byte (szx_TypeManager.cc:198-273)
-        const uint64_t nlead = (n + 3) / 4;
-#pragma unroll
-        for (int j = 0; j < NB_PER / 4; j++) {
-            const uint64_t lb = e0 / 4 + j;
-            if (lb < nlead)
-                out[NB_HDR + lb] = (uint8_t)((ld[4 * j] << 6) | (ld[4 * j + 1] << 4) | (ld[4 * j + 2] << 2) |
-                                             ld[4 * j + 3]);
-        }
-        if (threadIdx.x == 0) tsum[blockIdx.x] = total;
-        return;
-    }
-    uint8_t *q = out + NB_HDR + (n + 3) / 4 + toff[blockIdx.x] + ex;
-#pragma unroll
-    for (int k = 0; k < NB_PER; k++)
-        if (e0 + k < n)
-            for (int t = W - P.rb; t < W - ld[k]; t++) *q++ = (uint8_t)(s[k] >> (8 * t));
-}
+    constexpr int LV = NB_LV<T>;
+    __shared__ __attribute__((aligned(16))) uint32_t stage[4][NB_STAGE_DW];
+    __shared__ uint32_t s_tot[4];
+    __shared__ unsigned long long s_ex;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const uint64_t tile = blockIdx.x;
+    const uint64_t r0 = tile * (uint64_t)NB_TILE<T> + (uint64_t)wv * NB_RUN<T>;   // the wave's run
+    const uint64_t n = p.n, nlead = (n + 3) / 4;
+    uint32_t *sw = stage[wv];
 
-// One workgroup: exclusive scan of the tile sums (toff), total in P->total.
-__global__ __launch_bounds__(1024) void k_nb_scan(const uint32_t *tsum, uint64_t ntiles, uint64_t *toff,
-                                                  NbParams *P)
-{
-    __shared__ uint64_t s[1024];
-    const uint64_t per = (ntiles + 1023) / 1024;
-    const uint64_t a = threadIdx.x * per, b = a + per < ntiles ? a + per : ntiles;
-    uint64_t sum = 0;
-    for (uint64_t i = a; i < b; i++) sum += tsum[i];
-    s[threadIdx.x] = sum;
+    RangeFold<T> rf;
+    rf.load(p.parts, p.x);
+    T v[LV];
+    nb_load<T, LV>(p.x, r0 + (uint64_t)lane * LV, n, v);
+    const T xb = r0 > 0 && r0 <= n ? p.x[r0 - 1] : (T)0;
+    T lo, hi;
+    rf.minmax(lo, hi);
+    const NbParams P = nb_params<T>(lo, hi, p.rel_mode ? RangeFold<T>::bound(lo, hi, p.rel) : p.abs_eb);
+    if (tile == 0 && threadIdx.x == 0) {   // for k_nb_finish; total and err are the last tile's and any tile's
+        p.P->len = P.len;
+        p.P->hdr_bits = P.hdr_bits;
+        p.P->eb = P.eb;
+    }
+    const T msub = (T)P.msub;
+    wave_clear(sw, NB_CAP + 64, lane);
+    wave_lds_fence();
+
+    U before = r0 > 0 ? (U)(to_bits<T>(xb - msub) >> P.shift) : (U)0;
+    uint32_t sum = 0;
+    bool fits = true;
+    NbStep<T> st;
+#pragma unroll 1
+    for (int s = 0; s < NB_STEPS; s++) {
+        const uint64_t e0 = r0 + (uint64_t)s * (64 * LV) + (uint64_t)lane * LV;
+        T nx[LV];   // the next step's values load while this one is encoded
+        if (s + 1 < NB_STEPS) nb_load<T, LV>(p.x, e0 + 64 * LV, n, nx);
+        const int nv = e0 >= n ? 0 : n - e0 < (uint64_t)LV ? (int)(n - e0) : LV;
+        st.encode(v, nv, before, msub, P.rb, P.shift, lane);
+        // lead codes, MSB-first four to a byte (szx_TypeManager.cc:198-273),
+        // at an odd address
+        const uint64_t lb = e0 / 4;
+        uint8_t *q = p.out + NB_HDR + lb;
+        if (nv == LV) {
+            if constexpr (LV == 16) __builtin_memcpy(q, &st.code, 4);
+            else __builtin_memcpy(q, &st.code, 2);
+        } else {
+            for (int b = 0; 4 * b < nv; b++) q[b] = (uint8_t)(st.code >> (8 * b));
+        }
+        const uint32_t inc = seg_scan_incl<64>(st.tot, lane);
+        const uint32_t stot = __builtin_amdgcn_readlane(inc, 63);
+        fits = fits && sum + stot <= NB_CAP;
+        if (fits) st.stage(reinterpret_cast<uint64_t *>(sw), sum + inc - st.tot);
+        sum += stot;
+        before = last_lane(st.last);
+#pragma unroll
+        for (int k = 0; k < LV; k++) v[k] = nx[k];
+    }
+    if (lane == 0) s_tot[wv] = sum;
     __syncthreads();
-    for (int d = 1; d < 1024; d <<= 1) {
-        const uint64_t v = threadIdx.x >= (unsigned)d ? s[threadIdx.x - d] : 0;
-        __syncthreads();
-        s[threadIdx.x] += v;
-        __syncthreads();
+    const LookbackRefs L{p.tiles, p.chunks, p.cacc, p.ntiles};
+    const uint32_t total = s_tot[0] + s_tot[1] + s_tot[2] + s_tot[3];
+    unsigned long long pend = 0;
+    if (wv == 0) {
+        if (lane == 0) pend = lookback_publish(L, tile, total, 0);
+        unsigned long long ex = 0, none = 0;
+        const LookbackPoll q = lookback_poll(L, tile);
+        if (!lookback_finish(L, tile, q, true, ex, none)) {
+            ex = 0;   // every write stays in bounds; the call reports failure
+            if (lane == 0) atomicExch(&p.P->err, 1);
+        }
+        if (lane == 0) {
+            s_ex = ex;
+            if (tile == p.ntiles - 1) p.P->total = ex + total;
+        }
     }
-    uint64_t run = s[threadIdx.x] - sum;
-    for (uint64_t i = a; i < b; i++) {
-        toff[i] = run;
-        run += tsum[i];
+    __syncthreads();
+    uint64_t at = s_ex;
+    for (int k = 0; k < wv; k++) at += s_tot[k];
+    uint8_t *mids = p.out + NB_HDR + nlead;
+    if (fits) {
+        wave_copy_out(mids + at, sw, sum, lane);
+    } else {
+        // too many mid bytes for the stage: the run again, step by step
+        before = r0 > 0 ? (U)(to_bits<T>(xb - msub) >> P.shift) : (U)0;
+#pragma unroll 1
+        for (int s = 0; s < NB_STEPS; s++) {
+            const uint64_t e0 = r0 + (uint64_t)s * (64 * LV) + (uint64_t)lane * LV;
+            nb_load<T, LV>(p.x, e0, n, v);
+            const int nv = e0 >= n ? 0 : n - e0 < (uint64_t)LV ? (int)(n - e0) : LV;
+            st.encode(v, nv, before, msub, P.rb, P.shift, lane);
+            const uint32_t inc = seg_scan_incl<64>(st.tot, lane);
+            const uint32_t stot = __builtin_amdgcn_readlane(inc, 63);
+            wave_lds_fence();
+            wave_clear(sw, stot + 16, lane);
+            wave_lds_fence();
+            st.stage(reinterpret_cast<uint64_t *>(sw), inc - st.tot);
+            wave_lds_fence();
+            wave_copy_out(mids + at, sw, stot, lane);
+            at += stot;
+            before = last_lane(st.last);
+        }
     }
-    if (threadIdx.x == 1023) P->total = s[1023];
+    // the chunk aggregate last: its atomic's round trip stays off the tile's path
+    if (threadIdx.x == 0) lookback_chunk_done(L, tile, pend, total, 0);
 }
 
 // Header (szx_float.cc:1678-1688) and the results.
@@ -232,15 +330,14 @@ __global__ void k_nb_finish(uint64_t n, const NbParams *P, uint8_t *out, uint64_
     result[0] = 0;
     result[1] = NB_HDR + nlead + P->total;
     result[2] = f32_bits(P->eb);
-    result[3] = 0;
+    result[3] = (uint64_t)P->err;
 }
 
 // ---- decompression ----
 
 // szxd_float.cc:478-513: reqLength, median, lead-array size.
-__global__ void k_nb_header(const uint8_t *s, uint64_t len, uint64_t n, int w, NbParams *P, int32_t *status)
+__device__ inline int nb_check_header(const uint8_t *s, uint64_t len, uint64_t n, int w, NbParams &P)
 {
-    if (threadIdx.x != 0) return;
     int32_t rc = 0;
     const uint64_t nlead = (n + 3) / 4;
     int rl = 1;
@@ -257,282 +354,369 @@ __global__ void k_nb_header(const uint8_t *s, uint64_t len, uint64_t n, int w, N
         else if (NB_HDR + nlead > len) rc = -13;
     }
     if (rc) rl = 1;
-    P->len = rl;
-    P->rb = (rl + 7) >> 3;
-    P->shift = (-rl) & 7;
-    P->ok = rc == 0;
-    P->med = bits_f32(mb);
-    *status = rc;
+    P.len = rl;
+    P.rb = (rl + 7) >> 3;
+    P.shift = (-rl) & 7;
+    P.ok = rc == 0;
+    P.med = bits_f32(mb);
+    return rc;
 }
 
-// Lead code k of the lane's values from the stream.
-__device__ inline int nb_code(const uint8_t *s, uint64_t e)
+// The lane's lead-code bytes (zero past the array), its values from e0 on.
+template <int LV>
+__device__ inline uint32_t nb_codes(const uint8_t *s, uint64_t e0, uint64_t n, int nv)
 {
-    return (s[NB_HDR + (e >> 2)] >> (6 - 2 * (int)(e & 3))) & 3;
-}
-
-__global__ __launch_bounds__(256) void k_nb_dcount(const uint8_t *s, uint64_t n, const NbParams *Pp, uint32_t *tsum)
-{
-    const NbParams P = *Pp;
-    if (!P.ok) return;
-    const uint64_t e0 = blockIdx.x * (uint64_t)NB_TILE + threadIdx.x * (uint64_t)NB_PER;
-    uint32_t cnt = 0;
-    for (int k = 0; k < NB_PER; k++) {
-        if (e0 + k >= n) break;
-        const int ld = nb_code(s, e0 + k);
-        cnt += P.rb - (ld < P.rb ? ld : P.rb);
+    if (nv == LV) {
+        uint32_t c = 0;
+        __builtin_memcpy(&c, s + NB_HDR + e0 / 4, LV / 4);
+        return c;
     }
-    uint32_t total;
-    nb_block_excl(cnt, &total);
-    if (threadIdx.x == 0) tsum[blockIdx.x] = total;
-}
-
-// The payload must hold the mid bytes the lead codes ask for.
-__global__ void k_nb_check(uint64_t len, uint64_t n, NbParams *P, int32_t *status)
-{
-    if (threadIdx.x != 0 || !P->ok) return;
-    if (P->total > len - NB_HDR - (n + 3) / 4) {
-        P->ok = 0;
-        *status = -33;
+    uint32_t c = 0;
+    for (int b = 0; 4 * b < nv; b++) c |= (uint32_t)s[NB_HDR + e0 / 4 + b] << (8 * b);
+    if (nv & 3) {   // the codes past the last value do not count
+        const int b = nv >> 2;
+        const uint32_t keep = (0xFF00u >> (2 * (nv & 3))) & 0xFFu;
+        c &= ~((0xFFu & ~keep) << (8 * b));
     }
+    return c;
 }
 
-// The lane's words from the stream alone (inherited bytes still zero),
-// masked to the low 8W - shift bits, and its last-writer record.
+// What a tile says about itself: its mid bytes (low 16 bits), and for the
+// inheritable byte W-1-i (i = 0..2) the tile-relative mid byte that wrote it
+// last (bits 16 + 16 i): NB_NONE no value of the tile did, NB_ZERO a value
+// wrote a zero there (records of fewer than i + 1 bytes).
+constexpr uint32_t NB_NONE = 0xFFFF, NB_ZERO = 0xFFFE;
+
+// Lead codes alone: the tile's mid-byte count and last writers.
 template <typename T>
-__device__ inline uint32_t nb_words(const uint8_t *s, const uint8_t *mids, uint64_t n, uint64_t e0, const NbParams &P,
-                                    uint32_t q, int exact, typename Word<T>::U (&wv)[NB_PER], int (&lk)[NB_PER])
+__global__ __launch_bounds__(256) void k_nb_count(const uint8_t *s, uint64_t len, uint64_t n, NbParams *Pp,
+                                                  unsigned long long *trec, int32_t *status)
 {
-    using U = typename Word<T>::U;
-    constexpr int W = Word<T>::W;
-    const U mask = ~(U)0 >> P.shift;
-    uint32_t mine = 0;
-    for (int k = 0; k < NB_PER; k++) {
-        U cur = 0;
-        lk[k] = 0;
-        if (e0 + k < n) {
-            const int ld = nb_code(s, e0 + k);
-            lk[k] = ld < P.rb ? ld : P.rb;
-            for (int t = W - P.rb; t < W - lk[k]; t++) {
-                uint32_t src = (uint32_t)(t - (W - P.rb));
-                if (W == 8 && !exact && P.rb == 5 && lk[k] == 0 && t == 7) src = 3;   // szxd_double.cc:906
-                cur |= (U)mids[q + src] << (8 * t);
-            }
-            q += P.rb - lk[k];
-            cur &= mask;
-            uint32_t wr = 0;
-            for (int i = 0; i < 3; i++)
-                if (lk[k] <= i) wr |= ((uint32_t)(cur >> (8 * (W - 1 - i))) & 0xFFu) << (8 * i) | (1u << (24 + i));
-            mine = nb_combine(mine, wr);
-        }
-        wv[k] = cur;
+    constexpr int LV = NB_LV<T>;
+    __shared__ uint32_t s_tot[4], s_pos[3][4];
+    NbParams P{};
+    const int rc = nb_check_header(s, len, n, (int)sizeof(T), P);   // every workgroup checks: 17 cached bytes
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        *status = rc;
+        *Pp = P;
     }
-    return mine;
-}
-
-// Stage the tile's mid bytes [src, src + cnt) of the stream (ending at end)
-// into LDS words at byte offset (src & 3); returns that offset.
-__device__ inline uint32_t nb_stage(uint32_t *bw, const uint8_t *src, uint32_t cnt, const uint8_t *end)
-{
-    const uint32_t head = (uint32_t)((uintptr_t)src & 3);
-    const uint32_t *sw = reinterpret_cast<const uint32_t *>(src - head);
-    const uint32_t nw = (head + cnt + 3) / 4;
-    for (uint32_t i = threadIdx.x; i < nw; i += 256) {
-        const uint8_t *a = reinterpret_cast<const uint8_t *>(sw + i);
-        if (a + 4 <= end) {
-            bw[i] = sw[i];
-        } else {
-            uint32_t v = 0;
-            for (int j = 0; j < 4; j++)
-                if (a + j < end) v |= (uint32_t)a[j] << (8 * j);
-            bw[i] = v;
+    if (rc) return;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const uint64_t e0 = blockIdx.x * (uint64_t)NB_DTILE<T> + (uint64_t)threadIdx.x * LV;
+    const int nv = e0 >= n ? 0 : n - e0 < (uint64_t)LV ? (int)(n - e0) : LV;
+    const uint32_t code = nb_codes<LV>(s, e0, n, nv);
+    LaneCodes<LV> c;
+    c.set(code, P.rb, nv);
+    const uint32_t inc = seg_scan_incl<64>(c.tot, lane);
+    if (lane == 63) s_tot[wv] = inc;
+    if (lane < 3) s_pos[lane][wv] = NB_NONE;
+    __syncthreads();
+    uint32_t base = 0;
+    for (int k = 0; k < wv; k++) base += s_tot[k];
+    const uint32_t first = base + inc - c.tot;   // the lane's first mid byte in the tile
+    for (int i = 0; i < 3; i++) {
+        // the lane's last value with at most i lead bytes, if any
+        int last = -1;
+        for (int k = 0; k < LV; k++)
+            if (k < nv && ((c.z8[k & 3] >> (8 * (k >> 2))) & 0xFFu) <= 8u * i) last = k;
+        const unsigned long long any = __ballot(last >= 0);
+        if (any && lane == 63 - __builtin_clzll(any)) {
+            uint32_t off = 0;
+            for (int k = 0; k < LV; k++)
+                if (k == last) off = (c.pk[k & 3] >> (8 * (k >> 2))) & 0xFFu;
+            s_pos[i][wv] = i < P.rb ? first + off + (uint32_t)(P.rb - 1 - i) : NB_ZERO;
         }
     }
     __syncthreads();
-    return head;
-}
-
-template <typename T>
-__global__ __launch_bounds__(256) void k_nb_carry(const uint8_t *s, uint64_t len, uint64_t n, const NbParams *Pp,
-                                                  const uint64_t *toff, uint32_t *tcar, int exact)
-{
-    using U = typename Word<T>::U;
-    __shared__ uint32_t bw[(NB_TILE * sizeof(T)) / 4 + 2];
-    const NbParams P = *Pp;
-    if (!P.ok) return;
-    const uint64_t e0 = blockIdx.x * (uint64_t)NB_TILE + threadIdx.x * (uint64_t)NB_PER;
-    uint32_t cnt = 0;
-    for (int k = 0; k < NB_PER; k++) {
-        if (e0 + k >= n) break;
-        const int ld = nb_code(s, e0 + k);
-        cnt += P.rb - (ld < P.rb ? ld : P.rb);
+    if (threadIdx.x == 0) {
+        unsigned long long r = s_tot[0] + s_tot[1] + s_tot[2] + s_tot[3];
+        for (int i = 0; i < 3; i++) {
+            uint32_t at = NB_NONE;
+            for (int k = 0; k < 4; k++)
+                if (s_pos[i][k] != NB_NONE) at = s_pos[i][k];
+            r |= (unsigned long long)at << (16 + 16 * i);
+        }
+        trec[blockIdx.x] = r;
     }
-    uint32_t total;
-    const uint32_t ex = nb_block_excl(cnt, &total);
-    const uint32_t head = nb_stage(bw, s + NB_HDR + (n + 3) / 4 + toff[blockIdx.x], total, s + len);
-    U wv[NB_PER];
-    int lk[NB_PER];
-    const uint32_t mine = nb_words<T>(s, reinterpret_cast<const uint8_t *>(bw), n, e0, P, head + ex, exact, wv, lk);
-    uint32_t tot;
-    nb_block_excl_lw(mine, &tot);
-    if (threadIdx.x == 0) tcar[blockIdx.x] = tot;
 }
 
-// One workgroup: exclusive last-writer scan of the tile records (in place).
-__global__ __launch_bounds__(1024) void k_nb_carry_scan(uint32_t *tcar, uint64_t ntiles, const NbParams *P)
+// One tile's place: first mid byte, and per inheritable byte the mid byte of
+// the stream that an earlier tile wrote it from (NB_NO: none, a zero).
+constexpr uint64_t NB_NO = ~0ull;
+struct NbPlace {
+    uint64_t off, src[3];
+};
+
+__device__ inline void nb_step(NbPlace &a, unsigned long long r)
 {
-    __shared__ uint32_t s[1024];
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        const uint32_t q = (uint32_t)(r >> (16 + 16 * i)) & 0xFFFFu;
+        if (q != NB_NONE) a.src[i] = q == NB_ZERO ? NB_NO - 1 : a.off + q;
+    }
+    a.off += r & 0xFFFFu;
+}
+
+// One workgroup: exclusive scan of the tile records; the total, and whether
+// the payload holds the mid bytes the lead codes ask for.
+__global__ __launch_bounds__(1024) void k_nb_scan(const unsigned long long *trec, uint64_t ntiles, NbPlace *place,
+                                                  uint64_t len, uint64_t n, NbParams *P, int32_t *status)
+{
+    __shared__ NbPlace sw[16];
     if (!P->ok) return;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const uint64_t per = (ntiles + 1023) / 1024;
-    const uint64_t a = threadIdx.x * per, b = a + per < ntiles ? a + per : ntiles;
-    uint32_t acc = 0;
-    for (uint64_t i = a; i < b; i++) acc = nb_combine(acc, tcar[i]);
-    s[threadIdx.x] = acc;
-    __syncthreads();
-    for (int d = 1; d < 1024; d <<= 1) {
-        const uint32_t v = threadIdx.x >= (unsigned)d ? s[threadIdx.x - d] : 0u;
-        __syncthreads();
-        if (threadIdx.x >= (unsigned)d) s[threadIdx.x] = nb_combine(v, s[threadIdx.x]);
-        __syncthreads();
+    const uint64_t a = threadIdx.x * per < ntiles ? threadIdx.x * per : ntiles, b = a + per < ntiles ? a + per : ntiles;
+    // (off, last writers relative to the range's start) of this thread's tiles
+    NbPlace acc{0, {NB_NO, NB_NO, NB_NO}};
+    for (uint64_t i = a; i < b; i++) nb_step(acc, trec[i]);
+    // combine(x, y): y after x
+    const auto after = [](const NbPlace &x, const NbPlace &y) {
+        NbPlace r;
+        r.off = x.off + y.off;
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+            r.src[i] = y.src[i] == NB_NO ? x.src[i] : y.src[i] == NB_NO - 1 ? NB_NO - 1 : x.off + y.src[i];
+        return r;
+    };
+    NbPlace inc = acc;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        NbPlace o;
+        o.off = __shfl_up(inc.off, d, 64);
+#pragma unroll
+        for (int i = 0; i < 3; i++) o.src[i] = __shfl_up(inc.src[i], d, 64);
+        if (lane >= d) inc = after(o, inc);
     }
-    uint32_t run = threadIdx.x ? s[threadIdx.x - 1] : 0u;
+    if (lane == 63) sw[wv] = inc;
+    NbPlace run;
+    run.off = __shfl_up(inc.off, 1, 64);
+#pragma unroll
+    for (int i = 0; i < 3; i++) run.src[i] = __shfl_up(inc.src[i], 1, 64);
+    if (lane == 0) run = NbPlace{0, {NB_NO, NB_NO, NB_NO}};
+    __syncthreads();
+    NbPlace pre{0, {NB_NO, NB_NO, NB_NO}};
+    for (int k = 0; k < wv; k++) pre = after(pre, sw[k]);
+    run = after(pre, run);
     for (uint64_t i = a; i < b; i++) {
-        const uint32_t t = tcar[i];
-        tcar[i] = run;
-        run = nb_combine(run, t);
+        place[i] = run;
+        nb_step(run, trec[i]);
+    }
+    if (threadIdx.x == 1023) {   // its range ends the array (or is empty: run is the total either way)
+        P->total = run.off;
+        if (run.off > len - NB_HDR - (n + 3) / 4) {
+            P->ok = 0;
+            *status = -33;
+        }
     }
 }
 
+// One tile per workgroup: its mid bytes (contiguous in the stream) staged in
+// LDS, every lane's words, a last-writer scan over the workgroup, and the
+// values out through LDS in whole 16-byte chunks.  The tile's place, records
+// and lead codes are all in flight together; memory bounds it (256^3 fp32, REL
+// 1e-3: a carry pass of 40 us over all mid bytes and a decode of 103 with byte
+// reads and 64-byte-strided stores -> 20 us, 4.3 TB/s).
 template <typename T>
 __global__ __launch_bounds__(256) void k_nb_decode(const uint8_t *s, uint64_t len, uint64_t n, const NbParams *Pp,
-                                                   const uint64_t *toff, const uint32_t *tcar, T *out, int exact)
+                                                   const unsigned long long *trec, const NbPlace *place, T *out,
+                                                   int exact)
 {
-    using U = typename Word<T>::U;
+    typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
     constexpr int W = Word<T>::W;
-    __shared__ uint32_t bw[(NB_TILE * sizeof(T)) / 4 + 2];
+    constexpr int LV = NB_LV<T>;
+    constexpr int VC = 16 / W;
+    constexpr int DW = NB_DTILE<T> * W / 4 + 16;
+    __shared__ __attribute__((aligned(16))) uint32_t bw[DW];
+    __shared__ uint32_t s_tot[4], s_cd[4], s_cm[4], s_inh;
     const NbParams P = *Pp;
+    const NbPlace *at = place + blockIdx.x;
+    const uint64_t off = at->off;
+    const uint32_t total = (uint32_t)(trec[blockIdx.x] & 0xFFFFu);
     if (!P.ok) return;
-    const uint64_t e0 = blockIdx.x * (uint64_t)NB_TILE + threadIdx.x * (uint64_t)NB_PER;
-    uint32_t cnt = 0;
-    for (int k = 0; k < NB_PER; k++) {
-        if (e0 + k >= n) break;
-        const int ld = nb_code(s, e0 + k);
-        cnt += P.rb - (ld < P.rb ? ld : P.rb);
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const uint64_t e0 = blockIdx.x * (uint64_t)NB_DTILE<T> + (uint64_t)threadIdx.x * LV;
+    const int nv = e0 >= n ? 0 : n - e0 < (uint64_t)LV ? (int)(n - e0) : LV;
+    const uint8_t *mids = s + NB_HDR + (n + 3) / 4, *end = s + len;
+    // the tile's mid bytes: 16-byte loads that stay inside the stream (it
+    // starts NB_HDR bytes earlier at least), bytes at its very end
+    const uint8_t *src = mids + off;
+    const uint32_t head = (uint32_t)((uintptr_t)src & 15);
+    const uint32_t nchunk = total ? (head + total + 15) / 16 : 0;
+    const uint32_t c1 = nchunk && src - head + 16ull * nchunk > end ? nchunk - 1 : nchunk;
+    const u32x4_t *g = reinterpret_cast<const u32x4_t *>(src - head);
+    u32x4_t *sv = reinterpret_cast<u32x4_t *>(bw);
+    u32x4_t c0v{}, c1v{};
+    const uint32_t t = threadIdx.x;
+    if (t < c1) c0v = g[t];
+    if (t + 256 < c1) c1v = g[t + 256];
+    const uint32_t code = nb_codes<LV>(s, e0, n, nv);
+    uint32_t inherit = 0;   // the bytes the tile inherits, top byte highest
+    if (t < 3) {
+        const uint64_t q = at->src[t];
+        uint32_t b = q < NB_NO - 1 ? mids[q] : 0u;
+        if (t == 0) b &= 0xFFu >> P.shift;
+        // fp64 records of five bytes: byte 7 comes from the fourth mid byte
+        // (szxd_double.cc:906), here one before the position kept
+        if (t == 0 && W == 8 && !exact && P.rb == 5 && q < NB_NO - 1) b = mids[q - 1] & (0xFFu >> P.shift);
+        inherit = b << (24 - 8 * t);
     }
-    uint32_t total;
-    const uint32_t ex = nb_block_excl(cnt, &total);
-    const uint32_t head = nb_stage(bw, s + NB_HDR + (n + 3) / 4 + toff[blockIdx.x], total, s + len);
-    U wv[NB_PER];
-    int lk[NB_PER];
-    const uint32_t mine = nb_words<T>(s, reinterpret_cast<const uint8_t *>(bw), n, e0, P, head + ex, exact, wv, lk);
-    uint32_t tot;
-    const uint32_t cin = nb_combine(tcar[blockIdx.x], nb_block_excl_lw(mine, &tot));
-    U prev = ((U)(cin & 0xFFu) << (8 * (W - 1))) | ((U)((cin >> 8) & 0xFFu) << (8 * (W - 2))) |
-             ((U)((cin >> 16) & 0xFFu) << (8 * (W - 3)));
+    if (t < c1) sv[t] = c0v;
+    if (t + 256 < c1) sv[t + 256] = c1v;
+    for (uint32_t c = t + 512; c < c1; c += 256) sv[c] = g[c];
+    if (c1 != nchunk && t < 16) {
+        const uint8_t *a = src - head + 16ull * c1 + t;
+        if (a < end) reinterpret_cast<uint8_t *>(bw)[16 * c1 + t] = *a;
+    }
+    LaneCodes<LV> c;
+    c.set(code, P.rb, nv);
+    const uint32_t inc = seg_scan_incl<64>(c.tot, lane);
+    if (lane == 63) s_tot[wv] = inc;
+    __syncthreads();
+    uint32_t base = head;
+    for (int k = 0; k < wv; k++) base += s_tot[k];
+    LaneWords<T, LV> w;
+    w.gather(reinterpret_cast<const uint8_t *>(bw), base + inc - c.tot, c, P.rb, exact);
+    // last-writer scan: lanes of the wave, then the waves, then the tile's own
+    // inheritance; a lane past the array wrote nothing and passes on
+    uint32_t cd = w.top, cm = w.wrote;
+    if (nv == 0) {
+        cd = 0;
+        cm = 0;
+    }
+    seg_scan_last_writer_head<64>(cd, cm);
+    if (lane == 63) {
+        s_cd[wv] = cd;
+        s_cm[wv] = cm;
+    }
+    const uint32_t ld = seg_prev<64>(cd, lane), lm = seg_prev<64>(cm, lane);
+    if (wv == 0) {   // combined by wave 0, read by all after the barrier
+        inherit = (uint32_t)__builtin_amdgcn_readlane(inherit, 0) | (uint32_t)__builtin_amdgcn_readlane(inherit, 1) |
+                  (uint32_t)__builtin_amdgcn_readlane(inherit, 2);
+        if (lane == 0) s_inh = inherit;
+    }
+    __syncthreads();
+    uint32_t pre = s_inh;
+    for (int k = 0; k < wv; k++) pre = (s_cd[k] & s_cm[k]) | (pre & ~s_cm[k]);
+    const uint32_t cin = (ld & lm) | (pre & ~lm);
     const T med = (T)P.med;
-    for (int k = 0; k < NB_PER; k++) {
-        if (e0 + k >= n) break;
-        const U top = lk[k] ? ~(U)0 << (8 * (W - lk[k])) : (U)0;
-        const U cur = wv[k] | (prev & top);
-        out[e0 + k] = from_bits<T>(cur << P.shift) + med;
-        prev = cur;
+    T v[LV];
+#pragma unroll
+    for (int k = 0; k < LV; k++) v[k] = w.value(k, cin, P.shift, med);
+    const uint64_t t0 = blockIdx.x * (uint64_t)NB_DTILE<T>;
+    if (t0 + NB_DTILE<T> <= n) {
+        // out through the stage: whole chunks across the wave, permuted so
+        // that lanes 64 bytes apart use different banks
+        const auto slot = [](int k) { return k ^ ((k >> 3) & 3); };
+#pragma unroll
+        for (int k = 0; k < LV; k += VC) {
+            u32x4_t q;
+            __builtin_memcpy(&q, &v[k], 16);
+            sv[slot(((int)t * LV + k) / VC)] = q;
+        }
+        __syncthreads();
+        typedef unsigned int u32x4_ot __attribute__((ext_vector_type(4), aligned(4)));
+        u32x4_ot *ov = reinterpret_cast<u32x4_ot *>(out + t0);   // out needs its type's alignment only
+#pragma unroll
+        for (int k = (int)t; k < NB_DTILE<T> / VC; k += 256) __builtin_nontemporal_store((u32x4_ot)sv[slot(k)], ov + k);
+    } else {
+#pragma unroll
+        for (int k = 0; k < LV; k++)
+            if (k < nv) out[e0 + k] = v[k];
     }
 }
 
 // ---- host side ----
 
-static uint64_t nb_tiles(uint64_t n) { return n ? (n + NB_TILE - 1) / NB_TILE : 1; }
+static uint64_t nb_enc_tiles(uint64_t n, int w)
+{
+    const uint64_t t = w == 4 ? NB_TILE<float> : NB_TILE<double>;
+    return n ? (n + t - 1) / t : 1;
+}
+static uint64_t nb_dec_tiles(uint64_t n, int w)
+{
+    const uint64_t t = w == 4 ? NB_DTILE<float> : NB_DTILE<double>;
+    return n ? (n + t - 1) / t : 1;
+}
 
 uint64_t nb_capacity(uint64_t n, int w) { return NB_HDR + (n + 3) / 4 + n * (uint64_t)w + 16; }
 
-// params | range partials | tile sums (u32) | tile offsets (u64) | tile carries (u32)
-uint64_t nb_workspace(uint64_t n)
-{
-    const uint64_t t = nb_tiles(n);
-    auto al = [](uint64_t v) { return (v + 255) & ~255ull; };
-    return 256 + al(range_workspace_bytes()) + al(4 * t) + al(8 * t) + al(4 * t);
-}
-
+// One workspace serves both directions: parameters | range partials | tile
+// words, chunk words and accumulators (encoder; cleared by the range pass with
+// the parameters) or tile records and places (decoder).
 struct NbWs {
     NbParams *P;
-    float *eb;
-    void *mm;
-    uint8_t *range;
-    uint32_t *tsum;
-    uint64_t *toff;
-    uint32_t *tcar;
+    void *parts;
+    unsigned long long *tiles, *cacc;
+    ChunkState *chunks;
+    uint64_t zero_words;   // from P: parameters and look-back words
+    unsigned long long *trec;
+    NbPlace *place;
+    uint64_t bytes;
 };
 
-static NbWs nb_ws(uint8_t *ws, uint64_t n)
+static NbWs nb_ws(uint8_t *ws, uint64_t n, int w)
 {
-    const uint64_t t = nb_tiles(n);
+    const uint64_t te = nb_enc_tiles(n, w), td = nb_dec_tiles(n, w), ch = (te + LB_CHUNK - 1) / LB_CHUNK;
     auto al = [](uint64_t v) { return (v + 255) & ~255ull; };
     NbWs r;
     r.P = reinterpret_cast<NbParams *>(ws);
-    r.eb = reinterpret_cast<float *>(ws + 128);
-    r.mm = ws + 192;
     uint64_t off = 256;
-    r.range = ws + off; off += al(range_workspace_bytes());
-    r.tsum = reinterpret_cast<uint32_t *>(ws + off); off += al(4 * t);
-    r.toff = reinterpret_cast<uint64_t *>(ws + off); off += al(8 * t);
-    r.tcar = reinterpret_cast<uint32_t *>(ws + off);
+    r.tiles = reinterpret_cast<unsigned long long *>(ws + off); off += al(8 * te);
+    r.chunks = reinterpret_cast<ChunkState *>(ws + off); off += al(sizeof(ChunkState) * ch);
+    r.cacc = reinterpret_cast<unsigned long long *>(ws + off); off += al(8 * ch);
+    r.zero_words = off / 8;
+    r.parts = ws + off; off += al(2 * RANGE_LB_PARTS * sizeof(double));
+    uint64_t dec = 256;
+    r.trec = reinterpret_cast<unsigned long long *>(ws + dec); dec += al(8 * td);
+    r.place = reinterpret_cast<NbPlace *>(ws + dec); dec += al(sizeof(NbPlace) * td);
+    r.bytes = off > dec ? off : dec;
     return r;
+}
+
+uint64_t nb_workspace(uint64_t n, int w) { return nb_ws(nullptr, n, w).bytes; }
+
+template <typename T>
+static void nb_encode(const T *x, uint64_t n, int rel_mode, float abs_eb, float rel, uint8_t *d_out, const NbWs &S,
+                      hipStream_t st)
+{
+    range_partials_launch(x, n, (int)sizeof(T), S.parts, reinterpret_cast<unsigned long long *>(S.P), S.zero_words, st);
+    const uint64_t t = nb_enc_tiles(n, (int)sizeof(T));
+    const NbEncode<T> p{x, n, static_cast<const T *>(S.parts), rel_mode, abs_eb, rel, d_out, S.P, S.tiles, S.chunks,
+                        S.cacc, t};
+    timing_mark_begin(KK_COMPRESS, st);
+    hipLaunchKernelGGL(k_nb_encode<T>, dim3((unsigned)t), dim3(256), 0, st, p);
+    timing_mark_end(KK_COMPRESS, st);
 }
 
 void nb_compress_launch(const void *d_in, uint64_t n, int w, int rel_mode, float abs_eb, float rel, uint8_t *d_out,
                         uint8_t *d_ws, uint64_t *d_result, hipStream_t st)
 {
-    const NbWs S = nb_ws(d_ws, n);
-    const uint64_t t = nb_tiles(n);
-    range_bound_launch(d_in, n, w, rel, S.range, rel_mode ? S.eb : nullptr, S.mm, st);
-    const float *ebd = rel_mode ? S.eb : nullptr;
-    timing_mark_begin(KK_COMPRESS, st);
-    if (w == 4) {
-        hipLaunchKernelGGL(k_nb_setup<float>, dim3(1), dim3(64), 0, st, static_cast<const float *>(S.mm), ebd, abs_eb,
-                           S.P);
-        hipLaunchKernelGGL((k_nb_pass<float, false>), dim3((unsigned)t), dim3(256), 0, st,
-                           static_cast<const float *>(d_in), n, S.P, d_out, S.tsum, S.toff);
-    } else {
-        hipLaunchKernelGGL(k_nb_setup<double>, dim3(1), dim3(64), 0, st, static_cast<const double *>(S.mm), ebd,
-                           abs_eb, S.P);
-        hipLaunchKernelGGL((k_nb_pass<double, false>), dim3((unsigned)t), dim3(256), 0, st,
-                           static_cast<const double *>(d_in), n, S.P, d_out, S.tsum, S.toff);
-    }
-    hipLaunchKernelGGL(k_nb_scan, dim3(1), dim3(1024), 0, st, S.tsum, t, S.toff, S.P);
-    if (w == 4)
-        hipLaunchKernelGGL((k_nb_pass<float, true>), dim3((unsigned)t), dim3(256), 0, st,
-                           static_cast<const float *>(d_in), n, S.P, d_out, S.tsum, S.toff);
-    else
-        hipLaunchKernelGGL((k_nb_pass<double, true>), dim3((unsigned)t), dim3(256), 0, st,
-                           static_cast<const double *>(d_in), n, S.P, d_out, S.tsum, S.toff);
-    timing_mark_end(KK_COMPRESS, st);
+    const NbWs S = nb_ws(d_ws, n, w);
+    if (w == 4) nb_encode<float>(static_cast<const float *>(d_in), n, rel_mode, abs_eb, rel, d_out, S, st);
+    else nb_encode<double>(static_cast<const double *>(d_in), n, rel_mode, abs_eb, rel, d_out, S, st);
     hipLaunchKernelGGL(k_nb_finish, dim3(1), dim3(64), 0, st, n, S.P, d_out, d_result);
+}
+
+template <typename T>
+static void nb_decode(const uint8_t *d_stream, uint64_t len, uint64_t n, T *d_out, const NbWs &S, int exact,
+                      int32_t *d_status, hipStream_t st)
+{
+    const uint64_t t = nb_dec_tiles(n, (int)sizeof(T));
+    timing_mark_begin(KK_DECODE, st);
+    hipLaunchKernelGGL(k_nb_count<T>, dim3((unsigned)t), dim3(256), 0, st, d_stream, len, n, S.P, S.trec, d_status);
+    hipLaunchKernelGGL(k_nb_scan, dim3(1), dim3(1024), 0, st, S.trec, t, S.place, len, n, S.P, d_status);
+    hipLaunchKernelGGL(k_nb_decode<T>, dim3((unsigned)t), dim3(256), 0, st, d_stream, len, n, S.P, S.trec, S.place,
+                       d_out, exact);
+    timing_mark_end(KK_DECODE, st);
 }
 
 void nb_decompress_launch(const uint8_t *d_stream, uint64_t len, uint64_t n, int w, void *d_out, uint8_t *d_ws,
                           int exact, int32_t *d_status, hipStream_t st)
 {
-    const NbWs S = nb_ws(d_ws, n);
-    const uint64_t t = nb_tiles(n);
-    hipLaunchKernelGGL(k_nb_header, dim3(1), dim3(64), 0, st, d_stream, len, n, w, S.P, d_status);
-    timing_mark_begin(KK_DECODE, st);
-    hipLaunchKernelGGL(k_nb_dcount, dim3((unsigned)t), dim3(256), 0, st, d_stream, n, S.P, S.tsum);
-    hipLaunchKernelGGL(k_nb_scan, dim3(1), dim3(1024), 0, st, S.tsum, t, S.toff, S.P);
-    hipLaunchKernelGGL(k_nb_check, dim3(1), dim3(64), 0, st, len, n, S.P, d_status);
-    if (w == 4) {
-        hipLaunchKernelGGL(k_nb_carry<float>, dim3((unsigned)t), dim3(256), 0, st, d_stream, len, n, S.P, S.toff,
-                           S.tcar, exact);
-        hipLaunchKernelGGL(k_nb_carry_scan, dim3(1), dim3(1024), 0, st, S.tcar, t, S.P);
-        hipLaunchKernelGGL(k_nb_decode<float>, dim3((unsigned)t), dim3(256), 0, st, d_stream, len, n, S.P, S.toff,
-                           S.tcar, static_cast<float *>(d_out), exact);
-    } else {
-        hipLaunchKernelGGL(k_nb_carry<double>, dim3((unsigned)t), dim3(256), 0, st, d_stream, len, n, S.P, S.toff,
-                           S.tcar, exact);
-        hipLaunchKernelGGL(k_nb_carry_scan, dim3(1), dim3(1024), 0, st, S.tcar, t, S.P);
-        hipLaunchKernelGGL(k_nb_decode<double>, dim3((unsigned)t), dim3(256), 0, st, d_stream, len, n, S.P, S.toff,
-                           S.tcar, static_cast<double *>(d_out), exact);
-    }
-    timing_mark_end(KK_DECODE, st);
+    const NbWs S = nb_ws(d_ws, n, w);
+    if (w == 4) nb_decode<float>(d_stream, len, n, static_cast<float *>(d_out), S, exact, d_status, st);
+    else nb_decode<double>(d_stream, len, n, static_cast<double *>(d_out), S, exact, d_status, st);
 }
 
 // SZx_fast_decompress_pred (szxd_float.cc:25-32): x[i] += pred[i] after a

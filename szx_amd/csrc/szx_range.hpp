@@ -1,0 +1,64 @@
+// szx_range.hpp -- the value range of a whole array inside the kernel that
+// needs it: a range pass (range_partials_launch) leaves RANGE_LB_PARTS {min,
+// max} pairs, and every wave of the next kernel folds them itself, so no
+// launch and no barrier lies between the two.
+#pragma once
+
+#include "szx_batch.hpp"
+#include "szx_common.hpp"
+#include "szx_wave.hpp"
+
+namespace szxamd {
+
+template <typename T> struct RangeFold {
+    static constexpr int PL = RANGE_LB_PARTS / 64;   // partials per lane
+    static_assert(RANGE_LB_PARTS % 128 == 0, "whole 16-byte loads per lane");
+    T mn[PL], mx[PL];
+    T first;
+    // issue the loads (parts 16-byte aligned; x[0] decides the NaN rule)
+    __device__ void load(const T *parts, const T *x)
+    {
+        const T *q = parts + 2 * PL * (threadIdx.x & 63);
+#pragma unroll
+        for (int k = 0; k < PL; k++) {
+            mn[k] = q[2 * k];
+            mx[k] = q[2 * k + 1];
+        }
+        first = x[0];
+    }
+    // Min and max skip NaNs (the partials hold none), except that a NaN x[0]
+    // makes both NaN, as the reference's comparisons do (szx_float.cc:478-493).
+    __device__ void minmax(T &lo, T &hi) const
+    {
+        using U = typename Word<T>::U;
+        T a = mn[0], b = mx[0];
+#pragma unroll
+        for (int k = 1; k < PL; k++) {
+            a = mn[k] < a ? mn[k] : a;
+            b = mx[k] > b ? mx[k] : b;
+        }
+        a = from_bits<T>(seg_reduce<64>(to_bits<T>(a), [](U x, U y) {
+            const T fx = from_bits<T>(x), fy = from_bits<T>(y);
+            return fy < fx ? y : x;
+        }));
+        b = from_bits<T>(seg_reduce<64>(to_bits<T>(b), [](U x, U y) {
+            const T fx = from_bits<T>(x), fy = from_bits<T>(y);
+            return fy > fx ? y : x;
+        }));
+        if (first != first) {
+            a = first;
+            b = first;
+        }
+        lo = a;
+        hi = b;
+    }
+    // The REL bound, rounded as the reference rounds it: fl32(range * rel) for
+    // fp32, (float)(range * (double)rel) for fp64 (szx.cc:249-253, 303-308).
+    static __device__ float bound(T lo, T hi, float rel)
+    {
+        const T range = hi - lo;
+        return (float)(range * (T)rel);
+    }
+};
+
+}  // namespace szxamd

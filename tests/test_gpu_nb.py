@@ -102,3 +102,42 @@ def test_non_blocked_rejects_damage(device):
     st = torch.from_numpy(np.frombuffer(bytes(s), np.uint8).copy()).to(device)
     c.decompress(st, len(s), Z.DECODE_REFERENCE)
     assert c.check() != 0
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_non_blocked_edges(dtype, device):
+    """Sizes around a wave step, a wave's run and a workgroup's tile; mid bytes
+    that fit a wave's stage and that do not; bytes inherited over many tiles;
+    input and output at their type's alignment only."""
+    import torch
+    r = np.random.default_rng(9)
+    step = 1024 if dtype == np.float32 else 512
+    for n in (1, step - 1, step + 1, 4 * step, 4 * step + 5, 16 * step, 16 * step + 3, 150 * step + 7):
+        t = np.arange(n)
+        for kind, rel in (("noise", 1e-12), ("noise", 1e-3), ("flat", 1e-3), ("smooth", 1e-4)):
+            if kind == "noise":
+                x = r.standard_normal(n)
+            elif kind == "flat":   # one value but for the first two: every byte inherited
+                x = np.where(t < 2, t - 0.5, 0.3)
+            else:
+                x = np.sin(t * 1e-4) + 2.0
+            x = x.astype(dtype)
+            eb = float(np.float32((float(np.ptp(x)) + 1e-30) * rel))
+            say("nb edge", dtype.__name__, n, kind, rel)
+            room = torch.zeros(n + 1, dtype=torch.float32 if dtype == np.float32 else torch.float64, device=device)
+            room[1:] = torch.from_numpy(x).to(device)
+            c = Z.DeviceNonBlocked(n, dtype)
+            c.compress(room[1:], Z.ABS, eb)
+            view, size, _ = c.stream_view()
+            s = view.cpu().numpy().tobytes()
+            assert s == O.compress_nb(x, eb)
+            back = torch.full_like(room, -7.0)
+            c.dec = back[1:]
+            buf = torch.empty(size + 3, dtype=torch.uint8, device=device)
+            buf[3:] = view
+            for flags in (Z.DECODE_REFERENCE, Z.DECODE_EXACT):
+                c.decompress(buf[3:], size, flags)
+                assert c.check() == 0
+                want = O.decompress_nb(s, n, dtype, ref_quirk=flags == Z.DECODE_REFERENCE)
+                assert bits_equal(c.dec.cpu().numpy(), want)
+            assert float(back[0]) == -7.0
