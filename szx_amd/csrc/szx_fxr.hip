@@ -19,6 +19,7 @@
 //    bounds eb_k = 2^e (1 + k / OCT_BINS), k = 0 .. OCT_BINS-1.
 #include "szx_common.hpp"
 #include "szx_fxr.hpp"
+#include "szx_wave.hpp"
 
 namespace szxamd {
 
@@ -512,30 +513,330 @@ __global__ __launch_bounds__(256) void k_rate_stats(const T *x, uint64_t n, int 
     for (int k = threadIdx.x; k < RATE_HIST; k += 256) o.hist[k] = s_hist[k];
 }
 
-// Fold wg_per_chunk partials per chunk (one workgroup per chunk).
-__global__ void k_rate_stats_fold(const RateStats *part, int wg_per_chunk, RateStats *out)
+// ---------------------------------------------------------------------------
+// 2b. the same two passes for power-of-two block sizes
+// ---------------------------------------------------------------------------
+// A block is an aligned group of BS / LV lanes, each lane holding LV
+// consecutive values (the compressor's layout), so the block extremes and sums
+// are a few DPP steps for as many blocks as a wave holds, where one wave per
+// block spends most of its time in 64-lane shuffles.  A wave takes steps of
+// 64 x LV values, the next step's loads in flight while it works on one.
+// 256^3 fp32, bs 128: octave pair with edges 109 -> 31 us, statistics 61 -> 20
+// (memory bound from here: 67 MB).
+
+template <typename T, int BS> struct TiledRate {
+    static constexpr int LV = sizeof(T) == 4 ? 16 : 8;
+    static constexpr int SEG = BS / LV;
+    static constexpr int STEP = 64 * LV;
+    static_assert(SEG >= 1 && (BS & (BS - 1)) == 0, "aligned lane groups");
+};
+
+template <typename T, int LV>
+__device__ inline void rate_load(const T *x, uint64_t e0, uint64_t n, T (&v)[LV])
 {
-    const RateStats *p = part + (uint64_t)blockIdx.x * wg_per_chunk;
-    RateStats &o = out[blockIdx.x];
-    for (int k = threadIdx.x; k < RATE_HIST; k += blockDim.x) {
-        unsigned h = 0;
-        for (int g = 0; g < wg_per_chunk; g++) h += p[g].hist[k];
-        o.hist[k] = h;
+    // x needs no more than its type's alignment
+    typedef unsigned int u32x4_t __attribute__((ext_vector_type(4), aligned(4)));
+    constexpr int VC = 16 / (int)sizeof(T);
+    if (e0 + LV <= n) {
+#pragma unroll
+        for (int k = 0; k < LV; k += VC) {
+            const u32x4_t q = *reinterpret_cast<const u32x4_t *>(x + e0 + k);
+            __builtin_memcpy(&v[k], &q, 16);
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < LV; k++) v[k] = e0 + k < n ? x[e0 + k] : (T)0;
+    }
+}
+
+// Block extremes: NaNs never win a comparison and a NaN first value makes both
+// NaN (block_min_max); nv = the lane's values inside the array.
+template <typename T, int SEG, int LV>
+__device__ inline void tiled_min_max(const T (&v)[LV], int nv, T &lo, T &hi)
+{
+    lo = nv > 0 ? v[0] : (T)__builtin_inf();
+    hi = nv > 0 ? v[0] : (T)-__builtin_inf();
+#pragma unroll
+    for (int k = 1; k < LV; k++)
+        if (k < nv) {
+            lo = __builtin_elementwise_min(lo, v[k]);
+            hi = __builtin_elementwise_max(hi, v[k]);
+        }
+    lo = from_bits<T>(seg_reduce<SEG>(to_bits<T>(lo), [](auto a, auto b) {
+        return to_bits<T>(__builtin_elementwise_min(from_bits<T>(a), from_bits<T>(b)));
+    }));
+    hi = from_bits<T>(seg_reduce<SEG>(to_bits<T>(hi), [](auto a, auto b) {
+        return to_bits<T>(__builtin_elementwise_max(from_bits<T>(a), from_bits<T>(b)));
+    }));
+    const T first = from_bits<T>(seg_first<SEG>(to_bits<T>(v[0])));
+    if (first != first) lo = hi = first;
+}
+
+// Leading zero bits of every value's word XOR the word before it in its block
+// (capped at 32): shifting both words right by s adds s, so one count serves
+// every bound.
+template <typename T, int SEG, int LV>
+__device__ inline void lead_zeros(const T (&v)[LV], T med, int lane, uint32_t (&lz)[LV])
+{
+    using U = typename Word<T>::U;
+    U prev = seg_prev<SEG>(to_bits<T>(v[LV - 1] - med), lane);
+#pragma unroll
+    for (int k = 0; k < LV; k++) {
+        const U w = to_bits<T>(v[k] - med);
+        const U xr = w ^ prev;
+        lz[k] = (uint32_t)__builtin_clzg(sizeof(U) == 4 ? (uint32_t)xr : (uint32_t)((uint64_t)xr >> 32), 32);
+        prev = w;
+    }
+}
+
+// k_rate_octave for power-of-two block sizes (the same accumulators).
+template <typename T, int BS, bool EDGES, int NOCT>
+__global__ __launch_bounds__(256) void k_rate_octave_tiled(const T *x, uint64_t n, int reqexp, unsigned long long *acc)
+{
+    using S = TiledRate<T, BS>;
+    constexpr int W = Word<T>::W, LV = S::LV, SEG = S::SEG;
+    constexpr int EDGE = NOCT * OCT_ACC;
+    constexpr int WIDTH = EDGE + (EDGES ? 4 : 0);
+    __shared__ unsigned long long s_acc[WIDTH];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, lseg = lane & (SEG - 1);
+    for (int k = threadIdx.x; k < WIDTH; k += 256) s_acc[k] = 0;
+    __syncthreads();
+    const uint64_t nsteps = (n + S::STEP - 1) / S::STEP, stride = gridDim.x * 4ull;
+    double lo_edge[NOCT];   // 2^(reqexp-j), exact for every float exponent
+#pragma unroll
+    for (int j = 0; j < NOCT; j++) lo_edge[j] = ldexp(1.0, reqexp - j);
+    const double top = 2.0 * lo_edge[0];
+    const double below = (double)nextafterf(ldexpf(1.0f, reqexp - NOCT + 1), 0.0f);
+    unsigned long long fixed[NOCT] = {}, a_const = 0, a_rec = 0, b_const = 0, b_rec = 0;
+    uint64_t s = blockIdx.x * 4ull + wv;
+    T v[LV];
+    if (s < nsteps) rate_load<T, LV>(x, s * S::STEP + (uint64_t)(LV * lane), n, v);
+    for (; s < nsteps; s += stride) {
+        T nx[LV];
+        if (s + stride < nsteps) rate_load<T, LV>(x, (s + stride) * S::STEP + (uint64_t)(LV * lane), n, nx);
+        const uint64_t e0 = s * S::STEP + (uint64_t)(LV * lane), b0 = e0 - (uint64_t)(LV * lseg);
+        const int nv = e0 >= n ? 0 : n - e0 < (uint64_t)LV ? (int)(n - e0) : LV;
+        const int cnt = b0 >= n ? 0 : n - b0 < (uint64_t)BS ? (int)(n - b0) : BS;
+        T lo, hi;
+        tiled_min_max<T, SEG, LV>(v, nv, lo, hi);
+        const T r = (hi - lo) / 2;
+        const float rf = (float)r, mf = (float)(lo + r);
+        const double rd = (double)r;
+        const int re = rad_expo(rf);
+        uint32_t lz[LV];
+        lead_zeros<T, SEG, LV>(v, (T)mf, lane, lz);
+        // record bytes at bound exponent e (record_bytes)
+        const auto record = [&](int e) -> uint32_t {
+            int clamped;
+            const int len = req_length<T>(re, e, clamped);
+            const int rb = (len + 7) >> 3;
+            const uint32_t shift = (uint32_t)(-len) & 7u, cap = rb < 3 ? (uint32_t)rb : 3u;
+            uint32_t leads = 0;
+            // the fp32 payload uses the zeroed median when the length clamps;
+            // the fp64 payload keeps the real one (szx_double.cc:2027-2030)
+            if (W == 4 && __builtin_amdgcn_ballot_w64(clamped)) {
+                uint32_t lc[LV];
+                lead_zeros<T, SEG, LV>(v, clamped ? (T)0 : (T)mf, lane, lc);
+#pragma unroll
+                for (int k = 0; k < LV; k++) {
+                    const uint32_t ld = (lc[k] + shift) >> 3;
+                    leads += k < nv ? (ld < cap ? ld : cap) : 0u;
+                }
+            } else {
+#pragma unroll
+                for (int k = 0; k < LV; k++) {
+                    const uint32_t ld = (lz[k] + shift) >> 3;
+                    leads += k < nv ? (ld < cap ? ld : cap) : 0u;
+                }
+            }
+            leads = seg_reduce<SEG>(leads, [](uint32_t a, uint32_t b) { return a + b; });
+            return 5u + (uint32_t)(cnt + 3) / 4u + (uint32_t)rb * (uint32_t)cnt - leads;
+        };
+        // a NaN radius is never constant; whole segments take every branch
+        // alike, and a pass no block of the wave needs is left out
+        const bool mine = lseg == 0 && cnt > 0;
+        if (EDGES) {
+            const bool ca = rd <= top, cb = rd <= below;
+            if (__builtin_amdgcn_ballot_w64(cnt > 0 && !ca)) {
+                const uint32_t rec = record(reqexp + 1);
+                if (mine && !ca) a_rec += rec;
+            }
+            if (__builtin_amdgcn_ballot_w64(cnt > 0 && !cb)) {
+                const uint32_t rec = record(reqexp - NOCT);
+                if (mine && !cb) b_rec += rec;
+            }
+            a_const += mine && ca;
+            b_const += mine && cb;
+        }
+#pragma unroll
+        for (int j = 0; j < NOCT; j++) {
+            const bool con = rd <= lo_edge[j];
+            fixed[j] += mine && con ? 4u : 0u;
+            if (!__builtin_amdgcn_ballot_w64(cnt > 0 && !con)) continue;
+            const uint32_t rec = record(reqexp - j);
+            if (!mine || con) continue;
+            if (!(rd <= 2.0 * lo_edge[j])) {
+                fixed[j] += rec;
+            } else {
+                // bin k holds radii in (2^e (1 + k/B), 2^e (1 + (k+1)/B)]
+                const double t = (ldexp(rd, j - reqexp) - 1.0) * OCT_BINS;   // in (0, OCT_BINS]
+                const int k = t >= OCT_BINS ? OCT_BINS - 1 : (t <= 1.0 ? 0 : (int)ceil(t) - 1);
+                atomicAdd(&s_acc[j * OCT_ACC + 1 + 2 * k], 1ull);
+                atomicAdd(&s_acc[j * OCT_ACC + 2 + 2 * k], (unsigned long long)rec);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < LV; k++) v[k] = nx[k];
+    }
+#pragma unroll
+    for (int j = 0; j < NOCT; j++) fixed[j] = wave_sum64(fixed[j]);
+    if (EDGES) {
+        a_const = wave_sum64(a_const);
+        a_rec = wave_sum64(a_rec);
+        b_const = wave_sum64(b_const);
+        b_rec = wave_sum64(b_rec);
+    }
+    if (lane == 0) {
+#pragma unroll
+        for (int j = 0; j < NOCT; j++)
+            if (fixed[j]) atomicAdd(&s_acc[j * OCT_ACC], fixed[j]);
+        if (EDGES) {
+            if (a_const) atomicAdd(&s_acc[EDGE + 0], a_const);
+            if (a_rec) atomicAdd(&s_acc[EDGE + 1], a_rec);
+            if (b_const) atomicAdd(&s_acc[EDGE + 2], b_const);
+            if (b_rec) atomicAdd(&s_acc[EDGE + 3], b_rec);
+        }
+    }
+    __syncthreads();
+    for (int k = threadIdx.x; k < WIDTH; k += 256)
+        if (s_acc[k]) atomicAdd(&acc[k], s_acc[k]);
+}
+
+// k_rate_stats for power-of-two block sizes: a wave's slice of the chunk is
+// contiguous (RATE_CHUNK / RATE_WG_PER_CHUNK / 4 values).
+template <typename T, int BS>
+__global__ __launch_bounds__(256) void k_rate_stats_tiled(const T *x, uint64_t n, RateStats *part)
+{
+    using S = TiledRate<T, BS>;
+    constexpr int LV = S::LV, SEG = S::SEG;
+    constexpr uint64_t SLICE = RATE_CHUNK / RATE_WG_PER_CHUNK;
+    constexpr int STEPS = (int)(SLICE / 4 / S::STEP);
+    static_assert(STEPS >= 1 && SLICE % (4 * S::STEP) == 0, "whole steps");
+    __shared__ double s_d[4][7];
+    __shared__ unsigned s_hist[RATE_HIST];
+    __shared__ unsigned s_cnt[2];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, lseg = lane & (SEG - 1);
+    for (int k = threadIdx.x; k < RATE_HIST; k += 256) s_hist[k] = 0;
+    if (threadIdx.x < 2) s_cnt[threadIdx.x] = 0;
+    const uint64_t w0 = blockIdx.x * SLICE + (uint64_t)wv * (SLICE / 4);
+    T v[LV];
+    rate_load<T, LV>(x, w0 + (uint64_t)(LV * lane), n, v);
+    __syncthreads();
+    double lo = __builtin_inf(), hi = -__builtin_inf(), sx = 0, sxx = 0, sa = 0, sq = 0, s2 = 0;
+    unsigned blocks = 0, zero = 0;
+#pragma unroll 1
+    for (int s = 0; s < STEPS; s++) {
+        const uint64_t e0 = w0 + (uint64_t)(s * S::STEP) + (uint64_t)(LV * lane);
+        T nx[LV];
+        if (s + 1 < STEPS) rate_load<T, LV>(x, e0 + S::STEP, n, nx);
+        const int nv = e0 >= n ? 0 : n - e0 < (uint64_t)LV ? (int)(n - e0) : LV;
+        const bool exists = e0 - (uint64_t)(LV * lseg) < n;
+        T blo, bhi;
+        tiled_min_max<T, SEG, LV>(v, nv, blo, bhi);
+        if (lseg == 0 && exists) {
+            const float r = (float)((bhi - blo) / 2);
+            blocks++;
+            zero += r == 0.0f;
+            atomicAdd(&s_hist[(f32_bits(r) >> 23) & 0xFF], 1u);
+        }
+        if (exists) {
+            lo = (double)blo < lo ? (double)blo : lo;
+            hi = (double)bhi > hi ? (double)bhi : hi;
+        }
+        // first and second differences inside the block; the value before the
+        // lane's first one and the difference before it come from the lane
+        // before (every lane before a block's last one is full)
+        double before = (double)from_bits<T>(seg_prev<SEG>(to_bits<T>(v[LV - 1]), lane));
+        double dbefore = before - (double)from_bits<T>(seg_prev<SEG>(to_bits<T>(v[LV - 2]), lane));
+#pragma unroll
+        for (int k = 0; k < LV; k++) {
+            const double xv = (double)v[k], d1 = xv - before;
+            if (k < nv) {
+                sx += xv;
+                sxx += xv * xv;
+                if (k >= 1 || lseg) {
+                    sa += fabs(d1);
+                    sq += d1 * d1;
+                }
+                if (k >= 2 || lseg) s2 += fabs(d1 - dbefore);
+            }
+            before = xv;
+            dbefore = d1;
+        }
+#pragma unroll
+        for (int k = 0; k < LV; k++) v[k] = nx[k];
+    }
+    double acc[7] = {lo, hi, sx, sxx, sa, sq, s2};
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) {
+        double o = __shfl_xor(acc[0], m, 64);
+        acc[0] = o < acc[0] ? o : acc[0];
+        o = __shfl_xor(acc[1], m, 64);
+        acc[1] = o > acc[1] ? o : acc[1];
+#pragma unroll
+        for (int k = 2; k < 7; k++) acc[k] += __shfl_xor(acc[k], m, 64);
+    }
+    if (blocks) atomicAdd(&s_cnt[0], blocks);
+    if (zero) atomicAdd(&s_cnt[1], zero);
+    if (lane == 0)
+        for (int k = 0; k < 7; k++) s_d[wv][k] = acc[k];
+    __syncthreads();
+    RateStats &o = part[blockIdx.x];
+    if (threadIdx.x < 7) {
+        const int k = threadIdx.x;
+        double a = s_d[0][k];
+        for (int w = 1; w < 4; w++) {
+            const double b = s_d[w][k];
+            a = k == 0 ? (b < a ? b : a) : k == 1 ? (b > a ? b : a) : a + b;
+        }
+        o.d[k] = a;
     }
     if (threadIdx.x == 0) {
-        double a[7];
-        for (int k = 0; k < 7; k++) a[k] = p[0].d[k];
-        unsigned blocks = p[0].blocks, zero = p[0].zero;
-        for (int g = 1; g < wg_per_chunk; g++) {
-            a[0] = p[g].d[0] < a[0] ? p[g].d[0] : a[0];
-            a[1] = p[g].d[1] > a[1] ? p[g].d[1] : a[1];
-            for (int k = 2; k < 7; k++) a[k] += p[g].d[k];
-            blocks += p[g].blocks;
-            zero += p[g].zero;
-        }
-        for (int k = 0; k < 7; k++) o.d[k] = a[k];
-        o.blocks = blocks;
-        o.zero = zero;
+        const uint64_t c0 = blockIdx.x / RATE_WG_PER_CHUNK * RATE_CHUNK;
+        o.blocks = s_cnt[0];
+        o.zero = s_cnt[1];
+        o.values = (c0 + RATE_CHUNK < n ? c0 + RATE_CHUNK : n) - c0;
+    }
+    for (int k = threadIdx.x; k < RATE_HIST; k += 256) o.hist[k] = s_hist[k];
+}
+
+// Fold RATE_WG_PER_CHUNK partials per chunk (one workgroup per chunk): a
+// column of the statistics per lane, every lane's loads independent.
+__global__ __launch_bounds__(256) void k_rate_stats_fold(const RateStats *part, RateStats *out)
+{
+    constexpr int G = RATE_WG_PER_CHUNK;
+    const RateStats *p = part + (uint64_t)blockIdx.x * G;
+    RateStats &o = out[blockIdx.x];
+    unsigned h = 0;
+#pragma unroll
+    for (int g = 0; g < G; g++) h += p[g].hist[threadIdx.x];
+    static_assert(RATE_HIST == 256, "one bin per lane");
+    o.hist[threadIdx.x] = h;
+    const int k = threadIdx.x;
+    if (k < 7) {
+        double t[G];
+#pragma unroll
+        for (int g = 0; g < G; g++) t[g] = p[g].d[k];
+        double a = t[0];
+#pragma unroll
+        for (int g = 1; g < G; g++) a = k == 0 ? (t[g] < a ? t[g] : a) : k == 1 ? (t[g] > a ? t[g] : a) : a + t[g];
+        o.d[k] = a;
+    } else if (k == 64 || k == 65) {   // blocks, zero-radius blocks
+        unsigned a = 0;
+#pragma unroll
+        for (int g = 0; g < G; g++) a += k == 64 ? p[g].blocks : p[g].zero;
+        (k == 64 ? o.blocks : o.zero) = a;
+    } else if (k == 66) {
         o.values = p[0].values;
     }
 }
@@ -552,14 +853,20 @@ __device__ inline float log2_ratio(double a, double r)
 __global__ void k_rate_ladder(const RateStats *st, int nchunks, int K, float *ebs)
 {
     __shared__ double s_range;
-    if (threadIdx.x == 0) {
+    if (threadIdx.x < 64) {   // the first wave folds the chunks' extremes
         double lo = st[0].d[0], hi = st[0].d[1];
-        for (int c = 1; c < nchunks; c++) {
+        for (int c = threadIdx.x; c < nchunks; c += 64) {
             lo = st[c].d[0] < lo ? st[c].d[0] : lo;
             hi = st[c].d[1] > hi ? st[c].d[1] : hi;
         }
+        for (int m = 1; m < 64; m <<= 1) {
+            double o = __shfl_xor(lo, m, 64);
+            lo = o < lo ? o : lo;
+            o = __shfl_xor(hi, m, 64);
+            hi = o > hi ? o : hi;
+        }
         const double r = hi - lo;
-        s_range = r > 0 ? r : 1.0;
+        if (threadIdx.x == 0) s_range = r > 0 ? r : 1.0;
     }
     __syncthreads();
     for (int k = threadIdx.x; k < K; k += blockDim.x) ebs[k] = (float)(s_range * exp2(-0.25 * k));
@@ -580,14 +887,15 @@ __global__ __launch_bounds__(256) void k_rate_inputs(const RateStats *st, int nc
     __shared__ unsigned s_pre[RATE_HIST + 1];   // s_pre[b] = blocks with exponent field < b
     const int c = blockIdx.x;
     const RateStats &s = st[c];
-    if (threadIdx.x == 0) {
-        unsigned a = 0;
-        for (int b = 0; b < RATE_HIST; b++) {
-            s_pre[b] = a;
-            a += s.hist[b];
-        }
-        s_pre[RATE_HIST] = a;
-    }
+    // prefix sums of the 256 bins: one per lane, waves joined through LDS
+    __shared__ unsigned s_wave[4];
+    const unsigned inc = seg_scan_incl<64>(s.hist[threadIdx.x], threadIdx.x & 63);
+    if ((threadIdx.x & 63) == 63) s_wave[threadIdx.x >> 6] = inc;
+    __syncthreads();
+    unsigned pre = 0;
+    for (unsigned w = 0; w < threadIdx.x >> 6; w++) pre += s_wave[w];
+    if (threadIdx.x == 0) s_pre[0] = 0;
+    s_pre[threadIdx.x + 1] = pre + inc;
     __syncthreads();
     double range = s.d[1] - s.d[0];
     if (!(range > 0)) range = 1e-300;
@@ -701,22 +1009,41 @@ uint64_t rate_stats_workspace_bytes(uint64_t n)
     return (nchunks ? nchunks : 1) * RATE_WG_PER_CHUNK * sizeof(RateStats);
 }
 
+template <typename T, int BS>
+static void stats_tiled_bs(const void *x, uint64_t n, RateStats *part, unsigned g, hipStream_t st)
+{
+    hipLaunchKernelGGL((k_rate_stats_tiled<T, BS>), dim3(g), dim3(256), 0, st, static_cast<const T *>(x), n, part);
+}
+template <typename T>
+static bool stats_tiled(int bs, const void *x, uint64_t n, RateStats *part, unsigned g, hipStream_t st)
+{
+    switch (bs) {
+    case 32: stats_tiled_bs<T, 32>(x, n, part, g, st); return true;
+    case 64: stats_tiled_bs<T, 64>(x, n, part, g, st); return true;
+    case 128: stats_tiled_bs<T, 128>(x, n, part, g, st); return true;
+    case 256: stats_tiled_bs<T, 256>(x, n, part, g, st); return true;
+    default: return false;
+    }
+}
+
 void rate_stats_launch(const void *x, uint64_t n, int w, int bs, uint8_t *ws, RateStats *d_stats,
                        hipStream_t st)
 {
     const uint64_t nchunks = (n + RATE_CHUNK - 1) / RATE_CHUNK;
     RateStats *part = reinterpret_cast<RateStats *>(ws);
     const unsigned g = (unsigned)(nchunks * RATE_WG_PER_CHUNK);
-    if (w == 4)
+    // power-of-two blocks of 32 to 256 values, a few lanes each, on the tiled
+    // kernels; one wave per block otherwise
+    const bool tiled = w == 4 ? stats_tiled<float>(bs, x, n, part, g, st) : stats_tiled<double>(bs, x, n, part, g, st);
+    if (!tiled && w == 4)
         hipLaunchKernelGGL(k_rate_stats<float>, dim3(g), dim3(256), 0, st,
                            static_cast<const float *>(x), n, bs, (uint64_t)RATE_CHUNK,
                            RATE_WG_PER_CHUNK, part);
-    else
+    else if (!tiled)
         hipLaunchKernelGGL(k_rate_stats<double>, dim3(g), dim3(256), 0, st,
                            static_cast<const double *>(x), n, bs, (uint64_t)RATE_CHUNK,
                            RATE_WG_PER_CHUNK, part);
-    hipLaunchKernelGGL(k_rate_stats_fold, dim3((unsigned)nchunks), dim3(256), 0, st, part,
-                       RATE_WG_PER_CHUNK, d_stats);
+    hipLaunchKernelGGL(k_rate_stats_fold, dim3((unsigned)nchunks), dim3(256), 0, st, part, d_stats);
 }
 
 void rate_ladder_launch(const RateStats *d_stats, int nchunks, int K, float *d_ebs, hipStream_t st)
@@ -733,12 +1060,42 @@ void rate_inputs_launch(const RateStats *d_stats, int nchunks, const float *d_eb
 
 uint64_t octave_workspace_bytes() { return 256; }
 
+template <typename T, int BS>
+static void octave_tiled_bs(const void *x, uint64_t n, int reqexp, unsigned long long *acc, bool edges, int nocts,
+                            hipStream_t st)
+{
+    const uint64_t steps = (n + TiledRate<T, BS>::STEP - 1) / TiledRate<T, BS>::STEP;
+    // 1024 workgroups (four per CU) share the field: each ends with a flush of
+    // its bins, which twice as many would double
+    const uint64_t g = (steps + 3) / 4 < 1024 ? (steps + 3) / 4 : 1024;
+    const dim3 grid((unsigned)(g ? g : 1)), blk(256);
+    const T *p = static_cast<const T *>(x);
+    if (nocts == 2) hipLaunchKernelGGL((k_rate_octave_tiled<T, BS, true, 2>), grid, blk, 0, st, p, n, reqexp, acc);
+    else if (edges) hipLaunchKernelGGL((k_rate_octave_tiled<T, BS, true, 1>), grid, blk, 0, st, p, n, reqexp, acc);
+    else hipLaunchKernelGGL((k_rate_octave_tiled<T, BS, false, 1>), grid, blk, 0, st, p, n, reqexp, acc);
+}
+template <typename T>
+static bool octave_tiled(int bs, const void *x, uint64_t n, int reqexp, unsigned long long *acc, bool edges,
+                         int nocts, hipStream_t st)
+{
+    switch (bs) {
+    case 32: octave_tiled_bs<T, 32>(x, n, reqexp, acc, edges, nocts, st); return true;
+    case 64: octave_tiled_bs<T, 64>(x, n, reqexp, acc, edges, nocts, st); return true;
+    case 128: octave_tiled_bs<T, 128>(x, n, reqexp, acc, edges, nocts, st); return true;
+    case 256: octave_tiled_bs<T, 256>(x, n, reqexp, acc, edges, nocts, st); return true;
+    default: return false;
+    }
+}
+
 void rate_octave_launch(const void *x, uint64_t n, int w, int bs, int reqexp, uint8_t *ws,
                         unsigned long long *d_acc, hipStream_t st, bool edges, int nocts)
 {
     (void)ws;
     const int width = nocts * OCT_ACC + (edges || nocts == 2 ? 4 : 0);
     hipLaunchKernelGGL(k_fill_u64, dim3((width + 255) / 256), dim3(256), 0, st, d_acc, width);
+    if (w == 4 ? octave_tiled<float>(bs, x, n, reqexp, d_acc, edges, nocts, st)
+               : octave_tiled<double>(bs, x, n, reqexp, d_acc, edges, nocts, st))
+        return;
     const uint64_t nb = (n + bs - 1) / bs;
     uint64_t g = (nb + 4 * PF - 1) / (4 * PF);
     if (g < 1) g = 1;

@@ -124,6 +124,33 @@ def test_rate_octave_span_is_exact(dtype, device):
             assert sizes[-1] == len(O.compress(x, float(ebs[-1]), 128))
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("bs", [16, 32, 64, 100, 128, 256])
+def test_rate_octave_block_sizes(bs, dtype, device):
+    """Every block size on either side of the tiled passes' range: sizes of
+    the octave pair and its edges equal the oracle's streams, at array ends
+    inside a lane, with constant blocks, NaNs, bounds small enough for the
+    reqLength to clamp, and an input at its type's alignment only."""
+    import torch
+    r = np.random.default_rng(bs)
+    for n in (1, 1023, 4 * 1024 + 5, 40_009):
+        t = np.arange(n)
+        x = (np.sin(t * 0.01) * 3 + r.standard_normal(n) * 1e-3).astype(dtype)
+        x[n // 3:n // 2] = 0.75
+        if n > 5000:
+            x[3 * bs] = np.nan        # a block's first value
+            x[7 * bs + 5] = np.nan    # another block's sixth
+        room = torch.zeros(n + 1, dtype=torch.float32 if dtype == np.float32 else torch.float64, device=device)
+        room[1:] = torch.from_numpy(x).to(device)
+        for e in (-2, -9, -40):
+            say("octave", dtype.__name__, bs, n, e)
+            sizes, ebs, up, dn = Z.rate_octave_span(room[1:], e, 2, bs)
+            for k in (0, 300, 511, 512, 700, 1023):
+                assert sizes[k] == len(O.compress(x, float(ebs[k]), bs)), (e, k)
+            for size, eb in (up, dn):
+                assert size == len(O.compress(x, float(eb), bs)), (e, float(eb))
+
+
 def test_rate_stats_match_numpy(device):
     import torch
     r = np.random.default_rng(15)
