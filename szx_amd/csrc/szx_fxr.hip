@@ -932,6 +932,20 @@ __global__ __launch_bounds__(256) void k_rate_inputs(const RateStats *st, int nc
     }
 }
 
+// One wave per bound.
+__global__ __launch_bounds__(64) void k_rate_predict(const float *y, int nchunks, uint64_t n, double head_bits,
+                                                     double *pred)
+{
+    const int k = blockIdx.x;
+    double bits = 0;
+    for (int c = threadIdx.x; c < nchunks; c += 64) {
+        const uint64_t c0 = (uint64_t)c * RATE_CHUNK, vals = n - c0 < RATE_CHUNK ? n - c0 : RATE_CHUNK;
+        bits += exp2((double)y[(uint64_t)k * nchunks + c]) * (double)vals;
+    }
+    for (int m = 1; m < 64; m <<= 1) bits += __shfl_xor(bits, m, 64);
+    if (threadIdx.x == 0) pred[k] = (head_bits + bits) / (double)n;
+}
+
 // ---------------------------------------------------------------------------
 // host launchers
 // ---------------------------------------------------------------------------
@@ -1056,6 +1070,12 @@ void rate_inputs_launch(const RateStats *d_stats, int nchunks, const float *d_eb
 {
     hipLaunchKernelGGL(k_rate_inputs, dim3((unsigned)nchunks), dim3(256), 0, st, d_stats, nchunks,
                        d_ebs, K, d_X);
+}
+
+void rate_predict_launch(const float *d_y, int nchunks, int K, uint64_t n, double head_bits, double *d_pred,
+                         hipStream_t st)
+{
+    hipLaunchKernelGGL(k_rate_predict, dim3((unsigned)K), dim3(64), 0, st, d_y, nchunks, n, head_bits, d_pred);
 }
 
 uint64_t octave_workspace_bytes() { return 256; }

@@ -62,5 +62,9 @@ void rate_ladder_launch(const RateStats *d_stats, int nchunks, int K, float *d_e
 // X[(k * nchunks + c)][RATE_INPUTS] for K bounds at d_ebs.
 void rate_inputs_launch(const RateStats *d_stats, int nchunks, const float *d_ebs, int K, float *d_X,
                         hipStream_t st);
+// d_pred[k] = the field's predicted bits per value at bound k: 2^y[k * nchunks
+// + c] bits per value of chunk c, plus head_bits.
+void rate_predict_launch(const float *d_y, int nchunks, int K, uint64_t n, double head_bits, double *d_pred,
+                         hipStream_t st);
 
 }  // namespace szxamd

@@ -70,11 +70,23 @@ struct MlpShared {
 
 __device__ inline void load_weights(const float *P, MlpShared &s)
 {
-    for (int e = threadIdx.x; e < H * IN_PAD; e += blockDim.x) {
+    // unrolled so that a thread's loads are in flight together: one after the
+    // other, their round trips were most of a small forward pass (5120
+    // samples: 21 -> 17 us)
+    static_assert(H * IN_PAD % 256 == 0 && H * H % 256 == 0, "256 threads, whole rounds");
+#pragma unroll
+    for (int e = threadIdx.x; e < H * IN_PAD; e += 256) {
         const int j = e / IN_PAD, k = e % IN_PAD;
         s.w1[j][k] = k < MLP_IN ? to_bf16(P[MLP_W1 + j * MLP_IN + k]) : (short)0;
     }
-    for (int e = threadIdx.x; e < H * H; e += blockDim.x) s.w2[e / H][e % H] = to_bf16(P[MLP_W2 + e]);
+    float w2[H * H / 256];
+#pragma unroll
+    for (int i = 0; i < H * H / 256; i++) w2[i] = P[MLP_W2 + threadIdx.x + 256 * i];
+#pragma unroll
+    for (int i = 0; i < H * H / 256; i++) {
+        const int e = threadIdx.x + 256 * i;
+        s.w2[e / H][e % H] = to_bf16(w2[i]);
+    }
 }
 
 // Forward pass of one 16-sample tile for the wave; rows past `rows` are zero.

@@ -42,7 +42,7 @@ constexpr int BISECT_MAX = 60;
 constexpr int STREAM_HEADER = 13;   // szx_float.cc:1091-1098
 
 struct RateLayout {
-    uint64_t comp, oct, acc, stats_ws, stats, ebs, X, y, range, minmax, bytes;
+    uint64_t comp, oct, acc, stats_ws, stats, ebs, X, y, pred, range, minmax, bytes;
     uint64_t nchunks;
 };
 
@@ -62,6 +62,7 @@ RateLayout rate_layout(uint64_t n, int w, int bs)
     L.ebs = off;      off += al(K_MAX * 4);
     L.X = off;        off += al((uint64_t)K_MAX * L.nchunks * RATE_INPUTS * 4);
     L.y = off;        off += al((uint64_t)K_MAX * L.nchunks * 4);
+    L.pred = off;     off += al(K_MAX * 8);
     L.range = off;    off += al(range_workspace_bytes());
     L.minmax = off;   off += 256;
     L.bytes = off;
@@ -315,10 +316,15 @@ int fixed_rate_solve(const void *d_in, uint64_t n, int w, int bs, float target, 
         rate_inputs_launch(d_stats, nch, d_ebs, K, (float *)(d_ws + S.L.X), st);
         mlp_forward_launch(d_params, (const float *)(d_ws + S.L.X), (uint64_t)K * nch,
                            (float *)(d_ws + S.L.y), st);
-        std::vector<float> ladder(K), y((size_t)K * nch);
+        // predicted field rate along the ladder (bits of the records, medians
+        // and bitmap per chunk, plus the 13-byte header)
+        rate_predict_launch((const float *)(d_ws + S.L.y), nch, K, n, 8.0 * STREAM_HEADER,
+                            (double *)(d_ws + S.L.pred), st);
+        std::vector<float> ladder(K);
+        std::vector<double> pred(K);
         if (!S.ok(hipMemcpyAsync(ladder.data(), d_ebs, 4 * (size_t)K, hipMemcpyDeviceToHost, st),
                   "D2H ladder") ||
-            !S.ok(hipMemcpyAsync(y.data(), d_ws + S.L.y, y.size() * 4, hipMemcpyDeviceToHost, st),
+            !S.ok(hipMemcpyAsync(pred.data(), d_ws + S.L.pred, 8 * (size_t)K, hipMemcpyDeviceToHost, st),
                   "D2H predictions") ||
             !S.ok(hipStreamSynchronize(st), "rate model")) {
             *err = S.err;
@@ -326,18 +332,6 @@ int fixed_rate_solve(const void *d_in, uint64_t n, int w, int bs, float target, 
         }
         feature_passes = 1;
         const double range = (double)ladder[0];
-        // predicted field rate along the ladder (bits of the records,
-        // medians and bitmap per chunk, plus the 13-byte header)
-        std::vector<double> pred(K);
-        for (int k = 0; k < K; k++) {
-            double bits = 8.0 * STREAM_HEADER;
-            for (int c = 0; c < nch; c++) {
-                const uint64_t vals = n - (uint64_t)c * RATE_CHUNK < RATE_CHUNK ? n - (uint64_t)c * RATE_CHUNK
-                                                                                : RATE_CHUNK;
-                bits += exp2((double)y[(size_t)k * nch + c]) * (double)vals;
-            }
-            pred[k] = bits / (double)n;
-        }
         // first rung whose predicted rate reaches the target; interpolate in
         // log2(rate) between it and the rung before
         double lg_eb = log2((double)ladder[K - 1]);

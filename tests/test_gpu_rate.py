@@ -137,18 +137,22 @@ def test_rate_octave_block_sizes(bs, dtype, device):
         t = np.arange(n)
         x = (np.sin(t * 0.01) * 3 + r.standard_normal(n) * 1e-3).astype(dtype)
         x[n // 3:n // 2] = 0.75
+        # blocks with a NaN follow the codec on the GPU: the sign of a NaN minus
+        # a median is not the CPU's, and it is part of the record
+        size_of = lambda y, eb: len(O.compress(y, eb, bs))
         if n > 5000:
             x[3 * bs] = np.nan        # a block's first value
             x[7 * bs + 5] = np.nan    # another block's sixth
+            size_of = lambda y, eb: len(Z.compress_blocked(y, eb, bs))
         room = torch.zeros(n + 1, dtype=torch.float32 if dtype == np.float32 else torch.float64, device=device)
         room[1:] = torch.from_numpy(x).to(device)
         for e in (-2, -9, -40):
             say("octave", dtype.__name__, bs, n, e)
             sizes, ebs, up, dn = Z.rate_octave_span(room[1:], e, 2, bs)
             for k in (0, 300, 511, 512, 700, 1023):
-                assert sizes[k] == len(O.compress(x, float(ebs[k]), bs)), (e, k)
+                assert sizes[k] == size_of(x, float(ebs[k])), (e, k)
             for size, eb in (up, dn):
-                assert size == len(O.compress(x, float(eb), bs)), (e, float(eb))
+                assert size == size_of(x, float(eb)), (e, float(eb))
 
 
 def test_rate_stats_match_numpy(device):
