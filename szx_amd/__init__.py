@@ -15,6 +15,7 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import weakref
 
 import numpy as np
 
@@ -299,6 +300,15 @@ def _take(ptr, nbytes: int) -> bytes:
     return out
 
 
+def _take_array(ptr, n: int, dtype) -> np.ndarray:
+    """The library's malloc'd buffer itself as a (writable) array, freed with
+    its last view: copying a decoded field out of it twice took longer than
+    decoding it on the GPU and bringing it back."""
+    buf = (C.c_char * (n * np.dtype(dtype).itemsize)).from_address(ptr)
+    weakref.finalize(buf, _libc.free, C.c_void_p(ptr)).atexit = False
+    return np.frombuffer(buf, dtype, n)
+
+
 # ---------------------------------------------------------------------------
 # drop-in host API (szx.h)
 # ---------------------------------------------------------------------------
@@ -327,11 +337,11 @@ def SZx_fast_decompress(fastMode: int, dtype, stream: bytes, shape) -> np.ndarra
     """szx.h:80: decode into an array of `shape`."""
     dtype = np.dtype(dtype)
     n = int(np.prod(shape))
-    buf = C.create_string_buffer(bytes(stream), len(stream))
+    buf = bytes(stream)   # no copy of a bytes object; read in place
     p = lib().SZx_fast_decompress(fastMode, _dtype_code(dtype), buf, len(stream), *_dims(shape))
     if not p:
         raise SZxError(last_error())
-    return np.frombuffer(_take(p, n * dtype.itemsize), dtype).reshape(shape).copy()
+    return _take_array(p, n, dtype).reshape(shape)
 
 
 def compress_blocked(data: np.ndarray, absErrBound: float, blockSize: int = 128) -> bytes:
@@ -349,12 +359,12 @@ def compress_blocked(data: np.ndarray, absErrBound: float, blockSize: int = 128)
 def decompress_blocked(stream: bytes, n: int, dtype) -> np.ndarray:
     """szx.h:98 SZx_fast_decompress_args_unpredictable_blocked (length-free)."""
     dtype = np.dtype(dtype)
-    buf = C.create_string_buffer(bytes(stream), len(stream))
+    buf = bytes(stream)   # no copy of a bytes object; read in place
     out = C.c_void_p(0)
     lib().SZx_fast_decompress_args_unpredictable_blocked(C.byref(out), _dtype_code(dtype), n, buf)
     if not out.value:
         raise SZxError(last_error())
-    return np.frombuffer(_take(out.value, n * dtype.itemsize), dtype).copy()
+    return _take_array(out.value, n, dtype)
 
 
 def cuszx_compress(data: np.ndarray, absErrBound: float, blockSize: int = 128) -> bytes:
@@ -372,12 +382,12 @@ def cuszx_compress(data: np.ndarray, absErrBound: float, blockSize: int = 128) -
 def cuszx_decompress(stream: bytes, n: int) -> np.ndarray:
     """cuszx_entry.h:11 cuSZx_fast_decompress_args_unpredictable_blocked_float:
     read a stream the reference's CUDA codec wrote (fp32, length-free)."""
-    buf = C.create_string_buffer(bytes(stream), len(stream))
+    buf = bytes(stream)   # no copy of a bytes object; read in place
     out = C.c_void_p(0)
     lib().cuSZx_fast_decompress_args_unpredictable_blocked_float(C.byref(out), n, buf)
     if not out.value:
         raise SZxError(last_error())
-    return np.frombuffer(_take(out.value, n * 4), np.float32).copy()
+    return _take_array(out.value, n, np.float32)
 
 
 def SZx_computeValueRange(data: np.ndarray):

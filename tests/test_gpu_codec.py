@@ -456,3 +456,24 @@ def test_decode_tile_edges(bs, dtype, device):
                     dec(buf[at:], size, Z.DECODE_EXACT, index=index)
                     assert dec.check() == 0
                     assert bits_equal(dec.out.cpu().numpy(), O.decompress(s, n, dtype, ref_quirk=False))
+
+
+def test_host_results_are_the_callers(device):
+    """Arrays returned by the host calls are writable, keep their values over
+    later calls and outlive everything but their last view."""
+    import gc
+    xs = [np.sin(np.arange(n) * 0.01 + n).astype(np.float32) for n in (1, 1000, 1_500_000, 1_500_000)]
+    streams = [Z.compress_blocked(x, 1e-3, 128) for x in xs]
+    want = [O.decompress(s, x.size, np.float32) for s, x in zip(streams, xs)]
+    got = [Z.SZx_fast_decompress(Z.SZx_WITH_BLOCK_FAST_CMPR, np.float32, s, (1, x.size)) for s, x in zip(streams, xs)]
+    got += [Z.decompress_blocked(s, x.size, np.float32) for s, x in zip(streams, xs)]
+    assert all(g.flags.writeable for g in got)
+    got[2][:] = 5.0
+    for i, g in enumerate(got):
+        assert i == 2 or bits_equal(g.ravel(), want[i % 4]), i
+    tails = [g.ravel()[-1:] for g in got]
+    del got, g
+    gc.collect()
+    for _ in range(3):
+        Z.decompress_blocked(streams[3], xs[3].size, np.float32)
+    assert all(t[0] == (5.0 if i == 2 else want[i % 4][-1]) for i, t in enumerate(tails))
