@@ -32,6 +32,7 @@
 #include "szx_common.hpp"
 #include "szx_batch.hpp"
 #include "szx_internal.hpp"
+#include "szx_lane.hpp"
 #include "szx_wave.hpp"
 
 namespace szxamd {
@@ -106,7 +107,7 @@ __device__ inline uint32_t wave0_exclusive_scan(uint32_t *a, int lane)
 }
 
 // What a lane keeps of one slab between encoding and staging.
-//   mid   = per value the word with its mid bytes as the low bytes
+//   mid   = per value its mid bytes as the low bytes of a word, zero above
 //   meta  = mid-byte offset in the record (12) | rb (4) << 12 |
 //           non-constant << 16 | reqLength (7) << 17
 //   code  = the lane's 2-bit lead codes (LV/4 bytes) | lead bytes of the
@@ -296,7 +297,7 @@ __device__ __forceinline__ void encode_slab(const T (&v)[LV], uint64_t e0, uint6
                     tot8 += mp;
                 }
             } else {
-                st.mid[k] = mid;
+                st.mid[k] = mid & ~(m8 >= 64 ? 0ull : ~0ull << m8);
                 mb |= (m8 >> 3) << (4 * k);
                 tot8 += m8;
             }
@@ -480,7 +481,6 @@ template <typename T, int BS, int LV, int SLABS, bool LDS>
 __device__ __forceinline__ void stage_slab(const SlabState<T, LV> &st, int u, const TileMeta<T, BS, LV, SLABS> &M,
                                            uint8_t *s_stage)
 {
-    using U = typename Word<T>::U;
     constexpr int SEG = BS / LV;
     constexpr int NLB = LV / 4;           // lead-code bytes per lane
     constexpr int BPS = 256 * LV / BS;    // blocks per slab
@@ -503,30 +503,19 @@ __device__ __forceinline__ void stage_slab(const SlabState<T, LV> &st, int u, co
     for (int b = 0; b < NLB; b++)
         if ((uint32_t)(lseg * NLB + b) < nlead)
             s_stage[base + 5 + lseg * NLB + b] = (uint8_t)(st.code >> (8 * b));
-    if constexpr (LDS && sizeof(U) == 4) {
-        // Mid bytes OR-ed into the zeroed stage as aligned 8-byte words: a
-        // run's bytes start at bit offset o8 of the stage.  LDS atomics are the expensive part here
-        // (measured: two unconditional ORs per value ran 0.28 ms against 0.22
-        // ms for predicated ones at 512^3), so the lanes with nothing to add
-        // sit out.  OR is idempotent and every stage byte has one writer, so
-        // the words a run shares with its neighbours need no care.
+    if constexpr (LDS) {
+        // Mid bytes OR-ed into the zeroed stage as aligned 8-byte words, fp32
+        // two neighbouring values at a time, fp64 value by value (a byte store
+        // per mid byte cost the fp64 compressor 13 %: 8192^2, bs 64, REL 1e-6,
+        // whole call 0.270 -> 0.248 ms).
         static_assert(TileShape<T, BS, LV, SLABS>::STAGE_DW % 2 == 0, "the stage is whole 8-byte words");
         uint64_t *sq = reinterpret_cast<uint64_t *>(s_stage);
         uint32_t o8 = 8u * (base + 5 + nlead + (meta & 0xFFFu));
 #pragma unroll
-        for (int r = 0; r < LV / 2; r++) {
-            // two neighbouring values as one run of mp <= 64 bits (zero
-            // above), OR-ed into the one or two 8-byte stage words it touches
-            const uint32_t mp = (st.mb >> (8 * r)) & 0xFFu;
-            if (mp) {
-                const uint64_t run = st.mid[r];
-                const uint32_t s = o8 & 63u;
-                uint64_t *pq = sq + (o8 >> 6);
-                __hip_atomic_fetch_or(pq, run << s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                // bits past the first word (only when s > 0): the run's top s
-                if (s + mp > 64u)
-                    __hip_atomic_fetch_or(pq + 1, run >> (64u - s), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            }
+        for (int r = 0; r < SlabState<T, LV>::NM; r++) {
+            const uint32_t mp = SlabState<T, LV>::PAIRS ? (uint32_t)(st.mb >> (8 * r)) & 0xFFu
+                                                        : ((uint32_t)(st.mb >> (4 * r)) & 0xFu) << 3;
+            stage_run(sq, o8, st.mid[r], mp);
             o8 += mp;
         }
     } else {
@@ -768,7 +757,7 @@ __device__ __forceinline__ void compress_tile(const CompressParams &p, uint64_t 
     } else if (p.eb_dev) {
         eb = *p.eb_dev;
     }
-    if constexpr (sizeof(T) == 4) {   // the fp32 stage is OR-ed into (stage_slab)
+    {   // the stage is OR-ed into (stage_slab)
         constexpr int N4 = TileShape<T, BS, LV, SLABS>::STAGE_DW / 4;
         for (int i = threadIdx.x; i < N4; i += 256) reinterpret_cast<uint4 *>(lds.stage.w)[i] = make_uint4(0, 0, 0, 0);
     }
