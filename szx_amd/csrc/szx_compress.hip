@@ -1169,22 +1169,20 @@ CompressLayout compress_layout(uint64_t n, int w, int bs)
     // The look-back words are sized for one index tile per compressor tile,
     // the smallest tile any launch shape uses (the batched launch shares this
     // layout).
-    uint64_t off = 0;
-    L.ws_tiles = off;   off += L.nidx * sizeof(unsigned long long);
-    L.ws_chunks = off;  off += ceil_div(L.nidx, LB_CHUNK) * sizeof(ChunkState);
-    L.ws_cacc = off;    off += ceil_div(L.nidx, LB_CHUNK) * sizeof(unsigned long long);
+    uint64_t off = 0, lb = L.nidx;
+    if (!bs_tiled(bs)) {
+        L.ntiles = generic_tiles(L.nb, w, bs);
+        if (L.ntiles > lb) lb = L.ntiles;   // the smallest blocks' tiles hold fewer values
+    }
+    L.ws_tiles = off;   off += lb * sizeof(unsigned long long);
+    L.ws_chunks = off;  off += ceil_div(lb, LB_CHUNK) * sizeof(ChunkState);
+    L.ws_cacc = off;    off += ceil_div(lb, LB_CHUNK) * sizeof(unsigned long long);
     L.ws_misc = off;    off += 64 * sizeof(uint64_t);   // totals at +128 B, eb at +256 B, error at +384 B
     off = (off + 255) & ~(uint64_t)255;   // the range partials are read as 16-byte vectors
     L.ws_parts = off;   off += 2 * kRangeParts * sizeof(double);
     L.ws_bitmap = off;  off += (L.nbit + 15) & ~(uint64_t)15;
     L.ws_cmed = off;    off += (4 * L.nb + 15) & ~(uint64_t)15;
     L.ws_osz = off;     off += (2 * L.nb + 15) & ~(uint64_t)15;
-    if (!bs_tiled(bs)) {
-        off = (off + 255) & ~(uint64_t)255;
-        L.ws_gsize = off;   off += (4 * L.nb + 255) & ~(uint64_t)255;
-        L.ws_gparts = off;  off += 16 * generic_parts(L.nb);
-        L.ws_gidx = off;    off += 8 * index_words(n, w, bs);
-    }
     L.ws_bytes = off;
     return L;
 }
@@ -1280,8 +1278,8 @@ int compress_launch(const void *d_in, uint64_t n, int w, int rel_mode, float abs
     const uint64_t zero_words = (L.ws_misc + 64 * sizeof(uint64_t)) / 8;
     unsigned long long *zero = reinterpret_cast<unsigned long long *>(d_ws);
     float *eb_dev = nullptr;        // REL: the bound, computed on the device
-    const void *rparts = nullptr;   // REL, tiled: the range partials k_compress folds
-    if (rel_mode && bs_tiled(bs)) {
+    const void *rparts = nullptr;   // REL: the range partials the compressor folds
+    if (rel_mode) {
         // one launch for the range partials and the clear; every compressor
         // workgroup folds the partials into the bound itself (fp64: the fold
         // of 256 pairs of doubles costs its kernel 3-4 %, the two launches
@@ -1293,29 +1291,10 @@ int compress_launch(const void *d_in, uint64_t n, int w, int rel_mode, float abs
         hipLaunchKernelGGL(k_zero_u64, dim3((unsigned)((zero_words + 255) / 256 < 1024 ? (zero_words + 255) / 256 : 1024)),
                            dim3(256), 0, st, zero, zero_words);
     }
-    if (rel_mode && !rparts) {
-        eb_dev = reinterpret_cast<float *>(misc + 32);
-        if (w == 4) {
-            float *part = reinterpret_cast<float *>(d_ws + L.ws_parts);
-            hipLaunchKernelGGL((k_range_partial<float, 256>), dim3(kRangeParts), dim3(256), 0, st,
-                               static_cast<const float *>(d_in), n, part, nullptr, 0);
-            hipLaunchKernelGGL(k_range_final<float>, dim3(1), dim3(256), 0, st,
-                               static_cast<const float *>(d_in), part, kRangeParts, rel, eb_dev,
-                               (float *)nullptr);
-        } else {
-            double *part = reinterpret_cast<double *>(d_ws + L.ws_parts);
-            hipLaunchKernelGGL((k_range_partial<double, 256>), dim3(kRangeParts), dim3(256), 0, st,
-                               static_cast<const double *>(d_in), n, part, nullptr, 0);
-            hipLaunchKernelGGL(k_range_final<double>, dim3(1), dim3(256), 0, st,
-                               static_cast<const double *>(d_in), part, kRangeParts, rel, eb_dev,
-                               (double *)nullptr);
-        }
-    }
     CompressParams p{};
     p.x = d_in;
     p.n = n;
     p.eb = abs_eb;
-    p.eb_dev = rparts ? nullptr : eb_dev;
     p.rparts = rparts;
     p.rel = rel;
     p.eb_out = rparts ? eb_dev : nullptr;
@@ -1340,22 +1319,8 @@ int compress_launch(const void *d_in, uint64_t n, int w, int rel_mode, float abs
     if (bs_tiled(bs)) {
         rc = w == 4 ? dispatch_bs<float>(bs, p, L.ntiles, st) : dispatch_bs<double>(bs, p, L.ntiles, st);
     } else if (bs_valid(bs)) {
-        GenericCompress g{};
-        g.x = d_in;
-        g.n = n;
-        g.nb = L.nb;
-        g.bs = bs;
-        g.eb = abs_eb;
-        g.eb_dev = eb_dev;
-        g.payload = p.payload;
-        g.bitmap = p.bitmap;
-        g.cmed = p.cmed;
-        g.totals = p.totals;
-        g.size = reinterpret_cast<uint32_t *>(d_ws + L.ws_gsize);
-        g.idx = d_index ? d_index : reinterpret_cast<uint64_t *>(d_ws + L.ws_gidx);
-        g.parts = reinterpret_cast<uint64_t *>(d_ws + L.ws_gparts);
-        g.nparts = generic_parts(L.nb);
-        generic_compress_launch(g, w, st);
+        p.bidx = nullptr;   // the index is per block
+        generic_compress_launch(p, w, bs, st);
     } else {
         rc = -1;
     }

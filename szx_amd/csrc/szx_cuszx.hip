@@ -698,9 +698,8 @@ void cuszx_compress_launch(const float *d_in, uint64_t n, float eb, int bs, uint
     if (L.nb) {
         const unsigned grid = (unsigned)ceil_div(L.nb, (uint64_t)(256 / p.S));
         czw_pass(p, false, grid, st);
-        GenericCompress g{};
+        GenericScan g{};
         g.nb = L.nb;
-        g.bs = bs;
         g.size = p.size;
         g.idx = reinterpret_cast<uint64_t *>(d_ws + L.o_idx);
         g.parts = reinterpret_cast<uint64_t *>(d_ws + L.o_parts);

@@ -5,268 +5,364 @@
 // aligned group of lanes and need a power-of-two block size of at least 4.
 // The reference's blocked API takes any block size that fits its one-byte
 // header field (szx_float.cc:1095), so every other size 1..255 runs here.
-// A block is a segment of S lanes (S = the smallest power of two with
-// 4 S >= bs), each lane holding 4 consecutive values; segment shuffles give
-// the block statistics, the byte offsets and the cross-lane carries of the
+// A block is a segment of S lanes (S a power of two), each lane holding LV
+// consecutive values: 16 fp32 / 8 fp64 (fewer for the smallest blocks);
+// segment steps give the block statistics, the byte offsets and the cross-lane
+// carries of the
 // reference's per-block loops (szx_float.cc:314-371 and 49-252 for
 // compression, szxd_float.cc:34-244 for decompression; fp64 in szx_double.cc
 // and szxd_double.cc).  The streams are the same bytes.
 //
-// Compression (two passes over the input, no per-block staging):
-//   k_gen_encode<T, false>  per block: statistics and record size (0 = constant)
-//   k_gen_part / k_gen_top / k_gen_apply
-//                           exclusive scan of (record bytes, constant blocks)
-//                           -> per-block pairs {record offset in the payload,
-//                           constant blocks before}, a closing pair {payload
-//                           bytes, constant blocks} and the totals
-//   k_gen_encode<T, true>   per block again: the record at its offset, or the
-//                           constant median at its rank
-//   k_gen_bitmap            one lane per bitmap byte
-// The per-block pairs are the record index for these block sizes; the
-// decoder's index builder (szx_index.hip) writes the same pairs.
+// Compression, after the range pass of a REL bound: k_gen_encode, one pass
+// over the input.  A wave takes a run of consecutive blocks, collects their
+// records in its own part of LDS, and the workgroup's size goes through the
+// compressor's decoupled look-back, as in the non-blocked codec.
+// The record index for these block sizes is per block: {record offset in the
+// payload, constant blocks before}, and a closing pair {payload bytes,
+// constant blocks}; the decoder's index builder (szx_index.hip) writes the
+// same pairs.
 //
 // Decompression: k_gen_decode, one segment per block, checks every record
 // against its pair and the next one.
+//
+// k_gen_part / k_gen_top / k_gen_apply (an exclusive scan of record sizes into
+// such pairs) and k_gen_bitmap serve the cuSZx writer.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
+#include "szx_batch.hpp"
 #include "szx_common.hpp"
 #include "szx_internal.hpp"
+#include "szx_lane.hpp"
+#include "szx_range.hpp"
+#include "szx_wave.hpp"
 
 namespace szxamd {
-
-// Lead bytes (capped at 3) a shifted word shares with the previous one
-// (szx_float.cc:96-101, szx_double.cc:80-85).
-template <typename U> __device__ inline int gen_lead(U xr)
-{
-    constexpr int W = sizeof(U);
-    if ((xr >> (8 * (W - 3))) == 0) return 3;
-    if ((xr >> (8 * (W - 2))) == 0) return 2;
-    if ((xr >> (8 * (W - 1))) == 0) return 1;
-    return 0;
-}
 
 __device__ inline bool gen_nonconst(const uint8_t *bitmap, uint64_t b)
 {
     return (bitmap[b >> 3] >> (7 - (b & 7))) & 1;
 }
 
-template <typename T> __device__ inline T gmin(T a, T b);
-template <typename T> __device__ inline T gmax(T a, T b);
-template <> __device__ inline float gmin<float>(float a, float b) { return __builtin_fminf(a, b); }
-template <> __device__ inline float gmax<float>(float a, float b) { return __builtin_fmaxf(a, b); }
-template <> __device__ inline double gmin<double>(double a, double b) { return __builtin_fmin(a, b); }
-template <> __device__ inline double gmax<double>(double a, double b) { return __builtin_fmax(a, b); }
+// Shape of a wave's run of blocks of up to S LV values.
+template <typename T, int LV, int S> struct GenShape {
+    static constexpr int W = Word<T>::W;
+    static constexpr int NLB = LV / 4;                 // lead-code bytes per lane
+    static constexpr int NR = LV * W / 8;              // runs of mid bytes per lane
+    static constexpr int STEPS = 4;
+    static constexpr int BPS = 64 / S;                 // blocks per step
+    static constexpr int NBLK = STEPS * BPS;           // blocks per run
+    static constexpr int STEP_MAX = BPS * (5 + S * LV / 4 + S * LV * W);
+    static constexpr int META = 8 * NBLK + 4;
+    // record bytes a wave collects before its place is known; above, it
+    // encodes its run again afterwards, step by step.  Four workgroups fit a
+    // CU's LDS (three with a lane per block).
+    static constexpr uint32_t CAP = (NBLK <= 128 ? 10208 - 48 - META : 9216) & ~15u;
+    static_assert(STEP_MAX + 16 <= (int)CAP, "a step fits the stage");
+    static_assert(NBLK % 8 == 0, "runs own whole bitmap bytes");
+};
+constexpr int GEN_WAVES = 4;
 
-// Payload bytes the blocks of one workgroup (256 / S of them) can span:
-// records of at most 5 + S + 4 S W bytes (bs <= 4 S), plus a 4-byte alignment
-// head; LDS words with 3 words of slack for the decoder's 8-byte windows.
-template <int S, int W> struct Span {
-    static constexpr int BYTES = (256 / S) * (5 + S + 4 * S * W) + 4;
-    static constexpr int WORDS = (BYTES + 3) / 4 + 3;
+// A wave's staged records, and per block {record bytes | constant blocks << 20}
+// before it in the run (one more word: the run's totals) and its median.
+template <typename T, int LV, int S> struct GenRun {
+    using G = GenShape<T, LV, S>;
+    __attribute__((aligned(16))) uint32_t stage[(G::CAP + 48) / 4];
+    uint32_t pack[G::NBLK + 1];
+    float med[G::NBLK];
 };
 
-// Values of one workgroup's blocks: at most 256 / S * bs <= 1024, staged
-// through LDS in aligned 16-byte chunks (the value array is 16-byte aligned),
-// plus one chunk of alignment slack at each end.
-template <typename T> struct Vals {
-    static constexpr int CE = 16 / (int)sizeof(T);   // values per chunk
-    static constexpr int N = 1024 + 2 * CE;
-};
+// One step, per lane: its mid bytes as runs of at most 64 bits (fp32: two
+// values each), lead codes and place.
+template <typename T, int LV, int S> struct GenStep {
+    using G = GenShape<T, LV, S>;
+    using U = typename Word<T>::U;
+    uint64_t run[G::NR];
+    uint32_t bits[G::NR];
+    uint32_t code, len, hbits;
+    int nlead;              // lead-code bytes of the block
+    bool nonconst, isconst;
+    float med;
+    uint32_t rec, mid, tot; // step-relative offsets of the record and the lane's mid bytes; bytes of the step
 
-// Load values [e0, e1) of x (n values) into xs, chunk-aligned: xs[i] holds
-// x[c0 * CE + i], c0 = e0 / CE.  Chunks past the array end go value by value.
-template <typename T>
-__device__ inline void stage_values(const T *x, uint64_t n, uint64_t e0, uint64_t e1, T *xs)
-{
-    constexpr int CE = Vals<T>::CE;
-    const uint64_t c0 = e0 / CE, c1 = (e1 + CE - 1) / CE;
-    for (uint64_t c = c0 + threadIdx.x; c < c1; c += 256) {
-        T *d = xs + (c - c0) * CE;
-        if ((c + 1) * CE <= n) {
-            *reinterpret_cast<uint4 *>(d) = *reinterpret_cast<const uint4 *>(x + c * CE);
-        } else {
-            for (int j = 0; j < CE; j++)
-                if (c * CE + j < n) d[j] = x[c * CE + j];
+    // v: the lane's values, nv of them inside the block; m: the block's values
+    // (0: no block)
+    __device__ void encode(T (&v)[LV], int nv, int m, int lane, int reqexp, float eb)
+    {
+        constexpr int W = G::W;
+        const int lseg = lane & (S - 1);
+        // block statistics (szx_float.cc:327-333, szx_double.cc:985-991): NaNs
+        // never win a comparison, except that a NaN first value makes both
+        // NaN.  Places past the lane's values repeat the one before, which
+        // changes neither.
+        T lo = nv > 0 ? v[0] : (T)__builtin_inf(), hi = nv > 0 ? v[0] : (T)-__builtin_inf();
+#pragma unroll
+        for (int k = 1; k < LV; k++) {
+            v[k] = k < nv ? v[k] : v[k - 1];
+            if (nv > 0) {
+                lo = __builtin_elementwise_min(lo, v[k]);
+                hi = __builtin_elementwise_max(hi, v[k]);
+            }
         }
+        lo = from_bits<T>(seg_reduce<S>(to_bits<T>(lo), [](U a, U b) {
+            return to_bits<T>(__builtin_elementwise_min(from_bits<T>(a), from_bits<T>(b)));
+        }));
+        hi = from_bits<T>(seg_reduce<S>(to_bits<T>(hi), [](U a, U b) {
+            return to_bits<T>(__builtin_elementwise_max(from_bits<T>(a), from_bits<T>(b)));
+        }));
+        const T first = from_bits<T>(seg_first<S>(to_bits<T>(v[0])));
+        if (first != first) lo = hi = first;
+        const T rad = (hi - lo) / (T)2;
+        const float rad_f = (float)rad;
+        med = (float)(lo + rad);
+        nonconst = m > 0 && !(rad <= (T)eb);
+        isconst = m > 0 && !nonconst;
+        int clamped;
+        len = (uint32_t)req_length<T>(rad_expo(rad_f), reqexp, clamped);
+        const int rb = ((int)len + 7) >> 3, shift = (-(int)len) & 7;
+        const float hmed = clamped ? 0.0f : med;
+        hbits = bswap32(f32_bits(hmed));
+        nlead = (m + 3) >> 2;
+        // fp32 encodes against the stored median; fp64 against the median
+        // before the clamp (szx_float.cc:60,90; szx_double.cc:38,78)
+        const T msub = W == 4 ? (T)hmed : (T)med;
+        U w[LV];
+#pragma unroll
+        for (int k = 0; k < LV; k++) w[k] = to_bits<T>(v[k] - msub) >> shift;
+        U prev = seg_prev<S>(w[LV - 1], lane);
+        const uint32_t rb8 = 8u * (uint32_t)rb, lo8 = 8u * W - rb8;
+        uint32_t c8[2] = {0, 0}, t8 = 0;
+#pragma unroll
+        for (int k = 0; k < LV; k++) {
+            const U xr = w[k] ^ prev;
+            const uint32_t top = W == 4 ? (uint32_t)xr : (uint32_t)((uint64_t)xr >> 32);
+            const int lz = __builtin_clzg(top, 32);
+            uint32_t ld8 = (uint32_t)((lz < 24 ? lz : 24) & ~7);
+            uint32_t m8 = __builtin_elementwise_sub_sat(rb8, ld8);
+            if (k >= nv) {
+                ld8 = 0;
+                m8 = 0;
+            }
+            c8[k >> 3] |= ld8 << (8 * ((k & 7) >> 2) + 6 - 2 * (k & 3));
+            if constexpr (W == 4) {
+                const uint32_t mid4 = m8 < 32 ? __builtin_amdgcn_ubfe((uint32_t)w[k], lo8, m8) : (uint32_t)w[k];
+                if ((k & 1) == 0) {
+                    run[k / 2] = mid4;
+                    bits[k / 2] = m8;
+                } else {
+                    run[k / 2] |= (uint64_t)mid4 << bits[k / 2];
+                    bits[k / 2] += m8;
+                }
+            } else {
+                run[k] = ((uint64_t)w[k] >> lo8) & ~(m8 >= 64 ? 0ull : ~0ull << m8);
+                bits[k] = m8;
+            }
+            t8 += m8;
+            prev = w[k];
+        }
+        code = (c8[0] >> 3) | ((c8[1] >> 3) << 16);
+        // one scan over the wave places every record and every lane's mid bytes
+        const uint32_t mids = nonconst ? t8 >> 3 : 0u;
+        const uint32_t own = mids + (nonconst && lseg == 0 ? 5u + (uint32_t)nlead : 0u);
+        const uint32_t inc = seg_scan_incl<64>(own, lane);
+        rec = seg_first<S>(inc - own);
+        mid = inc - mids;
+        tot = (uint32_t)__builtin_amdgcn_readlane((int)inc, 63);
+    }
+
+    // Stage the step's records at byte `at` of the wave's zeroed stage.
+    __device__ void stage(uint32_t *words, uint32_t at, int lane) const
+    {
+        if (!nonconst) return;
+        uint64_t *sq = reinterpret_cast<uint64_t *>(words);
+        const int lseg = lane & (S - 1);
+        if (lseg == 0)   // reqLength byte + big-endian median
+            stage_run(sq, 8u * (at + rec), (uint64_t)len | ((uint64_t)hbits << 8), 40);
+        const int have = nlead - lseg * G::NLB;   // the lane's lead-code bytes (szx_TypeManager.cc:198-273)
+        if (have > 0) {
+            const int nl = have < G::NLB ? have : G::NLB;
+            const uint32_t c = nl < 4 ? code & ((1u << (8 * nl)) - 1u) : code;
+            stage_run(sq, 8u * (at + rec + 5u + (uint32_t)(lseg * G::NLB)), c, 8 * nl);
+        }
+        uint32_t o8 = 8u * (at + mid);
+#pragma unroll
+        for (int r = 0; r < G::NR; r++) {
+            stage_run(sq, o8, run[r], bits[r]);
+            o8 += bits[r];
+        }
+    }
+};
+
+// The lane's values of block b (lane lseg of its segment): nv of them inside
+// the block, m values in the block.  x needs its type's alignment only.
+template <typename T, int LV>
+__device__ inline void gen_load(const CompressParams &p, int bs, uint64_t b, int lseg, T (&v)[LV], int &nv, int &m)
+{
+    typedef unsigned int u32x4_t __attribute__((ext_vector_type(4), aligned(4)));
+    constexpr int VC = 16 / (int)sizeof(T);
+    const T *x = static_cast<const T *>(p.x);
+    const uint64_t b0 = b * (uint64_t)bs, e0 = b0 + (uint64_t)(lseg * LV);
+    m = b < p.nb ? (p.n - b0 < (uint64_t)bs ? (int)(p.n - b0) : bs) : 0;
+    nv = m - lseg * LV;
+    nv = nv < 0 ? 0 : nv > LV ? LV : nv;
+    if (nv > 0 && e0 + LV <= p.n) {   // may read past the block, not past the array
+#pragma unroll
+        for (int k = 0; k < LV; k += VC) {
+            const u32x4_t q = *reinterpret_cast<const u32x4_t *>(x + e0 + k);
+            __builtin_memcpy(&v[k], &q, 16);
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < LV; k++) v[k] = k < nv ? x[e0 + k] : (T)0;
     }
 }
 
-// Store values [e0, e1) from xs (same layout) to x: chunks wholly inside the
-// range as 16-byte stores, the edge chunks (shared with the neighbouring
-// workgroups) value by value.
-template <typename T>
-__device__ inline void unstage_values(T *x, uint64_t e0, uint64_t e1, const T *xs)
+// One look-back tile of GEN_WAVES runs per workgroup.  256^3 fp32, bs 100, REL
+// 1e-3: a sizes pass of 34 us, a scan of 17, a records pass of 52 and a bitmap
+// pass of 5 -> 43 us.
+template <typename T, int LV, int S>
+__global__ __launch_bounds__(64 * GEN_WAVES) __attribute__((amdgpu_waves_per_eu(S == 1 ? 3 : 4))) void k_gen_encode(CompressParams p,
+                                                                                                       int bs)
 {
-    constexpr int CE = Vals<T>::CE;
-    const uint64_t c0 = e0 / CE, c1 = (e1 + CE - 1) / CE;
-    for (uint64_t c = c0 + threadIdx.x; c < c1; c += 256) {
-        const T *s = xs + (c - c0) * CE;
-        if (c * CE >= e0 && (c + 1) * CE <= e1) {
-            *reinterpret_cast<uint4 *>(x + c * CE) = *reinterpret_cast<const uint4 *>(s);
-        } else {
-            for (int j = 0; j < CE; j++) {
-                const uint64_t e = c * CE + j;
-                if (e >= e0 && e < e1) x[e] = s[j];
+    using G = GenShape<T, LV, S>;
+    __shared__ GenRun<T, LV, S> runs[GEN_WAVES];
+    __shared__ uint32_t s_tot[GEN_WAVES];
+    __shared__ unsigned long long s_ex[2];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, lseg = lane & (S - 1);
+    const uint64_t tile = blockIdx.x;
+    const uint64_t b0 = (tile * GEN_WAVES + wv) * (uint64_t)G::NBLK;   // the run's first block
+    GenRun<T, LV, S> &R = runs[wv];
+
+    T v[LV];
+    int nv, m;
+    float eb = p.eb;
+    if (p.rparts) {
+        RangeFold<T> rf;
+        rf.load(static_cast<const T *>(p.rparts), static_cast<const T *>(p.x));
+        gen_load<T, LV>(p, bs, b0 + lane / S, lseg, v, nv, m);
+        T lo, hi;
+        rf.minmax(lo, hi);
+        eb = RangeFold<T>::bound(lo, hi, p.rel);
+        if (tile == 0 && threadIdx.x == 0) *p.eb_out = eb;
+    } else {
+        gen_load<T, LV>(p, bs, b0 + lane / S, lseg, v, nv, m);
+    }
+    const int reqexp = req_expo(eb);
+    wave_clear(R.stage, G::CAP + 16, lane);
+    wave_lds_fence();
+    uint32_t bytes = 0, consts = 0;
+    bool fits = true;
+    GenStep<T, LV, S> st;
+#pragma unroll 1
+    for (int s = 0; s < G::STEPS; s++) {
+        T nx[LV];   // the next step's values load while this one is encoded
+        int nnv = 0, nm = 0;
+        if (s + 1 < G::STEPS) gen_load<T, LV>(p, bs, b0 + (uint64_t)((s + 1) * G::BPS + lane / S), lseg, nx, nnv, nm);
+        st.encode(v, nv, m, lane, reqexp, eb);
+        const uint64_t cb = __ballot(st.isconst && lseg == 0);
+        if (lseg == 0) {
+            const int lb = s * G::BPS + lane / S;
+            const uint32_t rank =
+                __builtin_amdgcn_mbcnt_hi((uint32_t)(cb >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)cb, 0u));
+            R.pack[lb] = (bytes + st.rec) | ((consts + rank) << 20);
+            R.med[lb] = st.med;
+        }
+        fits = fits && bytes + st.tot <= G::CAP;
+        if (fits) st.stage(R.stage, bytes, lane);
+        bytes += st.tot;
+        consts += (uint32_t)__builtin_popcountll(cb);
+        nv = nnv;
+        m = nm;
+#pragma unroll
+        for (int k = 0; k < LV; k++) v[k] = nx[k];
+    }
+    if (lane == 0) {
+        R.pack[G::NBLK] = bytes | (consts << 20);
+        s_tot[wv] = bytes | (consts << 20);
+    }
+    __syncthreads();
+    const LookbackRefs L{p.tiles, p.chunks, p.cacc, p.ntiles};
+    uint32_t tb = 0, tc = 0;
+    for (int k = 0; k < GEN_WAVES; k++) {
+        tb += s_tot[k] & 0xFFFFFu;
+        tc += s_tot[k] >> 20;
+    }
+    unsigned long long pend = 0;
+    LookbackPoll q{};
+    if (wv == 0) {
+        if (lane == 0) pend = lookback_publish(L, tile, tb, tc);
+        q = lookback_poll(L, tile);
+    }
+    // the bitmap needs no prefix: it covers the look-back's round trip
+#pragma unroll
+    for (int i = 0; i < G::NBLK; i += 64) {
+        const int lb = i + lane;
+        const bool in = lb < G::NBLK && b0 + lb < p.nb;
+        const bool rec = in && ((R.pack[lb] ^ R.pack[lb + 1]) & 0xFFFFFu) != 0;   // a record takes bytes
+        const uint64_t bm = __builtin_bswap64(__builtin_bitreverse64(__ballot(rec)));
+        const uint64_t gbyte = (b0 + i) / 8 + lane;
+        if (lane < (G::NBLK - i < 64 ? G::NBLK - i : 64) / 8 && gbyte < p.nbit)
+            p.bitmap[gbyte] = (uint8_t)(bm >> (8 * lane));
+    }
+    if (wv == 0) {
+        unsigned long long ebytes = 0, econst = 0;
+        if (!lookback_finish(L, tile, q, true, ebytes, econst)) {
+            ebytes = 0;   // every write stays in bounds; the call reports failure
+            econst = 0;
+            if (lane == 0) atomicExch(p.err, 1);
+        }
+        if (lane == 0) {
+            s_ex[0] = ebytes;
+            s_ex[1] = econst;
+            if (tile == p.ntiles - 1) {
+                p.totals[0] = ebytes + tb;
+                p.totals[1] = econst + tc;
+                if (p.index) {
+                    p.index[2 * p.nb] = ebytes + tb;
+                    p.index[2 * p.nb + 1] = econst + tc;
+                }
             }
         }
     }
-}
-
-// One block's encode state, per lane of its segment.
-template <typename T> struct GenBlock {
-    using U = typename Word<T>::U;
-    bool constant;
-    int m, len, rb;
-    float med_f, hmed;
-    bool val[4];
-    U sw[4];
-    int ld[4];
-    uint32_t lsum, incl, total;
-};
-
-// One block per segment of S lanes, 4 consecutive values per lane (S = the
-// smallest power of two with 4 S >= bs): statistics, reqLength, shifted
-// words, lead codes and the lane's byte offset in the block's mid bytes.
-// x = the block's values (staged in LDS).
-template <typename T, int S>
-__device__ inline void gen_block(const GenericCompress &g, uint64_t b, int l, const T *x, GenBlock<T> &k_)
-{
-    using U = typename Word<T>::U;
-    constexpr int W = Word<T>::W;
-    const float eb = g.eb_dev ? *g.eb_dev : g.eb;
-    const uint64_t rest = g.n - b * (uint64_t)g.bs;
-    const int m = rest < (uint64_t)g.bs ? (int)rest : g.bs;
-    k_.m = m;
-    T v[4];
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        k_.val[k] = 4 * l + k < m;
-        v[k] = k_.val[k] ? x[4 * l + k] : (T)0;
-    }
-    // block statistics (szx_float.cc:327-333, szx_double.cc:985-991): NaNs
-    // never win a comparison, so fmin / fmax over the values, except that a
-    // NaN first value makes both NaN.  Which of two zeros is kept cannot change
-    // the radius or the median.
-    T lo = v[0], hi = v[0];
-#pragma unroll
-    for (int k = 1; k < 4; k++)
-        if (k_.val[k]) {
-            lo = gmin(lo, v[k]);
-            hi = gmax(hi, v[k]);
-        }
-    if (4 * l >= m) {   // lanes past the block's end
-        lo = __builtin_huge_valf();
-        hi = -__builtin_huge_valf();
-    }
-#pragma unroll
-    for (int d = 1; d < S; d <<= 1) {
-        lo = gmin(lo, __shfl_xor(lo, d, S));
-        hi = gmax(hi, __shfl_xor(hi, d, S));
-    }
-    const T first = __shfl(v[0], 0, S);
-    if (first != first) {
-        lo = first;
-        hi = first;
-    }
-    const T rad = (hi - lo) / (T)2;
-    const T med = lo + rad;
-    k_.med_f = (float)med;
-    const float rad_f = (float)rad;
-    k_.constant = W == 4 ? (rad <= (T)eb) : ((double)rad <= (double)eb);
-    if (k_.constant) return;   // segment-uniform
-    int clamped;
-    k_.len = req_length<T>(rad_expo(rad_f), req_expo(eb), clamped);
-    k_.rb = (k_.len + 7) >> 3;
-    const int shift = (-k_.len) & 7;
-    k_.hmed = clamped ? 0.0f : k_.med_f;
-    // fp32 encodes against the stored median; fp64 against the median before
-    // the clamp (szx_float.cc:60,90; szx_double.cc:38,78)
-    const T msub = W == 4 ? (T)k_.hmed : (T)k_.med_f;
-#pragma unroll
-    for (int k = 0; k < 4; k++) k_.sw[k] = to_bits<T>(v[k] - msub) >> shift;
-    // the previous lane's last word (every lane before the last valid one is full)
-    U prev = __shfl_up(k_.sw[3], 1, S);
-    if (l == 0) prev = 0;
-    k_.lsum = 0;
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        k_.ld[k] = gen_lead<U>(k_.sw[k] ^ prev);
-        prev = k_.sw[k];
-        if (k_.val[k] && k_.ld[k] < k_.rb) k_.lsum += k_.rb - k_.ld[k];
-    }
-    k_.incl = seg_incl_sum<S>(k_.lsum, l);
-    k_.total = __shfl(k_.incl, S - 1, S);
-}
-
-// WRITE = false: record size per block (0 = constant).  WRITE = true: the
-// workgroup's records are built in LDS (they are contiguous in the payload)
-// and written out with aligned word stores; constant medians go to their rank.
-template <typename T, int S, bool WRITE>
-__global__ __launch_bounds__(256) void k_gen_encode(GenericCompress g)
-{
-    constexpr int W = Word<T>::W;
-    constexpr int BPW = 256 / S;
-    __shared__ __align__(16) T xs[Vals<T>::N];
-    const int l = threadIdx.x & (S - 1);
-    const uint64_t b0 = blockIdx.x * (uint64_t)BPW;
-    const uint64_t b = b0 + threadIdx.x / S;
-    const bool live = b < g.nb;   // whole segments
-    const uint64_t bend = b0 + BPW < g.nb ? b0 + BPW : g.nb;
-    const uint64_t e0 = b0 * (uint64_t)g.bs, e1 = bend * (uint64_t)g.bs < g.n ? bend * (uint64_t)g.bs : g.n;
-    stage_values<T>(static_cast<const T *>(g.x), g.n, e0, e1, xs);
     __syncthreads();
-    GenBlock<T> k_;
-    if (live) gen_block<T, S>(g, b, l, xs + (b * (uint64_t)g.bs - e0 / Vals<T>::CE * Vals<T>::CE), k_);
-    if (!WRITE) {
-        if (live && l == 0) g.size[b] = k_.constant ? 0u : 5u + (uint32_t)((k_.m + 3) >> 2) + k_.total;
-        return;
+    uint64_t ebytes = s_ex[0], econst = s_ex[1];
+    for (int k = 0; k < wv; k++) {
+        ebytes += s_tot[k] & 0xFFFFFu;
+        econst += s_tot[k] >> 20;
     }
-    __shared__ uint32_t stage[WRITE ? Span<S, W>::WORDS : 1];
-    uint8_t *lds = reinterpret_cast<uint8_t *>(stage);
-    const uint64_t P0 = g.idx[2 * b0], P1 = g.idx[2 * bend];
-    uint8_t *dst0 = g.payload + P0;
-    const uint32_t head = (uint32_t)((uintptr_t)dst0 & 3);
-    if (live && k_.constant && l == 0) g.cmed[g.idx[2 * b + 1]] = bswap32(f32_bits(k_.med_f));
-    if (live && !k_.constant) {
-        const int nlead = (k_.m + 3) >> 2;
-        uint8_t *rec = lds + head + (uint32_t)(g.idx[2 * b] - P0);
-        if (l == 0) {
-            const uint32_t hb = f32_bits(k_.hmed);
-            rec[0] = (uint8_t)k_.len;
-            rec[1] = (uint8_t)(hb >> 24);
-            rec[2] = (uint8_t)(hb >> 16);
-            rec[3] = (uint8_t)(hb >> 8);
-            rec[4] = (uint8_t)hb;
+    if (fits) {
+        wave_copy_out(p.payload + ebytes, R.stage, bytes, lane);
+    } else {
+        uint8_t *dst = p.payload + ebytes;
+#pragma unroll 1
+        for (int s = 0; s < G::STEPS; s++) {
+            gen_load<T, LV>(p, bs, b0 + (uint64_t)(s * G::BPS + lane / S), lseg, v, nv, m);
+            st.encode(v, nv, m, lane, reqexp, eb);
+            wave_lds_fence();
+            wave_clear(R.stage, st.tot + 16, lane);
+            wave_lds_fence();
+            st.stage(R.stage, 0, lane);
+            wave_lds_fence();
+            wave_copy_out(dst, R.stage, st.tot, lane);
+            dst += st.tot;
         }
-        if (4 * l < k_.m) {
-            uint32_t code = 0;
+    }
 #pragma unroll
-            for (int k = 0; k < 4; k++)
-                if (k_.val[k]) code |= (uint32_t)k_.ld[k] << (6 - 2 * k);
-            rec[5 + l] = (uint8_t)code;   // szx_TypeManager.cc:198-273
-        }
-        uint8_t *q = rec + 5 + nlead + (k_.incl - k_.lsum);
-#pragma unroll
-        for (int k = 0; k < 4; k++)
-            if (k_.val[k])
-                for (int t = W - k_.rb; t < W - k_.ld[k]; t++) *q++ = (uint8_t)(k_.sw[k] >> (8 * t));
-    }
-    __syncthreads();
-    // copy out: words wholly inside [P0, P1) as words, the two edge words
-    // (shared with the neighbouring workgroups' spans) byte by byte
-    const uint32_t span = (uint32_t)(P1 - P0);
-    const uint32_t nw = (head + span + 3) / 4;
-    uint32_t *dw = reinterpret_cast<uint32_t *>(dst0 - head);
-    for (uint32_t i = threadIdx.x; i < nw; i += 256) {
-        const uint32_t lo = 4 * i, hi = lo + 4;
-        if (lo >= head && hi <= head + span) {
-            dw[i] = stage[i];
-        } else {
-            uint8_t *db = reinterpret_cast<uint8_t *>(dw);
-            for (uint32_t j = lo < head ? head : lo; j < hi && j < head + span; j++) db[j] = lds[j];
+    for (int i = 0; i < G::NBLK; i += 64) {
+        const int lb = i + lane;
+        if (lb < G::NBLK && b0 + lb < p.nb) {
+            const uint32_t cur = R.pack[lb], nxt = R.pack[lb + 1];
+            if ((cur ^ nxt) >> 20) p.cmed[econst + (cur >> 20)] = bswap32(f32_bits(R.med[lb]));
+            if (p.index) {
+                p.index[2 * (b0 + lb)] = ebytes + (cur & 0xFFFFFu);
+                p.index[2 * (b0 + lb) + 1] = econst + (cur >> 20);
+            }
         }
     }
+    // the chunk aggregate last: its atomic's round trip stays off the tile's path
+    if (threadIdx.x == 0) lookback_chunk_done(L, tile, pend, tb, tc);
 }
 
 // ---- exclusive scan of (record bytes, constant blocks) over the blocks ----
@@ -324,7 +420,7 @@ __device__ inline void gen_sums(const uint32_t *size, uint64_t nb, uint64_t b0, 
     }
 }
 
-__global__ __launch_bounds__(256) void k_gen_part(GenericCompress g)
+__global__ __launch_bounds__(256) void k_gen_part(GenericScan g)
 {
     uint64_t a, c, ta, tc;
     gen_sums(g.size, g.nb, blockIdx.x * (uint64_t)GEN_CH + threadIdx.x * (uint64_t)GEN_PER, a, c);
@@ -336,7 +432,7 @@ __global__ __launch_bounds__(256) void k_gen_part(GenericCompress g)
 }
 
 // One workgroup: exclusive scan of the chunk sums, in place.
-__global__ __launch_bounds__(256) void k_gen_top(GenericCompress g)
+__global__ __launch_bounds__(256) void k_gen_top(GenericScan g)
 {
     uint64_t ca = 0, cc = 0;
     for (uint64_t base = 0; base < g.nparts; base += 256) {
@@ -353,7 +449,7 @@ __global__ __launch_bounds__(256) void k_gen_top(GenericCompress g)
     }
 }
 
-__global__ __launch_bounds__(256) void k_gen_apply(GenericCompress g)
+__global__ __launch_bounds__(256) void k_gen_apply(GenericScan g)
 {
     const uint64_t b0 = blockIdx.x * (uint64_t)GEN_CH + threadIdx.x * (uint64_t)GEN_PER;
     uint64_t a, c, ta, tc;
@@ -378,7 +474,7 @@ __global__ __launch_bounds__(256) void k_gen_apply(GenericCompress g)
     }
 }
 
-__global__ __launch_bounds__(256) void k_gen_bitmap(GenericCompress g)
+__global__ __launch_bounds__(256) void k_gen_bitmap(GenericScan g)
 {
     const uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
     if (i >= (g.nb + 7) / 8) return;
@@ -392,208 +488,212 @@ __global__ __launch_bounds__(256) void k_gen_bitmap(GenericCompress g)
 
 // ---- decompression ----
 
-// One block per segment of S lanes, 4 consecutive values per lane.  The
-// workgroup's records (contiguous in the payload) are staged in LDS with
-// aligned word loads, and its values leave through LDS with aligned 16-byte
-// stores.  The record's lead codes give every value's stream byte count; a
-// segment scan places each lane's bytes, and a second scan carries the
-// inherited top bytes (szxd_float.cc:78-199: a word takes its first
-// min(lead, rb) bytes from the previous word) from lane to lane.  Decodes
-// block b into out (its values in LDS); a block that fails a check sets the
-// status and leaves its values unwritten.
-template <typename T, int S>
-__device__ inline void decode_segment(const GenericDecode &p, uint64_t b, uint64_t bend, uint64_t P0,
-                                      uint64_t P1, uint32_t head, const uint32_t *stage, T *out)
-{
-    using U = typename Word<T>::U;
-    constexpr int W = Word<T>::W;
-    const DecodeHeader *h = p.h;
-    const uint64_t bs = h->bs;
-    const int l = threadIdx.x & (S - 1);
-    if (b >= bend) return;   // whole segments
-    const uint64_t rest = p.n - b * bs;
-    const int m = rest < bs ? (int)rest : (int)bs;
-    bool val[4];
-#pragma unroll
-    for (int k = 0; k < 4; k++) val[k] = 4 * l + k < m;
-    const uint64_t off = p.idx[2 * b], rank = p.idx[2 * b + 1];
-    const uint64_t noff = p.idx[2 * b + 2], nrank = p.idx[2 * b + 3];
-    if (!gen_nonconst(p.s + h->qbit, b)) {
-        // constant block: its median, widened for fp64 (szxd_float.cc:49-56)
-        if (rank >= h->nconst || nrank != rank + 1 || noff != off) {
-            if (l == 0) atomicMin(p.status, -21);
-            return;
-        }
-        const uint8_t *c = p.s + h->qmed + 4 * rank;
-        const uint32_t be = ((uint32_t)c[0] << 24) | ((uint32_t)c[1] << 16) | ((uint32_t)c[2] << 8) | (uint32_t)c[3];
-        const T med = (T)bits_f32(h->medle ? bswap32(be) : be);
-#pragma unroll
-        for (int k = 0; k < 4; k++)
-            if (val[k]) out[4 * l + k] = med;
-        return;
-    }
-    const int nlead = (m + 3) >> 2;
-    if (nrank != rank || off < P0 || noff > P1 || noff < off || noff - off < 5u + (uint64_t)nlead) {
-        if (l == 0) atomicMin(p.status, -21);
-        return;
-    }
-    const uint8_t *lds = reinterpret_cast<const uint8_t *>(stage);
-    const uint32_t r0 = head + (uint32_t)(off - P0);   // record start in LDS
-    const uint8_t *rec = lds + r0;
-    const int rl = rec[0];
-    if (rl < 1 || rl > 8 * W) {
-        if (l == 0) atomicMin(p.status, -21);
-        return;
-    }
-    const int rb = (rl + 7) >> 3;
-    const int shift = (-rl) & 7;
-    const T med = (T)bits_f32(((uint32_t)rec[1] << 24) | ((uint32_t)rec[2] << 16) | ((uint32_t)rec[3] << 8) |
-                              (uint32_t)rec[4]);
-    const uint32_t code = 4 * l < m ? rec[5 + l] : 0u;
-    int lk[4];
-    uint32_t lsum = 0;
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        const int ld = (int)(code >> (6 - 2 * k)) & 3;
-        lk[k] = ld < rb ? ld : rb;
-        if (val[k]) lsum += rb - lk[k];
-    }
-    const uint32_t incl = seg_incl_sum<S>(lsum, l);
-    const uint32_t total = __shfl(incl, S - 1, S);
-    if (5u + (uint64_t)nlead + total != noff - off) {   // segment-uniform
-        if (l == 0) atomicMin(p.status, -21);
-        return;
-    }
-    // the lane's words from the stream alone (inherited bytes still zero),
-    // masked to the low 8W - shift bits
-    const U mask = ~(U)0 >> shift;
-    uint32_t pos = r0 + 5 + (uint32_t)nlead + (incl - lsum);
-    U wv[4];
-    uint32_t mine = 0;   // this lane's carry contribution
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        const int cnt = rb - lk[k];
-        U cur = 0;
-        if (val[k] && cnt > 0) {
-            const U raw = W == 4 ? (U)lds_window4(stage, pos) : (U)lds_window8(stage, pos);
-            cur = (raw & (~(U)0 >> (8 * (W - cnt)))) << (8 * (W - rb));
-            if (W == 8 && !p.exact && rb == 5 && lk[k] == 0)   // szxd_double.cc:240-245: byte 7 <- 4th byte
-                cur = (cur & (~(U)0 >> 8)) | (((raw >> 24) & (U)0xFF) << (8 * (W - 1)));
-            pos += cnt;
-        }
-        cur &= mask;
-        if (val[k]) {
-            // bytes W-1-i (i < 3) this word writes: those below W - lk
-            uint32_t wr = 0;
-#pragma unroll
-            for (int i = 0; i < 3; i++)
-                if (lk[k] <= i) wr |= ((uint32_t)(cur >> (8 * (W - 1 - i))) & 0xFFu) << (8 * i) | (1u << (24 + i));
-            mine = carry_combine(mine, wr);
-        }
-        wv[k] = cur;
-    }
-    uint32_t acc = mine;
-#pragma unroll
-    for (int d = 1; d < S; d <<= 1) {
-        const uint32_t o = __shfl_up(acc, d, S);
-        if (l >= d) acc = carry_combine(o, acc);
-    }
-    uint32_t cin = __shfl_up(acc, 1, S);
-    if (l == 0) cin = 0;   // the first word of a block follows a zero word
-    U prev = ((U)(cin & 0xFFu) << (8 * (W - 1))) | ((U)((cin >> 8) & 0xFFu) << (8 * (W - 2))) |
-             ((U)((cin >> 16) & 0xFFu) << (8 * (W - 3)));
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        const U top = lk[k] ? ~(U)0 << (8 * (W - lk[k])) : (U)0;
-        const U cur = wv[k] | (prev & top);
-        if (val[k]) out[4 * l + k] = from_bits<T>(cur << shift) + med;
-        prev = cur;
-    }
-}
+// The workgroup's records (contiguous in the payload) staged in LDS, every
+// lane's words from its lead codes (LaneCodes, LaneWords), and the values out
+// through LDS with aligned 16-byte stores.  A block that fails a check sets
+// the status and leaves its values as they fall.
+template <typename T, int LV, int S> struct GenDecode {
+    static constexpr int W = Word<T>::W;
+    static constexpr int BPW = 256 / S;                       // blocks per workgroup
+    static constexpr int SPAN = BPW * (5 + S * LV / 4 + S * LV * W) + 64;   // record bytes, alignment and read slack
+    // value i of the workgroup sits at slot i + i / LV, so that lanes LV values
+    // apart use different banks; one chunk of alignment slack at each end
+    static constexpr int CE = 16 / W;
+    static constexpr int VALS = 256 * LV + 2 * CE;
+    static constexpr int BYTES = SPAN > W * (VALS + VALS / LV + 1) ? SPAN : W * (VALS + VALS / LV + 1);
+    __device__ static int slot(int i) { return i + i / LV; }
+};
 
-template <typename T, int S>
+// 256^3 fp32, bs 100: 59 us with one value at a time and four values a lane
+// -> 30 us.
+template <typename T, int LV, int S>
 __global__ __launch_bounds__(256) void k_gen_decode(GenericDecode p)
 {
-    constexpr int W = Word<T>::W;
-    constexpr int BPW = 256 / S;
-    __shared__ uint32_t stage[Span<S, W>::WORDS];
-    __shared__ __align__(16) T xs[Vals<T>::N];
-    const DecodeHeader *h = p.h;
-    if (h->rc != 0) return;
-    const uint64_t nb = h->nb, bs = h->bs, q0 = h->q0;
-    const uint64_t b0 = blockIdx.x * (uint64_t)BPW;
+    using G = GenDecode<T, LV, S>;
+    constexpr int W = G::W;
+    typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
+    __shared__ __align__(16) uint32_t stage[(G::BYTES + 15) / 16 * 4];
+    const DecodeHeader h = *p.h;
+    if (h.rc != 0) return;
+    const uint64_t nb = h.nb, bs = h.bs, q0 = h.q0;
+    const uint64_t b0 = blockIdx.x * (uint64_t)G::BPW;
     if (b0 >= nb) return;
-    const uint64_t bend = b0 + BPW < nb ? b0 + BPW : nb;
+    const uint64_t bend = b0 + G::BPW < nb ? b0 + G::BPW : nb;
     const uint64_t P0 = p.idx[2 * b0], P1 = p.idx[2 * bend];
     const uint64_t rmax = 5 + (bs + 3) / 4 + bs * W;
     if (P1 < P0 || P1 - P0 > (bend - b0) * rmax || P1 > p.len - q0) {   // workgroup-uniform
         if (threadIdx.x == 0) atomicMin(p.status, -21);
         return;
     }
-    // stage payload bytes [P0, P1): aligned words inside the stream, the last
-    // partial word byte by byte (q0 >= 13, so the first word starts inside)
-    const uint8_t *src = p.s + q0 + P0;
-    const uint8_t *end = p.s + p.len;
-    const uint32_t head = (uint32_t)((uintptr_t)src & 3);
-    const uint32_t *sw = reinterpret_cast<const uint32_t *>(src - head);
-    const uint32_t span = (uint32_t)(P1 - P0);
-    const uint32_t nw = (head + span + 3) / 4;
-    for (uint32_t i = threadIdx.x; i < nw; i += 256) {
-        const uint8_t *a = reinterpret_cast<const uint8_t *>(sw + i);
-        if (a + 4 <= end) {
-            stage[i] = sw[i];
-        } else {
-            uint32_t v = 0;
-            for (int j = 0; j < 4; j++)
-                if (a + j < end) v |= (uint32_t)a[j] << (8 * j);
-            stage[i] = v;
+    // payload bytes [P0, P1): 16-byte loads inside the stream (q0 >= 13, so
+    // the first chunk may start before it), bytes at its two ends
+    const uint8_t *src = p.s + q0 + P0, *end = p.s + p.len;
+    const uint32_t head = (uint32_t)((uintptr_t)src & 15), span = (uint32_t)(P1 - P0);
+    const uint32_t nchunk = span ? (head + span + 15) / 16 : 0u;
+    const uint32_t c0 = nchunk && src - head < p.s ? 1u : 0u;
+    const uint32_t c1 = nchunk && src - head + 16ull * nchunk > end ? nchunk - 1 : nchunk;
+    const u32x4_t *g = reinterpret_cast<const u32x4_t *>(src - head);
+    u32x4_t *sv = reinterpret_cast<u32x4_t *>(stage);
+    uint8_t *sb = reinterpret_cast<uint8_t *>(stage);
+    const uint32_t t = threadIdx.x;
+    u32x4_t l0{}, l1{};
+    if (t >= c0 && t < c1) l0 = g[t];
+    if (t + 256 < c1) l1 = g[t + 256];
+    // the lane's block: its pair, the next one, its bitmap bit
+    const int lane = t & 63, lseg = lane & (S - 1);
+    const uint64_t b = b0 + t / S;
+    const bool live = b < bend;   // whole segments
+    uint64_t off = 0, rank = 0, noff = 0, nrank = 0;
+    bool rec = false;
+    float cmed = 0.0f;   // a constant block's median, widened for fp64 (szxd_float.cc:49-56)
+    if (live) {
+        off = p.idx[2 * b];
+        rank = p.idx[2 * b + 1];
+        noff = p.idx[2 * b + 2];
+        nrank = p.idx[2 * b + 3];
+        rec = gen_nonconst(p.s + h.qbit, b);
+        if (!rec && rank < h.nconst && nrank == rank + 1 && noff == off) {
+            const uint8_t *c = p.s + h.qmed + 4 * rank;
+            const uint32_t be = ((uint32_t)c[0] << 24) | ((uint32_t)c[1] << 16) | ((uint32_t)c[2] << 8) | (uint32_t)c[3];
+            cmed = bits_f32(h.medle ? bswap32(be) : be);
+        } else if (!rec && lseg == 0) {
+            atomicMin(p.status, -21);
         }
     }
+    if (t >= c0 && t < c1) sv[t] = l0;
+    if (t + 256 < c1) sv[t + 256] = l1;
+    for (uint32_t c = t + 512; c < c1; c += 256) sv[c] = g[c];
+    if ((c0 != 0 || c1 != nchunk) && t < 32) {
+        const uint32_t c = t < 16 ? 0u : nchunk - 1, k = t & 15;
+        const uint8_t *a = src - head + 16ull * c + k;
+        if (nchunk && a >= p.s && a < end) sb[16 * c + k] = *a;
+    }
     __syncthreads();
+
+    const uint64_t first = b * bs;
+    const int m = !live ? 0 : p.n - first < bs ? (int)(p.n - first) : (int)bs;
+    int nv = m - lseg * LV;
+    nv = nv < 0 ? 0 : nv > LV ? LV : nv;
+    T v[LV];
+    if (live && !rec) {
+#pragma unroll
+        for (int k = 0; k < LV; k++) v[k] = (T)cmed;
+    } else if (live) {
+        const uint32_t nlead = (uint32_t)(m + 3) >> 2;
+        bool ok = nrank == rank && off >= P0 && noff <= P1 && noff >= off && noff - off >= 5u + (uint64_t)nlead;
+        const uint32_t r0 = ok ? head + (uint32_t)(off - P0) : head;   // record start in the stage
+        const uint64_t hw = lds_window8(stage, r0);
+        const int rl = (int)((uint32_t)hw & 0xFFu);
+        ok = ok && rl >= 1 && rl <= 8 * W;
+        const int rb = ok ? (rl + 7) >> 3 : 1, shift = (-rl) & 7;
+        const T med = (T)bits_f32(bswap32((uint32_t)(hw >> 8)));
+        // the lane's lead codes, those of its values only
+        uint32_t code = ok && nv > 0 ? lds_window4(stage, r0 + 5u + (uint32_t)(lseg * (LV / 4))) : 0u;
+        if (nv < 16) {   // whole lead bytes, then the last one's first codes
+            const int by = nv >> 2, r = nv & 3;
+            const uint32_t part = r ? ((0xFF00u >> (2 * r)) & 0xFFu) << (8 * by) : 0u;
+            code &= ((1u << (8 * by)) - 1u) | part;
+        }
+        LaneCodes<LV> c;
+        c.set(code, rb, nv);
+        const uint32_t inc = seg_scan_incl<S>(c.tot, lane);
+        ok = ok && 5u + (uint64_t)nlead + seg_last<S>(inc) == noff - off;   // segment-uniform
+        if (!ok && lseg == 0) atomicMin(p.status, -21);
+        LaneWords<T, LV> w;
+        w.gather(sb, ok ? r0 + 5u + nlead + (inc - c.tot) : 0u, c, rb, p.exact);
+        uint32_t cd = w.top, cm = lseg == 0 ? ~0u : w.wrote;
+        seg_scan_last_writer_head<S>(cd, cm);
+        const uint32_t cin = seg_prev<S>(cd, lane);
+#pragma unroll
+        for (int k = 0; k < LV; k++) v[k] = w.value(k, cin, shift, med);
+    }
+    __syncthreads();   // the records are read: the stage takes the values
     const uint64_t e0 = b0 * bs, e1 = bend * bs < p.n ? bend * bs : p.n;
-    decode_segment<T, S>(p, b0 + threadIdx.x / S, bend, P0, P1, head, stage,
-                         xs + (b0 + threadIdx.x / S) * bs - e0 / Vals<T>::CE * Vals<T>::CE);
+    const uint64_t f0 = e0 / G::CE * G::CE;   // first value of the first chunk
+    T *xs = reinterpret_cast<T *>(stage);
+    const int at = (int)(first - f0) + lseg * LV;
+#pragma unroll
+    for (int k = 0; k < LV; k++)
+        if (k < nv) xs[G::slot(at + k)] = v[k];
     __syncthreads();
-    unstage_values<T>(static_cast<T *>(p.out), e0, e1, xs);
+    // chunks wholly inside [e0, e1) as 16-byte stores, the edge chunks (shared
+    // with the neighbouring workgroups) value by value
+    T *out = static_cast<T *>(p.out);
+    for (uint64_t c = f0 + (uint64_t)t * G::CE; c < e1; c += 256 * G::CE) {
+        const int i = (int)(c - f0);
+        T q[G::CE];
+#pragma unroll
+        for (int k = 0; k < G::CE; k++) q[k] = xs[G::slot(i + k)];
+        if (c >= e0 && c + G::CE <= e1) {
+            typedef unsigned int u32x4_ot __attribute__((ext_vector_type(4), aligned(4)));
+            u32x4_ot o;
+            __builtin_memcpy(&o, q, 16);
+            *reinterpret_cast<u32x4_ot *>(out + c) = o;
+        } else {
+#pragma unroll
+            for (int k = 0; k < G::CE; k++)
+                if (c + k >= e0 && c + k < e1) out[c + k] = q[k];
+        }
+    }
 }
 
 // ---- host side ----
 
 uint64_t generic_parts(uint64_t nb) { return ceil_div(nb ? nb : 1, (uint64_t)GEN_CH); }
 
-// Lanes per block: the smallest power of two S with 4 S >= bs.
-static int seg_lanes(int bs)
+// Values per lane and lanes per block: 16 fp32 / 8 fp64 values a lane (one
+// word, two bytes of lead codes), fewer where a block has no more.
+static int gen_lv(int w, int bs) { return bs <= 4 ? 4 : (w == 4 && bs > 8) ? 16 : 8; }
+static int gen_lanes(int w, int bs)
 {
+    const int lv = gen_lv(w, bs);
     int s = 1;
-    while (4 * s < bs) s <<= 1;
+    while (lv * s < bs) s <<= 1;
     return s;
 }
 
-template <typename T, int S>
-static void encode_pass(const GenericCompress &g, bool write, hipStream_t st)
+uint64_t generic_tiles(uint64_t nb, int w, int bs)
 {
-    const unsigned gb = (unsigned)ceil_div(g.nb * S, 256);
-    if (write) hipLaunchKernelGGL((k_gen_encode<T, S, true>), dim3(gb), dim3(256), 0, st, g);
-    else hipLaunchKernelGGL((k_gen_encode<T, S, false>), dim3(gb), dim3(256), 0, st, g);
+    const uint64_t blocks = GEN_WAVES * 4ull * (64 / gen_lanes(w, bs));   // four steps a run (GenShape)
+    const uint64_t t = (nb + blocks - 1) / blocks;
+    return t ? t : 1;
 }
 
-template <typename T>
-static void encode_dispatch(const GenericCompress &g, bool write, hipStream_t st)
+// Calls go(values per lane, lanes per block) with the shape of a block size.
+template <int V> using Int = std::integral_constant<int, V>;
+template <typename T, typename Go> static void gen_shape(int bs, Go go)
 {
-    switch (seg_lanes(g.bs)) {
-    case 1: encode_pass<T, 1>(g, write, st); break;
-    case 2: encode_pass<T, 2>(g, write, st); break;
-    case 4: encode_pass<T, 4>(g, write, st); break;
-    case 8: encode_pass<T, 8>(g, write, st); break;
-    case 16: encode_pass<T, 16>(g, write, st); break;
-    case 32: encode_pass<T, 32>(g, write, st); break;
-    default: encode_pass<T, 64>(g, write, st); break;
+    constexpr int LV = sizeof(T) == 4 ? 16 : 8;
+    if (bs <= 4) return go(Int<4>{}, Int<1>{});
+    if constexpr (LV == 16)
+        if (bs <= 8) return go(Int<8>{}, Int<1>{});
+    switch (gen_lanes((int)sizeof(T), bs)) {
+    case 1: return go(Int<LV>{}, Int<1>{});
+    case 2: return go(Int<LV>{}, Int<2>{});
+    case 4: return go(Int<LV>{}, Int<4>{});
+    case 8: return go(Int<LV>{}, Int<8>{});
+    case 16: return go(Int<LV>{}, Int<16>{});
+    default:
+        if constexpr (LV == 8) return go(Int<LV>{}, Int<32>{});
     }
 }
 
-// The scan and the bitmap alone, from g.size (callers with their own
-// per-block passes, e.g. the cuSZx writer).
-void generic_scan_launch(const GenericCompress &g, hipStream_t st)
+template <typename T> static void gen_encode(const CompressParams &p, int bs, hipStream_t st)
+{
+    gen_shape<T>(bs, [&](auto lv, auto s) {
+        hipLaunchKernelGGL((k_gen_encode<T, decltype(lv)::value, decltype(s)::value>), dim3((unsigned)p.ntiles),
+                           dim3(64 * GEN_WAVES), 0, st, p, bs);
+    });
+}
+
+void generic_compress_launch(const CompressParams &p, int w, int bs, hipStream_t st)
+{
+    if (w == 4) gen_encode<float>(p, bs, st);
+    else gen_encode<double>(p, bs, st);
+}
+
+// The scan and the bitmap alone, from g.size.
+void generic_scan_launch(const GenericScan &g, hipStream_t st)
 {
     const unsigned np = (unsigned)g.nparts;
     hipLaunchKernelGGL(k_gen_part, dim3(np), dim3(256), 0, st, g);
@@ -602,44 +702,20 @@ void generic_scan_launch(const GenericCompress &g, hipStream_t st)
     hipLaunchKernelGGL(k_gen_bitmap, dim3((unsigned)ceil_div(ceil_div(g.nb, 8), 256)), dim3(256), 0, st, g);
 }
 
-void generic_compress_launch(const GenericCompress &g, int w, hipStream_t st)
+template <typename T> static void gen_decode(const GenericDecode &p, int bs, uint64_t nb, hipStream_t st)
 {
-    const unsigned np = (unsigned)g.nparts;
-    if (w == 4) encode_dispatch<float>(g, false, st);
-    else encode_dispatch<double>(g, false, st);
-    hipLaunchKernelGGL(k_gen_part, dim3(np), dim3(256), 0, st, g);
-    hipLaunchKernelGGL(k_gen_top, dim3(1), dim3(256), 0, st, g);
-    hipLaunchKernelGGL(k_gen_apply, dim3(np), dim3(256), 0, st, g);
-    if (w == 4) encode_dispatch<float>(g, true, st);
-    else encode_dispatch<double>(g, true, st);
-    hipLaunchKernelGGL(k_gen_bitmap, dim3((unsigned)ceil_div(ceil_div(g.nb, 8), 256)), dim3(256), 0, st, g);
-}
-
-template <typename T, int S>
-static void decode_pass(const GenericDecode &p, uint64_t nb, hipStream_t st)
-{
-    hipLaunchKernelGGL((k_gen_decode<T, S>), dim3((unsigned)ceil_div(nb * S, 256)), dim3(256), 0, st, p);
-}
-
-template <typename T>
-static void decode_dispatch(const GenericDecode &p, int bs, uint64_t nb, hipStream_t st)
-{
-    switch (seg_lanes(bs)) {
-    case 1: decode_pass<T, 1>(p, nb, st); break;
-    case 2: decode_pass<T, 2>(p, nb, st); break;
-    case 4: decode_pass<T, 4>(p, nb, st); break;
-    case 8: decode_pass<T, 8>(p, nb, st); break;
-    case 16: decode_pass<T, 16>(p, nb, st); break;
-    case 32: decode_pass<T, 32>(p, nb, st); break;
-    default: decode_pass<T, 64>(p, nb, st); break;
-    }
+    gen_shape<T>(bs, [&](auto lv, auto s) {
+        constexpr int S = decltype(s)::value;
+        hipLaunchKernelGGL((k_gen_decode<T, decltype(lv)::value, S>), dim3((unsigned)ceil_div(nb, (uint64_t)(256 / S))),
+                           dim3(256), 0, st, p);
+    });
 }
 
 void generic_decode_launch(const GenericDecode &p, int w, int bs, uint64_t nb, hipStream_t st)
 {
     if (!nb) return;
-    if (w == 4) decode_dispatch<float>(p, bs, nb, st);
-    else decode_dispatch<double>(p, bs, nb, st);
+    if (w == 4) gen_decode<float>(p, bs, nb, st);
+    else gen_decode<double>(p, bs, nb, st);
 }
 
 }  // namespace szxamd

@@ -69,8 +69,6 @@ struct CompressLayout {
     uint64_t ntiles;      // compressor tiles
     uint64_t nidx;        // index tiles
     uint64_t ws_tiles, ws_chunks, ws_cacc, ws_misc, ws_parts, ws_bitmap, ws_cmed, ws_bytes;
-    // per-block kernels only: record sizes, scan chunk sums, per-block pairs
-    uint64_t ws_gsize, ws_gparts, ws_gidx;
     uint64_t ws_osz;      // random-access container: u16 record sizes
 };
 
@@ -137,17 +135,19 @@ struct DecompressLayout {
 
 DecompressLayout decompress_layout(uint64_t n, int w, int bs, uint64_t stream_bytes);
 
-// Per-block kernels for the block sizes the tiled kernels do not take
-// (szx_generic.hip).
-struct GenericCompress {
-    const void *x;
-    uint64_t n, nb;
-    int bs;
-    float eb;
-    const float *eb_dev;  // REL: bound computed on the device
-    uint8_t *payload;     // records
+struct CompressParams;
+
+// Kernels for the block sizes the tiled ones do not take (szx_generic.hip).
+// Look-back tiles of a compress of nb blocks.
+uint64_t generic_tiles(uint64_t nb, int w, int bs);
+// p as for the tiled compressor; index (optional) is per block.
+void generic_compress_launch(const CompressParams &p, int w, int bs, hipStream_t st);
+
+// Scan of per-block record sizes into per-block pairs, with the totals and
+// the bitmap (callers with their own per-block passes: the cuSZx writer).
+struct GenericScan {
+    uint64_t nb;
     uint8_t *bitmap;
-    uint32_t *cmed;       // constant medians, big-endian, by rank
     uint64_t *totals;     // {payload bytes, constant blocks}
     uint32_t *size;       // per block: record bytes, 0 = constant
     uint64_t *idx;        // per-block pairs and the closing pair
@@ -155,8 +155,7 @@ struct GenericCompress {
     uint64_t nparts;
 };
 uint64_t generic_parts(uint64_t nb);
-void generic_compress_launch(const GenericCompress &g, int w, hipStream_t st);
-void generic_scan_launch(const GenericCompress &g, hipStream_t st);
+void generic_scan_launch(const GenericScan &g, hipStream_t st);
 
 struct GenericDecode {
     const uint8_t *s;

@@ -477,3 +477,39 @@ def test_host_results_are_the_callers(device):
     for _ in range(3):
         Z.decompress_blocked(streams[3], xs[3].size, np.float32)
     assert all(t[0] == (5.0 if i == 2 else want[i % 4][-1]) for i, t in enumerate(tails))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("bs", [1, 3, 6, 12, 20, 33, 65, 100, 129, 200, 255])
+def test_generic_run_edges(bs, dtype, device):
+    """Every lane-group shape of the per-block kernels, at array ends around a
+    wave's run and a workgroup's tile of blocks, with records that fit a wave's
+    stage and that do not, streams at any byte."""
+    import torch
+    r = np.random.default_rng(bs)
+    lanes = 1
+    while lanes * (16 if dtype == np.float32 else 8) < bs:
+        lanes *= 2
+    run = 4 * 64 // lanes * bs   # values of a wave's run
+    for n in (1, run - 1, run, 4 * run + bs // 2 + 1, 4 * run * 5 + 2):
+        t = np.arange(n)
+        x = np.where(t // (3 * bs + 7) % 4 == 0, 0.5, np.sin(t * 0.01) + r.standard_normal(n) * 1e-4).astype(dtype)
+        for eb, mode in ((1e-3, Z.ABS), (1e-13, Z.ABS), (1e-4, Z.REL)):
+            say("generic edge", dtype.__name__, bs, n, eb, mode)
+            comp = Z.DeviceCompressor(n, dtype, bs)
+            comp(torch.from_numpy(x).to(device), mode, absErrBound=eb, relBoundRatio=eb)
+            view, _, size, used = comp.stream_view()
+            s = view.cpu().numpy().tobytes()
+            want = float(np.float32(eb)) if mode == Z.ABS else O.rel_eb(x, eb)
+            assert np.float32(used) == np.float32(want)
+            assert s == O.compress(x, want, bs)
+            buf = torch.empty(3 + size, dtype=torch.uint8, device=device)
+            buf[3:] = view
+            for index in (comp.index, None):
+                dec = Z.DeviceDecompressor(n, dtype, bs, size)
+                dec.out.fill_(-7.0)
+                for flags in (Z.DECODE_REFERENCE, Z.DECODE_EXACT):
+                    dec(buf[3:], size, flags, index=index)
+                    assert dec.check() == 0
+                    ref = O.decompress(s, n, dtype, ref_quirk=flags == Z.DECODE_REFERENCE)
+                    assert bits_equal(dec.out.cpu().numpy(), ref)
