@@ -37,6 +37,7 @@ struct CompressParams {
     const void *rparts;
     float rel;            // the bound ratio
     float *eb_out;        // where tile 0 leaves the bound for the assembly
+    unsigned int *done;   // small fields: workgroups that have finished (zero before the launch)
 };
 
 // One field's header / bitmap / median assembly (device pointers).

@@ -207,7 +207,7 @@ struct LookbackRefs {
 // accumulator.  Returns the accumulator's previous value, which the caller
 // hands to lookback_chunk_done once convenient: waiting for the atomic's
 // round trip right away would stall the workgroup.  Chunk sums fit their
-// fields: a chunk holds 64 tiles of at most 2^16 record bytes and 2^11
+// fields: a chunk holds 64 tiles of at most 2^17 record bytes and 2^11
 // constant blocks each.
 __device__ inline unsigned long long lookback_publish(const LookbackRefs &L, uint64_t tile, uint32_t bytes,
                                                       uint32_t consts)

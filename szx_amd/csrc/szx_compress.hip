@@ -815,13 +815,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
     compress_tile<T, BS, LV, SLABS, IPT>(p, blockIdx.x, lds);
 }
 
-// Zero the look-back state and totals (a kernel, not a memset, so the
-// whole sequence can be captured in a HIP graph).
-__global__ void k_zero_u64(unsigned long long *p, uint64_t nwords)
+// nthr threads copy a 16-byte aligned source to any byte, in 16-byte pieces;
+// SWAP reverses each word's bytes.
+template <bool SWAP>
+__device__ inline void copy_front(uint8_t *dst, const uint8_t *src, uint64_t bytes, uint64_t gid, uint64_t nthr)
 {
-    for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < nwords;
-         i += (uint64_t)gridDim.x * blockDim.x)
-        p[i] = 0;
+    const uint4 *sv = reinterpret_cast<const uint4 *>(src);
+    const uint64_t nv = bytes / 16;
+    for (uint64_t i = gid; i < nv; i += nthr) {
+        uint4 v = sv[i];
+        if (SWAP) v = make_uint4(bswap32(v.x), bswap32(v.y), bswap32(v.z), bswap32(v.w));
+        __builtin_memcpy(dst + 16 * i, &v, 16);
+    }
+    for (uint64_t i = 16 * nv + gid; i < bytes; i += nthr)
+        dst[i] = src[SWAP ? (i & ~(uint64_t)3) | (3 - (i & 3)) : i];
 }
 
 // Header, bitmap and constant medians in front of the payload, by thread gid
@@ -858,13 +865,43 @@ __device__ inline void assemble_part(const AssembleParams &a, uint64_t gid, uint
         const uint8_t *ob = reinterpret_cast<const uint8_t *>(a.osz);   // little-endian u16
         for (uint64_t i = gid; i < 2 * nrec; i += nthr) s[20 + i] = ob[i];
     }
-    for (uint64_t i = gid; i < a.nbit; i += nthr) s[hdr + i] = a.bitmap[i];
-    const uint8_t *cm = reinterpret_cast<const uint8_t *>(a.cmed);   // big-endian medians
-    if (a.ra == 4) {
-        for (uint64_t i = gid; i < 4 * nconst; i += nthr) s[hdr + a.nbit + i] = cm[(i & ~(uint64_t)3) | (3 - (i & 3))];
-    } else {
-        for (uint64_t i = gid; i < 4 * nconst; i += nthr) s[hdr + a.nbit + i] = cm[i];
+    copy_front<false>(s + hdr, a.bitmap, a.nbit, gid, nthr);
+    // the medians are kept big-endian
+    const uint8_t *cm = reinterpret_cast<const uint8_t *>(a.cmed);
+    if (a.ra == 4) copy_front<true>(s + hdr + a.nbit, cm, 4 * nconst, gid, nthr);
+    else copy_front<false>(s + hdr + a.nbit, cm, 4 * nconst, gid, nthr);
+}
+
+// A small field's tiles: the same compress, and the workgroup that finishes
+// last assembles the stream's front itself (p.done counts them; its launch
+// costs more than the counter's round trips for so few workgroups).
+template <typename T, int BS, int LV, int SLABS, int IPT>
+__global__ __launch_bounds__(256) void k_compress_small(CompressParams p, AssembleParams a)
+{
+    __shared__ CompressLds<T, BS, LV, SLABS> lds;
+    __shared__ int s_last;
+    compress_tile<T, BS, LV, SLABS, IPT>(p, blockIdx.x, lds);
+    // Every wave's stores have reached the L2 before the one release that makes
+    // them visible to the other dies (a release by every wave: +5 us over 32 tiles).
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        s_last = __hip_atomic_fetch_add(p.done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
     }
+    __syncthreads();
+    if (!s_last) return;
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    assemble_part(a, threadIdx.x, 256);
+}
+
+// Zero the look-back state and totals (a kernel, not a memset, so the
+// whole sequence can be captured in a HIP graph).
+__global__ void k_zero_u64(unsigned long long *p, uint64_t nwords)
+{
+    for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < nwords;
+         i += (uint64_t)gridDim.x * blockDim.x)
+        p[i] = 0;
 }
 
 __global__ void k_assemble(AssembleParams a)
@@ -1164,8 +1201,8 @@ CompressLayout compress_layout(uint64_t n, int w, int bs)
     L.ntiles = ceil_div(n, compress_tile_values(w, bs));
     if (L.ntiles == 0) L.ntiles = 1;
     L.nidx = index_tiles(n, w);
-    // workspace: tile words | chunk words | chunk accumulators | misc (totals,
-    // eb) | range parts | bitmap | cmed.
+    // workspace: tile words | chunk words | chunk accumulators | misc (done count,
+    // totals, eb, error) | range parts | bitmap | cmed.
     // The look-back words are sized for one index tile per compressor tile,
     // the smallest tile any launch shape uses (the batched launch shares this
     // layout).
@@ -1177,7 +1214,7 @@ CompressLayout compress_layout(uint64_t n, int w, int bs)
     L.ws_tiles = off;   off += lb * sizeof(unsigned long long);
     L.ws_chunks = off;  off += ceil_div(lb, LB_CHUNK) * sizeof(ChunkState);
     L.ws_cacc = off;    off += ceil_div(lb, LB_CHUNK) * sizeof(unsigned long long);
-    L.ws_misc = off;    off += 64 * sizeof(uint64_t);   // totals at +128 B, eb at +256 B, error at +384 B
+    L.ws_misc = off;    off += 64 * sizeof(uint64_t);   // done count at +0, totals at +128 B, eb at +256 B, error at +384 B
     off = (off + 255) & ~(uint64_t)255;   // the range partials are read as 16-byte vectors
     L.ws_parts = off;   off += 2 * kRangeParts * sizeof(double);
     L.ws_bitmap = off;  off += (L.nbit + 15) & ~(uint64_t)15;
@@ -1199,6 +1236,38 @@ static void launch_main(const CompressParams &p, uint64_t ntiles, hipStream_t st
     constexpr int TILE = IPT * (sizeof(T) == 4 ? TILE_VALUES_F32 : TILE_VALUES_F64);
     constexpr int SLABS = TILE / (256 * LV);
     hipLaunchKernelGGL((k_compress<T, BS, LV, SLABS, IPT>), dim3((unsigned)ntiles), dim3(256), 0, st, p);
+}
+
+// Fields of so few wide tiles (1.5 MiB and less) that the chip stays mostly
+// idle and a tile's slabs, one after the other, are the kernel's time: tiles
+// of one index tile, and no launch for the assembly.  Whole REL calls at bs
+// 128, the wide tiles with k_assemble against these: 1024 fp32 values 15.7 ->
+// 11.4 us, 25600 fp32 17.1 -> 12.4, 393216 fp32 15.6 -> 13.0, 25600 fp64 15.9
+// -> 12.4.  Where every block is constant one workgroup copies all medians:
+// 13.6 -> 13.0 us at 4096 blocks, 13.7 -> 15.2 at 8192, the limit on blocks.
+// The tiles alone lose at 47 wide tiles (15.8 against 16.3 us).
+constexpr uint64_t SMALL_TILES = 24, SMALL_BLOCKS = 4096;
+static bool compress_small(const CompressLayout &L, int w, int bs)
+{
+    return bs_tiled(bs) && compress_wide(w, bs) && L.nidx && L.ntiles <= SMALL_TILES && L.nb <= SMALL_BLOCKS;
+}
+template <typename T, int BS>
+static void launch_small(CompressParams p, const AssembleParams &a, hipStream_t st)
+{
+    constexpr int LV = sizeof(T) == 4 ? 16 : 8;
+    constexpr int SLABS = (sizeof(T) == 4 ? TILE_VALUES_F32 : TILE_VALUES_F64) / (256 * LV);
+    p.ntiles = p.nidx;
+    hipLaunchKernelGGL((k_compress_small<T, BS, LV, SLABS, 1>), dim3((unsigned)p.ntiles), dim3(256), 0, st, p, a);
+}
+template <typename T>
+static void dispatch_small(int bs, const CompressParams &p, const AssembleParams &a, hipStream_t st)
+{
+    switch (bs) {   // compress_wide's block sizes
+    case 16: launch_small<T, 16>(p, a, st); break;
+    case 32: launch_small<T, 32>(p, a, st); break;
+    case 64: launch_small<T, 64>(p, a, st); break;
+    default: launch_small<T, 128>(p, a, st); break;
+    }
 }
 
 template <typename T>
@@ -1306,6 +1375,7 @@ int compress_launch(const void *d_in, uint64_t n, int w, int rel_mode, float abs
     p.cacc = reinterpret_cast<unsigned long long *>(d_ws + L.ws_cacc);
     p.totals = reinterpret_cast<uint64_t *>(misc + 16);
     p.err = reinterpret_cast<int *>(misc + 48);
+    p.done = reinterpret_cast<unsigned int *>(misc);
     p.index = d_index;
     p.bidx = d_index ? reinterpret_cast<uint16_t *>(d_index + 2 * (L.nidx + 1)) : nullptr;
     p.nidx = L.nidx;
@@ -1314,18 +1384,6 @@ int compress_launch(const void *d_in, uint64_t n, int w, int rel_mode, float abs
     p.nbit = L.nbit;
     p.osz = ra ? reinterpret_cast<uint16_t *>(d_ws + L.ws_osz) : nullptr;
     p.fm4 = fast_mode == 4;
-    int rc = 0;
-    timing_mark_begin(KK_COMPRESS, st);
-    if (bs_tiled(bs)) {
-        rc = w == 4 ? dispatch_bs<float>(bs, p, L.ntiles, st) : dispatch_bs<double>(bs, p, L.ntiles, st);
-    } else if (bs_valid(bs)) {
-        p.bidx = nullptr;   // the index is per block
-        generic_compress_launch(p, w, bs, st);
-    } else {
-        rc = -1;
-    }
-    timing_mark_end(KK_COMPRESS, st);
-    if (rc) return rc;
     AssembleParams a{};
     a.out = d_out;
     a.region = L.region;
@@ -1341,6 +1399,24 @@ int compress_launch(const void *d_in, uint64_t n, int w, int rel_mode, float abs
     a.ra = ra ? fast_mode : 0;
     a.nb = L.nb;
     a.osz = p.osz;
+    int rc = 0;
+    timing_mark_begin(KK_COMPRESS, st);
+    if (compress_small(L, w, bs)) {
+        if (w == 4) dispatch_small<float>(bs, p, a, st);
+        else dispatch_small<double>(bs, p, a, st);
+        timing_mark_end(KK_COMPRESS, st);
+        return 0;
+    }
+    if (bs_tiled(bs)) {
+        rc = w == 4 ? dispatch_bs<float>(bs, p, L.ntiles, st) : dispatch_bs<double>(bs, p, L.ntiles, st);
+    } else if (bs_valid(bs)) {
+        p.bidx = nullptr;   // the index is per block
+        generic_compress_launch(p, w, bs, st);
+    } else {
+        rc = -1;
+    }
+    timing_mark_end(KK_COMPRESS, st);
+    if (rc) return rc;
     const uint64_t work = L.nbit > 4 * L.nb ? L.nbit : 4 * L.nb;
     uint64_t blocks = (work + 255) / 256;
     if (blocks < 1) blocks = 1;

@@ -513,3 +513,36 @@ def test_generic_run_edges(bs, dtype, device):
                     assert dec.check() == 0
                     ref = O.decompress(s, n, dtype, ref_quirk=flags == Z.DECODE_REFERENCE)
                     assert bits_equal(dec.out.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("bs", [16, 32, 64, 128])
+def test_small_and_wide_compress_tiles(bs, dtype, device):
+    """Both sides of the line between the small-field launch and the wide
+    tiles, and ragged ends of both: constant fields, mixed ones and records
+    as long as the values, each container, launched again and again."""
+    import torch
+    tile = 16384 if dtype == np.float32 else 8192
+    line = min(24 * tile, 4096 * bs)
+    r = np.random.default_rng(bs)
+    for n in (1, bs + 1, tile // 4 + 1, 3 * tile - 5, line, line + 1, 26 * tile + 3):
+        t = np.arange(n)
+        noise = r.standard_normal(n)
+        mixed = np.where(t // (5 * bs + 3) % 3 == 0, -2.5, np.sin(t * 0.003) + noise * 1e-4)
+        for name, x, eb in (("constant", mixed, 10.0), ("mixed", mixed, 1e-3), ("noise", noise, 1e-20)):
+            x = x.astype(dtype)
+            d = torch.from_numpy(x).to(device)
+            for fm in (2, 3, 4):
+                say("tiles", dtype.__name__, bs, n, name, fm)
+                comp = Z.DeviceCompressor(n, dtype, bs, fastMode=fm)
+                want = O.compress(x, eb, bs) if fm == 2 else O.compress_ra(x, eb, bs, fm)
+                for _ in range(3):
+                    comp.out.zero_()
+                    comp(d, Z.ABS, eb)
+                    view, _, size, _ = comp.stream_view()
+                    assert view.cpu().numpy().tobytes() == want
+                dec = Z.DeviceDecompressor(n, dtype, bs, size, fastMode=fm)
+                dec(view, size, Z.DECODE_EXACT, index=comp.index)
+                assert dec.check() == 0
+                ref = O.decompress(want, n, dtype) if fm == 2 else O.decompress_ra(want, n, dtype, fm, ref_quirk=False)
+                assert bits_equal(dec.out.cpu().numpy(), ref)
