@@ -546,3 +546,26 @@ def test_small_and_wide_compress_tiles(bs, dtype, device):
                 assert dec.check() == 0
                 ref = O.decompress(want, n, dtype) if fm == 2 else O.decompress_ra(want, n, dtype, fm, ref_quirk=False)
                 assert bits_equal(dec.out.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("fm", [2, 3, 4])
+@pytest.mark.parametrize("bs", [100, 128])
+def test_index_free_decode_scan_edges(bs, fm, device):
+    """Index building where the scans of tiles (bs 128) and of blocks (bs 100,
+    a tile each) end at, before and after one workgroup's 1024."""
+    import torch
+    if fm != 2 and bs == 100:
+        pytest.skip("the random-access container takes the tiled block sizes")
+    per = 4096 if bs == 128 else bs
+    r = np.random.default_rng(fm)
+    for n in (1023 * per, 1024 * per, 1024 * per + 1, 2049 * per - 7):
+        t = np.arange(n)
+        x = np.where(t // 3001 % 3 == 0, 1.5, np.sin(t * 0.01) + r.standard_normal(n) * 1e-3).astype(np.float32)
+        want = O.compress(x, 1e-3, bs) if fm == 2 else O.compress_ra(x, 1e-3, bs, fm)
+        ref = O.decompress(want, n, np.float32) if fm == 2 else O.decompress_ra(want, n, np.float32, fm)
+        say("scan edge", bs, fm, n)
+        d = torch.from_numpy(np.frombuffer(want, np.uint8).copy()).to(device)
+        dec = Z.DeviceDecompressor(n, np.float32, bs, len(want), fastMode=fm)
+        dec(d, len(want), Z.DECODE_REFERENCE)
+        assert dec.check() == 0
+        assert bits_equal(dec.out.cpu().numpy(), ref)
