@@ -27,8 +27,8 @@
 //   D  scans        records before each chunk; non-constant blocks before
 //                   each compressor tile.
 //   E  k_ix_scatter record starts in record order.
-//   F  k_ix_tail    the last record's true size (its block may be partial) and
-//                   the payload end.
+//   F               in E, by the wave with the last record: its true size (its
+//                   block may be partial) and the payload end.
 //   G  k_ix_tiles   the tile pairs and the per-block entries of the index;
 //      k_ix_pairs   for the block sizes the tiled kernels do not take, the
 //                   per-block pairs instead (tiles of one block).
@@ -445,19 +445,6 @@ static void scan_u32(const uint32_t *in, uint64_t n, uint64_t *out, uint64_t *bs
     hipLaunchKernelGGL(k_scan_add, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, out, n, bsum);
 }
 
-// E: record starts (payload offsets) in record order.  One wave per chunk.
-__global__ __launch_bounds__(256) void k_ix_scatter(IxParams x)
-{
-    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const uint64_t c = blockIdx.x * 4ull + wv;
-    if (c >= x.nch || *x.status != 0) return;
-    const uint64_t base = x.cbase[c] + x.csum[c >> 10];
-    const uint32_t k = x.cnt[c];
-    const uint64_t K = x.h->nb - x.h->nconst;
-    for (uint32_t i = lane; i < k; i += 64)
-        if (base + i < K) x.rec[base + i] = c * IX_C + x.pos[c * x.maxr + i];
-}
-
 // Bitmap byte j of a block range [b0, b1) with b0 a multiple of 8: the bits of
 // blocks at or past b1 cleared (the bitmap is MSB first).
 __device__ inline uint32_t bitmap_byte(const IxParams &x, const DecodeHeader &h, uint64_t j, uint64_t b1)
@@ -515,70 +502,84 @@ __global__ __launch_bounds__(1024) void k_ix_scan_tops(IxParams x, uint64_t cblk
 
 __device__ inline uint64_t tile_base(const IxParams &x, uint64_t t) { return x.tbase[t] + x.tsum[t >> 10]; }
 
-// F: the last record's true size and the payload end; checks the record
-// count.  One wave: the bitmap is searched from its end 64 bytes at a time,
-// and the last record's lead codes are summed one byte per lane.
-__global__ void k_ix_tail(IxParams x)
+// F: the true size of the last record (it starts at byte q) and the payload
+// end.  One wave: the bitmap is searched from its end 64 bytes at a time, and
+// the record's lead codes are summed one byte per lane.
+__device__ inline void ix_tail(const IxParams &x, uint64_t q, int lane)
 {
-    const int lane = threadIdx.x;
-    if (*x.status != 0) return;
     const DecodeHeader &h = *x.h;
-    const uint64_t K = h.nb - h.nconst;
     const uint64_t P = x.len - h.q0;
     int32_t st = 0;
     uint64_t pend = 0;
-    if (*x.found < K) st = -30;
-    if (st == 0 && K > 0) {
-        // the last non-constant block (one exists: K > 0)
-        const uint64_t nbyte = (h.nb + 7) / 8;
-        uint64_t b = 0;
-        for (uint64_t top = nbyte; top > 0; top = top > 64 ? top - 64 : 0) {
-            uint32_t v = 0;
-            if ((uint64_t)lane < top) {
-                const uint64_t j = top - 1 - lane;
-                v = x.s[h.qbit + j];
-                if (8 * j + 8 > h.nb) v &= (0xFF00u >> (h.nb - 8 * j)) & 0xFFu;
-            }
-            const unsigned long long m = __ballot(v != 0);
-            if (m) {
-                const int l = __builtin_ctzll(m);   // the lowest lane holds the highest byte
-                const uint32_t vb = __shfl(v, l, 64);
-                b = 8 * (top - 1 - l) + 7 - __builtin_ctz(vb);
-                break;
-            }
+    // the last non-constant block (one exists: it has a record)
+    const uint64_t nbyte = (h.nb + 7) / 8;
+    uint64_t b = 0;
+    for (uint64_t top = nbyte; top > 0; top = top > 64 ? top - 64 : 0) {
+        uint32_t v = 0;
+        if ((uint64_t)lane < top) {
+            const uint64_t j = top - 1 - lane;
+            v = x.s[h.qbit + j];
+            if (8 * j + 8 > h.nb) v &= (0xFF00u >> (h.nb - 8 * j)) & 0xFFu;
         }
-        const uint64_t nel = (b + 1) * (uint64_t)x.bs <= x.n ? (uint64_t)x.bs : x.n - b * (uint64_t)x.bs;
-        const uint64_t nl = (nel + 3) / 4;
-        const uint64_t q = x.rec[K - 1];
-        if (q + 5 + nl > P) {
-            st = -31;
+        const unsigned long long m = __ballot(v != 0);
+        if (m) {
+            const int l = __builtin_ctzll(m);   // the lowest lane holds the highest byte
+            const uint32_t vb = __shfl(v, l, 64);
+            b = 8 * (top - 1 - l) + 7 - __builtin_ctz(vb);
+            break;
+        }
+    }
+    const uint64_t nel = (b + 1) * (uint64_t)x.bs <= x.n ? (uint64_t)x.bs : x.n - b * (uint64_t)x.bs;
+    const uint64_t nl = (nel + 3) / 4;
+    if (q + 5 + nl > P) {
+        st = -31;
+    } else {
+        const uint8_t *r = x.s + h.q0 + q;
+        const uint32_t rl = r[0];
+        if (rl == 0 || rl > 8u * x.w) {
+            st = -32;
         } else {
-            const uint8_t *r = x.s + h.q0 + q;
-            const uint32_t rl = r[0];
-            if (rl == 0 || rl > 8u * x.w) {
-                st = -32;
-            } else {
-                const uint32_t rb = (rl + 7) >> 3;
-                uint32_t add = 0;
-                for (uint64_t l = lane; l < nl; l += 64) {
-                    const uint32_t by = r[5 + l];
-                    for (uint32_t k = 0; k < 4 && 4 * l + k < nel; k++) {
-                        const uint32_t ld = (by >> (6 - 2 * k)) & 3;
-                        if (ld < rb) add += rb - ld;
-                    }
+            const uint32_t rb = (rl + 7) >> 3;
+            uint32_t add = 0;
+            for (uint64_t l = lane; l < nl; l += 64) {
+                const uint32_t by = r[5 + l];
+                for (uint32_t k = 0; k < 4 && 4 * l + k < nel; k++) {
+                    const uint32_t ld = (by >> (6 - 2 * k)) & 3;
+                    if (ld < rb) add += rb - ld;
                 }
-#pragma unroll
-                for (int m = 1; m < 64; m <<= 1) add += __shfl_xor(add, m, 64);
-                const uint64_t sz = 5 + nl + add;
-                if (q + sz > P) st = -33;
-                else pend = q + sz;
             }
+#pragma unroll
+            for (int m = 1; m < 64; m <<= 1) add += __shfl_xor(add, m, 64);
+            const uint64_t sz = 5 + nl + add;
+            if (q + sz > P) st = -33;
+            else pend = q + sz;
         }
     }
     if (lane == 0) {
         if (st) *x.status = st;
         else *x.pend = pend;
     }
+}
+
+// E: record starts (payload offsets) in record order, and the record count's
+// check.  One wave per chunk; the wave that holds the last record finishes it
+// (with a launch of its own for that one wave a decode of 25 M fp32 values took
+// 79.6 us, so 77.9).
+__global__ __launch_bounds__(256) void k_ix_scatter(IxParams x)
+{
+    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const uint64_t c = blockIdx.x * 4ull + wv;
+    if (c >= x.nch || *x.status != 0) return;
+    const uint64_t base = x.cbase[c] + x.csum[c >> 10];
+    const uint32_t k = x.cnt[c];
+    const uint64_t K = x.h->nb - x.h->nconst;
+    for (uint32_t i = lane; i < k; i += 64)
+        if (base + i < K) x.rec[base + i] = c * IX_C + x.pos[c * x.maxr + i];
+    if (c == 0 && lane == 0) {
+        if (*x.found < K) *x.status = -30;
+        else if (K == 0) *x.pend = 0;
+    }
+    if (*x.found >= K && base < K && K <= base + k) ix_tail(x, c * IX_C + x.pos[c * x.maxr + (K - 1 - base)], lane);
 }
 
 // G: tile pairs and per-block entries.  One wave per tile; the non-constant
@@ -782,7 +783,6 @@ void index_build_launch(const uint8_t *s, uint64_t len, uint64_t n, int w, int b
     hipLaunchKernelGGL(k_ix_repair, dim3(1), dim3(64), 0, st, x);
     index_scans_launch(x, L, ws, true, st);
     hipLaunchKernelGGL(k_ix_scatter, dim3((nch + 3) / 4), dim3(256), 0, st, x);
-    hipLaunchKernelGGL(k_ix_tail, dim3(1), dim3(64), 0, st, x);
     index_tiles_launch(x, L, bs_tiled(bs), st);
 }
 
