@@ -141,3 +141,21 @@ def test_non_blocked_edges(dtype, device):
                 want = O.decompress_nb(s, n, dtype, ref_quirk=flags == Z.DECODE_REFERENCE)
                 assert bits_equal(c.dec.cpu().numpy(), want)
             assert float(back[0]) == -7.0
+
+
+@pytest.mark.parametrize("tiles", [1024, 1025, 8 * 1024, 8 * 1024 + 1, 10 * 1024 - 3])
+def test_non_blocked_scan_edges(tiles, device):
+    """Decoder tiles (2048 doubles) at the edges of what a lane of the scan
+    takes at once; long runs of one value hand bytes over many tiles."""
+    import torch
+    r = np.random.default_rng(tiles)
+    n = tiles * 2048 - 1
+    x = np.sin(np.arange(n) * 1e-5)
+    x[n // 3: n // 2] = 0.25
+    x[-5000:] = r.standard_normal(5000)
+    say("nb scan", tiles, n)
+    want = O.compress_nb(x, 1e-6)
+    c = Z.DeviceNonBlocked(n, np.float64)
+    c.decompress(torch.from_numpy(np.frombuffer(want, np.uint8).copy()).to(device), len(want), Z.DECODE_REFERENCE)
+    assert c.check() == 0
+    assert bits_equal(c.dec.cpu().numpy(), O.decompress_nb(want, n, np.float64, ref_quirk=True))
